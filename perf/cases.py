@@ -81,7 +81,20 @@ def _mesh(rng, dim, els_lo, els_hi, even=False):
     return {"dim": dim, "nx": n[0], "ny": n[1], "nz": n[2] if dim == 3 else 0}
 
 
+def _cost(case):
+    w = work(case)
+    return max(w["bytes"], w["flops"] / 50)
+
+
 def draw(rng):
+    most = max(_cost(c) for c in listed())
+    case = _draw(rng)
+    while _cost(case) > most:
+        case = _draw(rng)
+    return case
+
+
+def _draw(rng):
     kind = rng.choice(["csr", "csr", "mf", "mf", "mf", "cg", "cg", "cg_multi", "ir", "batch", "adjoint", "assemble"])
     dim = rng.choice([2, 3])
     p = rng.randint(1, 5) if dim == 2 else rng.randint(1, 4)
