@@ -22,8 +22,10 @@ struct CsrOp : ngsamd_op_s {
   DevBuf<int> val_ptr;  // first value of each run, nruns + 1
   DevBuf<int> rcols;    // shared column lists
   DevBuf<double> rvals; // values, run by run, [L][R]
-  DevBuf<int> blk_run;  // runs kernel blocks: first run, nblocks + 1
-  DevBuf<int> blk_len;  // runs kernel blocks: rows per run (all runs of a block alike)
+  // runs kernel: {first run, its first value, its first row,
+  // runs | rows per run << 8 | log2 of the lanes per run << 16 | slots per lane << 24}
+  DevBuf<int4> tasks;
+  int ntasks = 0;
   DevBuf<int> row_run;  // run of each row (structure-only operators, runs layout)
   int64_t nruns = 0, nshared = 0;
   int64_t max_row_len = 0;
@@ -33,10 +35,11 @@ struct CsrOp : ngsamd_op_s {
   int group = 32;  // lanes per row (rowgroup kernel)
   int algo = 1;    // 0: rowgroup, 1: stream, 2: runs
   DevBuf<int> blk_row;  // stream kernel row blocks
-  int nblocks = 0;
+  int nblocks = 0;      // stream: row blocks; runs: rounds of 4 tasks
   int block_nnz = 2048;
-  int max_grid = 16384;  // workgroups of the stream/runs kernels
-  int flip = 0;          // direction of the next Mult / MultAdd block walk (alternates)
+  int max_grid = 16384;  // most workgroups of the stream/runs kernels
+  int walk_grid = 16384; // of the runs kernel for several vectors and with partial sums
+  int flip = 0;          // direction of the next Mult / MultAdd walk (alternates)
   // v null: the structure only, values zero until filled on the device
   CsrOp(int64_t h, int64_t w, const int64_t* rp, const int* c, const double* v);
   void MultAdd(double s, const double* x, double* y, hipStream_t st) override;

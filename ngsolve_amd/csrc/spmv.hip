@@ -11,8 +11,7 @@
 // or cell of an H1 space) form a run that stores the list once and its values
 // column by column.  Values still stream once (8 B per nonzero) but the column
 // numbers drop to 4 B per run entry and each gathered x entry serves the
-// whole run.  Blocks hold runs of one length and at most 2048 values; the
-// block loop is the stream kernel's.
+// whole run.
 //
 // stream: int32 row pointers, int32 column numbers, FP64 values (12 B per
 // nonzero streamed once); the rows are cut on the host into blocks of consecutive
@@ -89,6 +88,7 @@ __global__ __launch_bounds__(kSpmvBlock) void CsrSpmvKernel(
 
 
 constexpr int kStreamBlock = 256;
+constexpr int kRunWaves = kStreamBlock / 64;  // tasks of the runs kernel in flight per workgroup
 
 // y[r] = (ACCUM ? y[r] : 0) + s * (A x)[r] over the row blocks
 // [blk_row[b], blk_row[b+1]) of at most NNZ nonzeros; DOT as in CsrSpmvKernel.
@@ -174,245 +174,286 @@ __global__ __launch_bounds__(kStreamBlock) void CsrStreamKernel(
 }
 
 
-// y = (ACCUM ? y : 0) + s * A x over the run blocks [blk_run[b], blk_run[b+1])
-// with blk_len[b] rows per run (at most NNZ values and NNZ rows per block);
-// DOT as in CsrSpmvKernel.  Block b: lane k of its value range forms value k
-// times x[column of shared slot k / R] into LDS (values stream coalesced, the
-// R lanes of one slot read one column number and one x entry); row j = run R
-// + q then sums the slots of its run at stride R.  A block holding more
-// than NNZ values is a single row (R = 1) that the whole workgroup strides.
-// NNZ <= 2048: at most 64 VGPRs, so 8 workgroups fit a CU (72 registers
-// allowed 7; 394 vs 398 us at 32^3 p=4).
-// Consecutive plain applies (Mult / MultAdd) alternate the direction of the
-// block walk (reverse), so that each apply starts on the blocks the previous
-// one read last, which the 256 MB Infinity Cache still holds; their values
-// are read with plain loads for that (non-temporal ones are not kept):
-// 374-375 against 383-384 us per apply at 32^3 p=4 (forward only with plain
-// loads: 395).  Every row is summed by the same code in the same order
-// either way.  Inside CG (DOT) the vector kernels between two applies take
-// that cache, so the CG variant keeps the forward walk and non-temporal
-// value loads (with the alternating walk and plain loads Jacobi-CG at 32^3
-// p=4 took 0.142 against 0.140 s, and with the sparse Cholesky coarse solve
-// 0.184 against 0.173 s).
-template <int NNZ, bool ACCUM, bool DOT>
-__global__ __launch_bounds__(kStreamBlock, NNZ <= 2048 ? 8 : 4) void CsrRunsKernel(
-    const int* __restrict__ run_row, const int* __restrict__ run_ptr, const int* __restrict__ val_ptr,
-    const int* __restrict__ rcols, const double* __restrict__ rvals, const double* __restrict__ x,
-    double* __restrict__ y, const int* __restrict__ blk_run, const int* __restrict__ blk_len, int nblocks,
-    int blocks_per_wg, double s, double* __restrict__ partials, const int* __restrict__ stop_flag, int reverse) {
-  static_assert(NNZ <= 4096, "RunDiv is exact below 4096");
-  if (stop_flag && *stop_flag) return;
-  constexpr int PER = NNZ / kStreamBlock;
-  __shared__ double prod[NNZ];
-  __shared__ double lds[kStreamBlock / 64];
-  const int tid = threadIdx.x;
-  // reverse: the first workgroups dispatched take the last blocks, each
-  // workgroup walks its range backwards
-  const int lx = XcdContiguousBlock(blockIdx.x, gridDim.x);
-  const int lb = reverse ? (int)gridDim.x - 1 - lx : lx;
-  const int b0 = lb * blocks_per_wg;
-  const int b1 = min(b0 + blocks_per_wg, nblocks);
-  auto blk = [&](int t) { return reverse ? b0 + b1 - 1 - t : t; };
-  double dotacc = 0.0;
+// ------------------------------------------------------------- runs kernel
+// A task is up to 64 / G consecutive runs of R rows each, one wavefront's
+// work: a group of G lanes per run (RunGroup: 8 to 64 by the run's length).
+// Lane l of a group takes the column slots l, l + G, ... of its run: one
+// column number and one x entry per slot serve the R values of the slot
+// (adjacent in memory), and the R row sums stay in the lane's registers until
+// a butterfly over the group ends them.  No LDS and no barrier: every
+// wavefront runs on its own, so the loads of one cover the sums of another.
 
-  // header and register-held loads of the block in flight
-  int u0 = 0, u1 = 0, R = 1, inv = 65536, c0 = 0, vb = 0, nv = 0;
-  int c[PER];
-  double v[PER];
-  auto fetch = [&](int b) {
-    u0 = blk_run[b];
-    u1 = blk_run[b + 1];
-    R = blk_len[b];
-    inv = (65536 + R - 1) / R;
-    c0 = run_ptr[u0];
-    vb = val_ptr[u0];
-    nv = val_ptr[u1] - vb;
-    if (nv > NNZ) return;  // long row: streamed when it is reached
-    // unconditional loads (lanes past the block read entry 0 of it, kept in
-    // bounds by the padding) so that every load is in flight at once
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int k = tid + i * kStreamBlock;
-      const int kk = k < nv ? k : 0;
-      c[i] = __builtin_nontemporal_load(&rcols[c0 + RunDiv(kk, inv)]);
-      v[i] = DOT ? __builtin_nontemporal_load(&rvals[vb + kk]) : rvals[vb + kk];
-    }
-  };
-  if (b0 < b1) fetch(blk(b0));
-  for (int b = b0; b < b1; b++) {
-    if (nv > NNZ) {
-      // one long row: the whole workgroup strides over it
-      double a = 0.0;
-      for (int k = tid; k < nv; k += kStreamBlock)
-        a += __builtin_nontemporal_load(&rvals[vb + k]) * x[__builtin_nontemporal_load(&rcols[c0 + k])];
-      a = BlockSum<kStreamBlock>(a, lds);
-      const int r = run_row[u0];
-      if (tid == 0) {
-        if (ACCUM) y[r] += s * a; else y[r] = s * a;
-        if (DOT) dotacc += x[r] * a;
-      }
-      if (b + 1 < b1) fetch(blk(b + 1));
-      continue;
-    }
-    {
-      double xv[PER];
-#pragma unroll
-      for (int i = 0; i < PER; i++) xv[i] = x[c[i]];
-#pragma unroll
-      for (int i = 0; i < PER; i++) {
-        const int k = tid + i * kStreamBlock;
-        prod[k] = k < nv ? v[i] * xv[i] : 0.0;
-      }
-    }
-    __syncthreads();
-    // this block's header, then the next block's loads
-    const int cu0 = u0, cR = R, cinv = inv, cc0 = c0;
-    const int row0 = run_row[cu0];
-    const int nr = (u1 - u0) * R;
-    int tpr = 64;
-    while (tpr > 1 && tpr * nr > kStreamBlock) tpr >>= 1;
-    const int l = tid & (tpr - 1);
-    for (int j0 = 0; j0 < nr; j0 += kStreamBlock / tpr) {
-      const int j = j0 + tid / tpr;
-      double sum = 0.0;
-      if (j < nr) {
-        const int run = RunDiv(j, cinv), q = j - run * cR;
-        const int s0 = run_ptr[cu0 + run] - cc0, s1 = run_ptr[cu0 + run + 1] - cc0;
-        // four independent partial sums so that the LDS reads overlap
-        double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-        int k = s0 + l;
-        for (; k + 3 * tpr < s1; k += 4 * tpr) {
-          a0 += prod[k * cR + q];
-          a1 += prod[(k + tpr) * cR + q];
-          a2 += prod[(k + 2 * tpr) * cR + q];
-          a3 += prod[(k + 3 * tpr) * cR + q];
-        }
-        for (; k < s1; k += tpr) a0 += prod[k * cR + q];
-        sum = (a0 + a1) + (a2 + a3);
-      }
-      for (int off = tpr / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-      if (j < nr && l == 0) {
-        if (ACCUM) y[row0 + j] += s * sum; else y[row0 + j] = s * sum;
-        if (DOT) dotacc += x[row0 + j] * sum;
-      }
-    }
-    __syncthreads();
-    if (b + 1 < b1) fetch(blk(b + 1));
+// column slots per lane and pass, whose loads are all in flight together:
+// about 50 registers of loads whatever R, fewer slots where several vectors'
+// sums take the registers
+constexpr int RunUnroll(int R, int KC = 1) {
+  const int one = R == 1 ? 8 : R == 2 ? 6 : R <= 4 ? 4 : R <= 6 ? 3 : 2;
+  const int fit = (130 - 2 * R * KC) / (3 + 2 * KC + 2 * R);
+  return KC == 1 || fit > one ? one : fit < 1 ? 1 : fit;
+}
+
+// Calls f(R, U) as compile-time constants for a task of run length R whose
+// runs hold up to m slots per lane: U = min(m, RunUnroll(R, KC)), so that no
+// pass loads slots that no lane has (KC = 8: R <= 3 only).
+template <int KC, int R, int U, class F>
+__device__ __forceinline__ void ForRunSlots(int m, F&& f) {
+  if constexpr (U < RunUnroll(R, KC)) {
+    if (m <= U) f(std::integral_constant<int, R>{}, std::integral_constant<int, U>{});
+    else ForRunSlots<KC, R, U + 1>(m, f);
+  } else {
+    f(std::integral_constant<int, R>{}, std::integral_constant<int, U>{});
   }
-  if (DOT) StorePartial<kStreamBlock>(dotacc, partials, lds);
+}
+template <int KC, int R = 1, class F>
+__device__ __forceinline__ void ForRunShape(int r, int m, F&& f) {
+  if constexpr (R < (KC == 8 ? 3 : kMaxRun)) {
+    if (r == R) ForRunSlots<KC, R, 1>(m, f);
+    else ForRunShape<KC, R + 1>(r, m, f);
+  } else {
+    ForRunSlots<KC, R, 1>(m, f);
+  }
+}
+
+template <int CTRL>
+__device__ __forceinline__ double DppMove(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// Sum over the lane's group of 2^lg lanes, in every lane of it (lg uniform,
+// 3 to 6): lanes i and i ^ 1, then i ^ 2 (quad permutations), then the other
+// quad of 8, the other 8 of 16 (mirrors), then by shuffles.
+__device__ __forceinline__ double GroupSum(double v, int lg) {
+  v += DppMove<0xB1>(v);
+  v += DppMove<0x4E>(v);
+  v += DppMove<0x141>(v);
+  if (lg > 3) v += DppMove<0x140>(v);
+  if (lg > 4) v += __shfl_xor(v, 16, 64);
+  if (lg > 5) v += __shfl_xor(v, 32, 64);
+  return v;
+}
+
+// two adjacent doubles in one 16-byte load, aligned like a double
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void LoadPair(const double* p, double& a, double& b) {
+  const double2u t = *reinterpret_cast<const double2u*>(p);
+  a = t.x;
+  b = t.y;
+}
+
+// acc[q][j] = this lane's share of row q of its run (first column c0, first
+// value v0, L slots) times component j0 + j of the K-vector x
+template <int R, int KC, int U>
+__device__ __forceinline__ void RunPartials(const int* __restrict__ rcols, const double* __restrict__ rvals,
+                                            const double* __restrict__ x, int K, int j0, int c0, int v0, int L, int l,
+                                            int G, double (&acc)[R][KC]) {
+#pragma unroll
+  for (int q = 0; q < R; q++)
+#pragma unroll
+    for (int j = 0; j < KC; j++) acc[q][j] = 0.0;
+  for (int k0 = l; k0 < L; k0 += U * G) {
+    // unconditional loads from clamped slots, so that all are in flight at once
+    int c[U];
+    double v[U][R], xv[U][KC];
+#pragma unroll
+    for (int i = 0; i < U; i++) c[i] = rcols[c0 + min(k0 + i * G, L - 1)];
+#pragma unroll
+    for (int i = 0; i < U; i++) {
+      const double* vp = rvals + (v0 + min(k0 + i * G, L - 1) * R);
+#pragma unroll
+      for (int q = 0; q + 1 < R; q += 2) LoadPair(vp + q, v[i][q], v[i][q + 1]);
+      if constexpr (R % 2 == 1) v[i][R - 1] = vp[R - 1];
+    }
+#pragma unroll
+    for (int i = 0; i < U; i++) {
+      const double* xp = x + ((int64_t)c[i] * K + j0);
+      if constexpr (KC == 1) xv[i][0] = xp[0];
+      else {
+#pragma unroll
+        for (int j = 0; j < KC; j += 2) LoadPair(xp + j, xv[i][j], xv[i][j + 1]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < U; i++) {
+      const bool ok = k0 + i * G < L;
+#pragma unroll
+      for (int q = 0; q < R; q++)
+#pragma unroll
+        for (int j = 0; j < KC; j++) {
+          const double t = __builtin_fma(v[i][q], xv[i][j], acc[q][j]);
+          acc[q][j] = ok ? t : acc[q][j];
+        }
+    }
+  }
+}
+
+// A task and, per lane, the first column, first value and length of its run.
+// The walk loads the record two tasks ahead and the run pointers one task
+// ahead, so that a task starts with its value and column loads.
+struct RunHead {
+  int4 t;
+  int c0, c1, base;
+};
+__device__ __forceinline__ void LoadRunHead(RunHead& h, const int* __restrict__ run_ptr) {
+  const int n = h.t.w & 0xff, lg = (h.t.w >> 16) & 0xff;
+  const int u = h.t.x + min((int)(threadIdx.x & 63) >> lg, n - 1);
+  h.c0 = run_ptr[u];
+  h.c1 = run_ptr[u + 1];
+  h.base = run_ptr[h.t.x];
+}
+// Calls f(head) for the wavefront's tasks of workgroup lb of grid: every
+// kRunWaves-th of the workgroup's contiguous share (reverse: downwards).
+template <class F>
+__device__ __forceinline__ void WalkRunTasks(const int4* __restrict__ tasks, int ntasks,
+                                             const int* __restrict__ run_ptr, int lb, int grid, int reverse, F f) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int first = (int)((int64_t)lb * ntasks / grid) + wave;
+  const int end = (int)((int64_t)(lb + 1) * ntasks / grid);
+  if (first >= end) return;
+  const int cnt = (end - first + kRunWaves - 1) / kRunWaves;
+  auto at = [&](int i) {
+    const int k = min(i, cnt - 1);
+    return tasks[first + (reverse ? cnt - 1 - k : k) * kRunWaves];
+  };
+  RunHead h, next;
+  h.t = at(0);
+  LoadRunHead(h, run_ptr);
+  next = h;
+  if (cnt > 1) next.t = at(1);
+  for (int i = 0; i < cnt; i++) {
+    int4 t2 = next.t;
+    if (i + 1 < cnt) {
+      t2 = at(i + 2);
+      LoadRunHead(next, run_ptr);
+    }
+    f(h);
+    h = next;
+    next.t = t2;
+  }
+}
+
+// The task's rows: y[r] = (ACCUM ? y[r] : 0) + s * (A x)[r]; with DOT the
+// lane's sum of x[r] * (A x)[r] is added to dotacc.
+template <int R, int U, bool ACCUM, bool DOT>
+__device__ __forceinline__ void RunTaskRows(const RunHead& h, const int* __restrict__ rcols,
+                                            const double* __restrict__ rvals, const double* __restrict__ x,
+                                            double* __restrict__ y, double s, double& dotacc) {
+  const int4 t = h.t;
+  const int n = t.w & 0xff, lg = (t.w >> 16) & 0xff;
+  const int lane = threadIdx.x & 63, G = 1 << lg;
+  const int g = lane >> lg, l = lane & (G - 1);
+  const int c0 = h.c0, L = h.c1 - h.c0;
+  const int v0 = t.y + (c0 - h.base) * R;
+  double acc[R][1];
+  RunPartials<R, 1, U>(rcols, rvals, x, 1, 0, c0, v0, L, l, G, acc);
+  double mine = 0.0;
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    const double sum = GroupSum(acc[q][0], lg);
+    mine = l == q ? sum : mine;
+  }
+  if (g < n && l < R) {
+    const int r = t.z + g * R + l;
+    if (ACCUM) y[r] += s * mine; else y[r] = s * mine;
+    if (DOT) dotacc += x[r] * mine;
+  }
+}
+
+// y = (ACCUM ? y : 0) + s * A x over the tasks (see above); DOT as in
+// CsrSpmvKernel.  Each workgroup takes 4 * rounds consecutive tasks, its wavefronts
+// in turn.
+// Consecutive plain applies (Mult / MultAdd) alternate the direction of the
+// walk (reverse), so that each apply starts on the values the previous one
+// read last, which the 256 MB Infinity Cache still holds.  Every row is
+// summed by the same code in the same order either way.  Inside CG (DOT) the
+// vector kernels between two applies take that cache: it keeps the forward
+// walk.  (Non-temporal value loads are slower here: the loads of one slot's
+// R values share lines that L1 has to keep; CG on 64^2 p=3 17.2 -> 19.5 us an
+// iteration.)
+//
+// Bound by the value stream and the loads per byte of it.  Against the former
+// kernel (products of 2048-value blocks through LDS, one column and x load
+// per value), us per apply: 32^3 p=4 (159M nonzeros) 389 -> 298 (4.3 TB/s of
+// values alone, 5.2 TB/s with the shared columns), 20x16x24 p=4 97 -> 64,
+// 61x67 p=3 6.0 -> 4.3.
+template <bool ACCUM, bool DOT>
+__global__ __launch_bounds__(kStreamBlock, 6) void CsrRunsKernel(
+    const int4* __restrict__ tasks, int ntasks, const int* __restrict__ run_ptr,
+    const int* __restrict__ rcols, const double* __restrict__ rvals, const double* __restrict__ x,
+    double* __restrict__ y, double s, double* __restrict__ partials, const int* __restrict__ stop_flag, int reverse) {
+  if (stop_flag && *stop_flag) return;
+  const int lx = XcdContiguousBlock(blockIdx.x, gridDim.x);
+  double dotacc = 0.0;
+  WalkRunTasks(tasks, ntasks, run_ptr, reverse ? (int)gridDim.x - 1 - lx : lx, gridDim.x, reverse, [&](const RunHead& h) __attribute__((always_inline)) {
+    ForRunShape<1>((h.t.w >> 8) & 0xff, h.t.w >> 24, [&](auto r, auto u) __attribute__((always_inline)) {
+      RunTaskRows<decltype(r)::value, decltype(u)::value, ACCUM, DOT>(h, rcols, rvals, x, y, s, dotacc);
+    });
+  });
+  if (DOT) {
+    __shared__ double lds[kStreamBlock / 64];
+    StorePartial<kStreamBlock>(dotacc, partials, lds);
+  }
+}
+
+template <int R, int U, int KC>
+__device__ __forceinline__ void RunTaskRowsMulti(const RunHead& h, const int* __restrict__ rcols,
+                                                 const double* __restrict__ rvals, const double* __restrict__ x,
+                                                 double* __restrict__ y, int K, int j0) {
+  const int4 t = h.t;
+  const int n = t.w & 0xff, lg = (t.w >> 16) & 0xff;
+  const int lane = threadIdx.x & 63, G = 1 << lg;
+  const int g = lane >> lg, l = lane & (G - 1);
+  const int c0 = h.c0, L = h.c1 - h.c0;
+  const int v0 = t.y + (c0 - h.base) * R;
+  double acc[R][KC];
+  RunPartials<R, KC, U>(rcols, rvals, x, K, j0, c0, v0, L, l, G, acc);
+  double mine[KC];
+#pragma unroll
+  for (int j = 0; j < KC; j++) mine[j] = 0.0;
+#pragma unroll
+  for (int q = 0; q < R; q++)
+#pragma unroll
+    for (int j = 0; j < KC; j++) {
+      const double sum = GroupSum(acc[q][j], lg);
+      mine[j] = l == q ? sum : mine[j];
+    }
+  if (g < n && l < R) {
+    double* yp = y + ((int64_t)(t.z + g * R + l) * K + j0);
+#pragma unroll
+    for (int j = 0; j < KC; j++) yp[j] = mine[j];
+  }
 }
 
 // Y = A X for K vectors stored interleaved (entry j of dof i at i K + j, the
-// layout of a BaseVector with K components): each block's values and column
-// numbers are loaded once and used for all K vectors; the x entries of G
-// components of a value's column come in one pass (16-byte loads), then
-// each component goes through the single kernel's products (16 KB of LDS)
-// and row sums in the same order, so each column of Y is bit-identical to
-// a single apply.
-template <int NNZ, int G>
-__global__ __launch_bounds__(kStreamBlock, NNZ <= 2048 && G == 1 ? 8 : 4) void CsrRunsMultiKernel(
-    const int* __restrict__ run_row, const int* __restrict__ run_ptr, const int* __restrict__ val_ptr,
+// layout of a BaseVector with K components): the runs kernel with KC row sums
+// per value (the KC components of a column's x are adjacent), the components
+// in passes of KC = 4, 2, 1.  Each component is summed in the single kernel's
+// order: bit-identical to a single apply.
+__global__ __launch_bounds__(kStreamBlock, 3) void CsrRunsMultiKernel(
+    const int4* __restrict__ tasks, int ntasks, const int* __restrict__ run_ptr,
     const int* __restrict__ rcols, const double* __restrict__ rvals, const double* __restrict__ x,
-    double* __restrict__ y, int K, const int* __restrict__ blk_run, const int* __restrict__ blk_len, int nblocks,
-    int blocks_per_wg, const int* __restrict__ stop) {
+    double* __restrict__ y, int K, const int* __restrict__ stop) {
   if (stop && *stop) return;
-  constexpr int PER = NNZ / kStreamBlock;
-  __shared__ double prod[NNZ];
-  __shared__ double lds[kStreamBlock / 64];
-  const int tid = threadIdx.x;
-  const int lb = XcdContiguousBlock(blockIdx.x, gridDim.x);
-  const int b0 = lb * blocks_per_wg;
-  const int b1 = min(b0 + blocks_per_wg, nblocks);
-  int u0 = 0, u1 = 0, R = 1, inv = 65536, c0 = 0, vb = 0, nv = 0;
-  int c[PER];
-  double v[PER];
-  auto fetch = [&](int b) {
-    u0 = blk_run[b];
-    u1 = blk_run[b + 1];
-    R = blk_len[b];
-    inv = (65536 + R - 1) / R;
-    c0 = run_ptr[u0];
-    vb = val_ptr[u0];
-    nv = val_ptr[u1] - vb;
-    if (nv > NNZ) return;
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int k = tid + i * kStreamBlock;
-      const int kk = k < nv ? k : 0;
-      c[i] = __builtin_nontemporal_load(&rcols[c0 + RunDiv(kk, inv)]);
-      v[i] = __builtin_nontemporal_load(&rvals[vb + kk]);
+  WalkRunTasks(tasks, ntasks, run_ptr, XcdContiguousBlock(blockIdx.x, gridDim.x), gridDim.x, 0, [&](const RunHead& h) __attribute__((always_inline)) {
+    const int R = (h.t.w >> 8) & 0xff;
+    int j0 = 0;
+    while (j0 < K) {
+      // 8 components at once up to 3 rows: 48 registers of sums
+      const int rem = K - j0, kc = rem >= 8 && R <= 3 ? 8 : rem >= 4 ? 4 : rem >= 2 ? 2 : 1;
+      auto go = [&](auto comps) __attribute__((always_inline)) {
+        constexpr int KC = decltype(comps)::value;
+        ForRunShape<KC>(R, h.t.w >> 24, [&](auto r, auto u) __attribute__((always_inline)) {
+          RunTaskRowsMulti<decltype(r)::value, decltype(u)::value, KC>(h, rcols, rvals, x, y, K, j0);
+        });
+      };
+      if (kc == 8) go(std::integral_constant<int, 8>{});
+      else if (kc == 4) go(std::integral_constant<int, 4>{});
+      else if (kc == 2) go(std::integral_constant<int, 2>{});
+      else go(std::integral_constant<int, 1>{});
+      j0 += kc;
     }
-  };
-  if (b0 < b1) fetch(b0);
-  for (int b = b0; b < b1; b++) {
-    if (nv > NNZ) {
-      const int r = run_row[u0];
-      for (int j = 0; j < K; j++) {
-        double a = 0.0;
-        for (int k = tid; k < nv; k += kStreamBlock)
-          a += rvals[vb + k] * x[(int64_t)rcols[c0 + k] * K + j];
-        a = BlockSum<kStreamBlock>(a, lds);
-        if (tid == 0) y[(int64_t)r * K + j] = a;
-      }
-      if (b + 1 < b1) fetch(b + 1);
-      continue;
-    }
-    const int row0 = run_row[u0];
-    const int nr = (u1 - u0) * R;
-    int tpr = 64;
-    while (tpr > 1 && tpr * nr > kStreamBlock) tpr >>= 1;
-    const int l = tid & (tpr - 1);
-    for (int j0 = 0; j0 < K; j0 += G) {
-      // x of the G components of each value's column: loaded together
-      double xg[PER][G];
-#pragma unroll
-      for (int i = 0; i < PER; i++) {
-        const double* xp = x + (int64_t)c[i] * K + j0;
-        if constexpr (G == 1) {
-          xg[i][0] = xp[0];
-        } else {
-#pragma unroll
-          for (int h = 0; h < G / 2; h++) {
-            const double2 t = reinterpret_cast<const double2*>(xp)[h];
-            xg[i][2 * h] = t.x;
-            xg[i][2 * h + 1] = t.y;
-          }
-        }
-      }
-      // then, component by component, the single kernel's products and sums
-#pragma unroll
-      for (int g = 0; g < G; g++) {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-          const int k = tid + i * kStreamBlock;
-          prod[k] = k < nv ? v[i] * xg[i][g] : 0.0;
-        }
-        __syncthreads();
-        for (int jr = 0; jr < nr; jr += kStreamBlock / tpr) {
-          const int j = jr + tid / tpr;
-          double sum = 0.0;
-          if (j < nr) {
-            const int run = RunDiv(j, inv), q = j - run * R;
-            const int s0 = run_ptr[u0 + run] - c0, s1 = run_ptr[u0 + run + 1] - c0;
-            double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-            int k = s0 + l;
-            for (; k + 3 * tpr < s1; k += 4 * tpr) {
-              a0 += prod[k * R + q];
-              a1 += prod[(k + tpr) * R + q];
-              a2 += prod[(k + 2 * tpr) * R + q];
-              a3 += prod[(k + 3 * tpr) * R + q];
-            }
-            for (; k < s1; k += tpr) a0 += prod[k * R + q];
-            sum = (a0 + a1) + (a2 + a3);
-          }
-          for (int off = tpr / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-          if (j < nr && l == 0) y[(int64_t)(row0 + j) * K + j0 + g] = sum;
-        }
-        __syncthreads();
-      }
-    }
-    if (b + 1 < b1) fetch(b + 1);
-  }
+  });
 }
 
 // Component j of an interleaved K-vector to a plain vector and back (the
@@ -434,6 +475,21 @@ template <bool ACCUM, bool DOT>
 static int LaunchSpmv(const CsrOp& A, double s, const double* x, double* y, hipStream_t st, double* partials,
                       const int* stop, int reverse = 0);
 
+// Workgroups of a runs launch: one task per wavefront if cap allows, a
+// multiple of 8 beyond 8 (the XCD mapping).
+static int RunsGrid(const CsrOp& A, int cap) {
+  const int wg = A.nblocks <= 8 ? A.nblocks : (A.nblocks + 7) & ~7;
+  return std::max(1, std::min(wg, cap > 8 ? cap & ~7 : cap));
+}
+
+// The runs kernel with partial sums: a fold kernel (4.4 us) follows a grid of
+// over 1024 workgroups, so up to 6144 workgroups' worth of tasks run on 1024
+// (CG iteration on 128^2 p=5, 5,100: 41.8 -> 39.2 us; 23x19x27 p=3, 9,300:
+// 57.5 against 57.9, 20x16x24 p=4, 11,500: 100.5 against 103.2).
+static int RunsDotCap(const CsrOp& A) {
+  return std::min(A.walk_grid, A.nblocks <= 6144 ? 1024 : kMaxWideBlocks);
+}
+
 void CsrOp::MultMulti(int K, const double* x, double* y, hipStream_t st, const int* stop) {
   NGSAMD_REQUIRE(K >= 1 && K <= 64, "multi-vector apply: 1 <= K <= 64 vectors");
   if (height == 0) return;
@@ -443,26 +499,8 @@ void CsrOp::MultMulti(int K, const double* x, double* y, hipStream_t st, const i
     return;
   }
   if (algo == 2) {
-    auto pick = [&](auto g) {
-      constexpr int Gc = decltype(g)::value;
-      return block_nnz == 1024 ? CsrRunsMultiKernel<1024, Gc>
-             : block_nnz == 4096 ? CsrRunsMultiKernel<4096, Gc>
-                                 : CsrRunsMultiKernel<2048, Gc>;
-    };
-    // x of four components per pass when K allows (two 16-byte loads per
-    // value, more registers: 4 workgroups per CU); NGSAMD_MULTI_PASS=2 keeps
-    // two per pass (for comparison)
-    const char* pass_env = getenv("NGSAMD_MULTI_PASS");
-    const bool four = K % 4 == 0 && !(pass_env && std::string(pass_env) == "2");
-    auto kern = four ? pick(std::integral_constant<int, 4>{})
-                : (K % 2 == 0) ? pick(std::integral_constant<int, 2>{})
-                               : pick(std::integral_constant<int, 1>{});
-    int wg = nblocks < max_grid ? nblocks : max_grid;
-    if (wg > 8) wg &= ~7;
-    if (wg < 1) wg = 1;
-    const int per = (nblocks + wg - 1) / wg;
-    kern<<<wg, kStreamBlock, 0, st>>>(run_row.p, run_ptr.p, val_ptr.p, rcols.p, rvals.p, x, y, K, blk_run.p,
-                                      blk_len.p, nblocks, per, stop);
+    CsrRunsMultiKernel<<<RunsGrid(*this, walk_grid), kStreamBlock, 0, st>>>(tasks.p, ntasks, run_ptr.p, rcols.p,
+                                                                           rvals.p, x, y, K, stop);
     NGSAMD_CHECK_LAUNCH();
     return;
   }
@@ -490,6 +528,38 @@ __global__ void RunsDiagKernel(const int* __restrict__ run_row, const int* __res
       d[r0 + q] = val;
     }
   }
+}
+
+// Lanes per run of R rows and L columns (log2): the fewest, from 8 (16 for
+// runs of 4 and more rows and 9 and more columns), whose first pass covers the
+// run.  us per apply with at least 8 / 16 lanes: 128^2 p=5 (runs of 4 and 6
+// rows) 27.2 / 21.7; runs of up to 3 rows 32^3 p=4 327 / 340, 64^2 p=3 4.4 /
+// 4.8.
+static int RunGroupLog2(int R, int L) {
+  int lg = L <= 8 || R < 4 ? 3 : 4;
+  while (lg < 6 && L > RunUnroll(R) << lg) lg++;
+  return lg;
+}
+
+// The runs kernel's tasks: consecutive runs of equal length (rows) and group
+// size, at most one wavefront's lanes; slots per lane are those of the
+// task's longest run.
+static std::vector<int4> RunTasks(const std::vector<int>& rr, const std::vector<int>& rpp, const std::vector<int>& vp) {
+  std::vector<int4> tk;
+  const int nruns = (int)rr.size() - 1;
+  for (int u = 0; u < nruns;) {
+    const int R = rr[u + 1] - rr[u], lg = RunGroupLog2(R, rpp[u + 1] - rpp[u]);
+    int n = 1, len = rpp[u + 1] - rpp[u];
+    while (n < (64 >> lg) && u + n < nruns && rr[u + n + 1] - rr[u + n] == R &&
+           RunGroupLog2(R, rpp[u + n + 1] - rpp[u + n]) == lg) {
+      len = std::max(len, rpp[u + n + 1] - rpp[u + n]);
+      n++;
+    }
+    const int m = std::max(1, std::min(127, (len + (1 << lg) - 1) >> lg));
+    tk.push_back(make_int4(u, vp[u], rr[u], n | R << 8 | lg << 16 | m << 24));
+    u += n;
+  }
+  return tk;
 }
 
 CsrOp::CsrOp(int64_t h, int64_t w, const int64_t* rp, const int* c, const double* v)
@@ -549,29 +619,28 @@ CsrOp::CsrOp(int64_t h, int64_t w, const int64_t* rp, const int* c, const double
     if (algo_name == "runs" || 4 * nshared <= 3 * nnz) {
       algo = 2;
       nruns = (int64_t)rr.size() - 1;
-      nblocks = (int)br.size() - 1;
-      // Up to 4096 blocks: one block per workgroup (all resident at once;
-      // 128^2 p=3, 1.2K blocks: 8.4 us against 12.1 us on 1024 workgroups).
-      // Beyond: about three blocks per workgroup, so that each workgroup's
-      // next block is in flight (16^3 p=4, 20M nonzeros: 57 us on 4096
-      // workgroups against 78 us on one block per workgroup), at most 16384.
-      if (!grid_env && nblocks > 4096) max_grid = std::max(4096, std::min(16384, nblocks / 3));
+      std::vector<int4> tk = RunTasks(rr, rpp, vp);
+      ntasks = (int)tk.size();
+      tasks.alloc(std::max<size_t>(tk.size(), 1));
+      if (!tk.empty()) tasks.upload(tk.data(), tk.size());
+      nblocks = (ntasks + kRunWaves - 1) / kRunWaves;
+      // One task per wavefront (32^3 p=4, 53K workgroups: 298 us per apply;
+      // 16,384 workgroups 327, 2,048, the resident ones, 361).  Several
+      // vectors' sums fill the registers: there a wavefront of 16,384
+      // workgroups walks its tasks, each one's records loaded ahead (4
+      // vectors 563 us against 650 with one task each).
+      if (!grid_env) {
+        max_grid = 1 << 28;
+        walk_grid = 16384;
+        if (nblocks > 4096) walk_grid = std::max(4096, std::min(16384, nblocks / 3));
+      } else {
+        walk_grid = max_grid;
+      }
       run_row.alloc(rr.size());
       run_ptr.alloc(rpp.size());
       val_ptr.alloc(vp.size());
-      // 4 padding entries (column 0, value 0): the kernel's lanes past the
-      // end of the last block read entry nshared / nnz
-      rcols.alloc(nshared + 4);
-      rvals.alloc(nnz + 4);
-      {
-        const int zc[4] = {0, 0, 0, 0};
-        const double zv[4] = {0, 0, 0, 0};
-        rcols.upload_at(zc, nshared, 4);
-        rvals.upload_at(zv, nnz, 4);
-        NGSAMD_HIP(hipStreamSynchronize(Stream()));
-      }
-      blk_run.alloc(br.size());
-      blk_len.alloc(std::max<size_t>(bl.size(), 1));
+      rcols.alloc(std::max<int64_t>(nshared, 1));
+      rvals.alloc(std::max<int64_t>(nnz, 1));
       run_row.upload(rr.data(), rr.size());
       run_ptr.upload(rpp.data(), rpp.size());
       val_ptr.upload(vp.data(), vp.size());
@@ -586,8 +655,6 @@ CsrOp::CsrOp(int64_t h, int64_t w, const int64_t* rp, const int* c, const double
         row_run.upload(rrun.data(), rrun.size());
         NGSAMD_HIP(hipStreamSynchronize(Stream()));
       }
-      blk_run.upload(br.data(), br.size());
-      if (!bl.empty()) blk_len.upload(bl.data(), bl.size());
       NGSAMD_HIP(hipStreamSynchronize(Stream()));
       return;
     }
@@ -704,22 +771,11 @@ static int LaunchStream(const CsrOp& A, double s, const double* x, double* y, hi
 template <bool ACCUM, bool DOT>
 static int LaunchRuns(const CsrOp& A, double s, const double* x, double* y, hipStream_t st, double* partials,
                       const int* stop, int reverse) {
-  auto kern = A.block_nnz == 1024   ? CsrRunsKernel<1024, ACCUM, DOT>
-              : A.block_nnz == 4096 ? CsrRunsKernel<4096, ACCUM, DOT>
-                                    : CsrRunsKernel<2048, ACCUM, DOT>;
-  // a wide grid (many more workgroups than resident slots) lets the hardware
-  // balance blocks of uneven cost: measured faster than one workgroup per
-  // resident slot (412 vs 452 us for the runs kernel at 32^3 p=4); the
-  // variant with partial sums stays within the partials workspace
-  const int cap = DOT ? std::min(A.max_grid, kMaxWideBlocks) : A.max_grid;
-  int wg = A.nblocks < cap ? A.nblocks : cap;
-  if (wg > 8) wg &= ~7;
-  if (wg < 1) wg = 1;
-  const int per = (A.nblocks + wg - 1) / wg;
-  kern<<<(int)wg, kStreamBlock, 0, st>>>(A.run_row.p, A.run_ptr.p, A.val_ptr.p, A.rcols.p, A.rvals.p, x, y,
-                                         A.blk_run.p, A.blk_len.p, A.nblocks, per, s, partials, stop, reverse);
+  const int wg = RunsGrid(A, DOT ? RunsDotCap(A) : A.max_grid);
+  CsrRunsKernel<ACCUM, DOT><<<wg, kStreamBlock, 0, st>>>(A.tasks.p, A.ntasks, A.run_ptr.p, A.rcols.p, A.rvals.p, x,
+                                                         y, s, partials, stop, reverse);
   NGSAMD_CHECK_LAUNCH();
-  return (int)wg;
+  return wg;
 }
 
 template <bool ACCUM, bool DOT>
@@ -752,6 +808,7 @@ void CsrOp::Mult(const double* x, double* y, hipStream_t st) {
 // LaunchStream and LaunchSpmvG choose them.
 static int DotWorkgroups(const CsrOp& A) {
   if (A.algo == 0) return kMaxReduceBlocks;  // at most this many (LaunchSpmvG)
+  if (A.algo == 2) return RunsGrid(A, RunsDotCap(A));
   const int cap = std::min(A.max_grid, kMaxWideBlocks);
   int wg = A.nblocks < cap ? A.nblocks : cap;
   if (wg > 8) wg &= ~7;
