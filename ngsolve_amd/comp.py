@@ -180,7 +180,7 @@ def Integrate(cf, mesh, element_wise=False, order=5):
         fes = cf.a.space
         if cf.b.space.mesh.ngmesh is not fes.mesh.ngmesh or mesh.ngmesh is not fes.mesh.ngmesh:
             raise ValueError("Integrate: the grid functions must live on the mesh that is integrated over")
-        mf = DevMatrixFree(fes, max(2 * fes.order - 2, 1), None, "f64")
+        mf = DevMatrixFree(fes, max(2 * fes.order - 2, 1), None, "f64", atomic=True)  # element tables only
         g = N.DeviceVector(mf.op.ne, 8)
         mf.op.element_grad(cf.a.vec._device(), cf.b.vec._device(), g)
         vals = -g.download()  # element_grad gives -(a_e^T K_e b_e) / kappa_e with kappa = 1
@@ -476,13 +476,14 @@ class BilinearForm:
             term, meas = self.integrals[0]
             order = self._order(term, meas)
             if term.kind == "laplace":
-                mf = DevMatrixFree(fes, order, self._coef(term), "f64")
+                # only the element tables are used: no tables of the gather's patches
+                mf = DevMatrixFree(fes, order, self._coef(term), "f64", atomic=True)
                 rowptr, cols = N.PatternDevice(mf.op)
                 op = N.AssembleCSRDevice(mf.op, rowptr, cols)
             else:
                 # the mesh and dof tables of a matrix-free operator, the mass
                 # form's own rule and coefficient
-                mf = DevMatrixFree(fes, max(2 * fes.order - 2, 1), None, "f64")
+                mf = DevMatrixFree(fes, max(2 * fes.order - 2, 1), None, "f64", atomic=True)
                 rowptr, cols = N.PatternDevice(mf.op)
                 ir = fes.integration_rule(order)
                 shape = np.ascontiguousarray(np.stack([c["shape"] for c in N.BuildClasses(fes.space, ir)]))

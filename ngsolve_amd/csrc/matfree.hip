@@ -39,54 +39,14 @@
 #include "common.hpp"
 #include "half.hpp"
 #include "matfree.hpp"
+#include "mfdev.hpp"
 #include "reduce.hpp"
 #include "runtime_state.hpp"
 
 namespace ngsamd {
 
-typedef double double4v __attribute__((ext_vector_type(4)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-
 constexpr int kMfWaves = 8;
 constexpr int kMfBlock = 64 * kMfWaves;
-
-__device__ __forceinline__ double4v Mfma(double a, double b, double4v c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ float4v Mfma(float a, float b, float4v c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-template <class T> struct Acc4;
-template <> struct Acc4<double> { typedef double4v type; };
-template <> struct Acc4<float> { typedef float4v type; };
-
-// Row of the 16x16 result held in accumulator element r of a lane in lane
-// group grp = lane/16 (the column is lane%16).  Measured on gfx950:
-// v_mfma_f32_16x16x4f32 holds rows 4*grp+r, v_mfma_f64_16x16x4f64 holds
-// rows grp+4*r.
-template <class T>
-__device__ __forceinline__ constexpr int AccRow(int grp, int r) {
-  return sizeof(T) == 8 ? grp + 4 * r : 4 * grp + r;
-}
-
-template <class V>
-__device__ __forceinline__ void AtomicAddV(V* p, V v) {
-  atomicAdd(p, v);
-}
-
-// Metric G (symmetric, packed) times vector: 2D (xx,yy,xy), 3D (xx,yy,zz,xy,xz,yz).
-template <int DIM, class T>
-__device__ __forceinline__ void ApplyMetric(const T* g, const T* u, T* v) {
-  if constexpr (DIM == 2) {
-    v[0] = g[0] * u[0] + g[2] * u[1];
-    v[1] = g[2] * u[0] + g[1] * u[1];
-  } else {
-    v[0] = g[0] * u[0] + g[3] * u[1] + g[4] * u[2];
-    v[1] = g[3] * u[0] + g[1] * u[1] + g[5] * u[2];
-    v[2] = g[4] * u[0] + g[5] * u[1] + g[2] * u[2];
-  }
-}
 
 // Work schedule shared by the MFMA kernels: the element tiles (16 elements)
 // of every class are numbered class after class in rounds of kMfWaves tiles,
@@ -104,27 +64,6 @@ struct MfRounds {
 
 // classes whose schedule the reference-matrix kernels keep in LDS
 constexpr int kMaxLdsClasses = 64;
-
-// Copy n 16-byte words of a class's matrices from global memory into LDS.
-// Each thread issues 4 loads before its first LDS write (from clamped
-// indices, so no load sits behind a branch): a plain load-then-store loop
-// waits for every load in turn.
-template <int BLOCK = kMfBlock>
-__device__ __forceinline__ void CopyToLds(void* dst, const void* src, int n) {
-  constexpr int U = 4;
-  const uint4* s = reinterpret_cast<const uint4*>(src);
-  uint4* d = reinterpret_cast<uint4*>(dst);
-  for (int base = 0; base < n; base += BLOCK * U) {
-    uint4 v[U];
-#pragma unroll
-    for (int j = 0; j < U; j++) v[j] = s[min(base + j * BLOCK + (int)threadIdx.x, n - 1)];
-#pragma unroll
-    for (int j = 0; j < U; j++) {
-      const int i = base + j * BLOCK + (int)threadIdx.x;
-      if (i < n) d[i] = v[j];
-    }
-  }
-}
 
 // Class of round r, scanning on from the class of the previous round.
 __device__ __forceinline__ int RoundClass(const MfRounds& R, int r, int from) {
@@ -163,7 +102,7 @@ __global__ __launch_bounds__(kMfBlock) void MfMfmaKernel(
     if (c != cls) {
       if (cls >= 0) __syncthreads();
       // nlds * sizeof(T) and the class offset are multiples of 64 bytes
-      CopyToLds(lb, bmat + (int64_t)c * bstride, (int)(nlds * sizeof(T) / 16));
+      CopyToLds<kMfBlock>(lb, bmat + (int64_t)c * bstride, (int)(nlds * sizeof(T) / 16));
       __syncthreads();
       cls = c;
     }
@@ -260,18 +199,6 @@ __global__ __launch_bounds__(kMfBlock) void MfMfmaKernel(
 //   B1[q][d][K1P]            first product, dofs contiguous (K1P = nd -> 8k)
 //   B2[chunk][d][MT*16][32]  second product, the 32 points of a chunk in the
 //                            order the first product's accumulators hold them
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-template <class H> struct Vec8;
-template <> struct Vec8<__bf16> { typedef bf16x8 type; };
-template <> struct Vec8<_Float16> { typedef half8 type; };
-__device__ __forceinline__ float4v Mfma16(bf16x8 a, bf16x8 b, float4v c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ float4v Mfma16(half8 a, half8 b, float4v c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
 template <class H, int DIM, int KS1, int MT, int MODE, class V>
 __global__ __launch_bounds__(kMfBlock) void MfBf16Kernel(
     const uint16_t* __restrict__ bmat, int64_t bstride, MfRounds R, int k1p, int nqc,
@@ -297,7 +224,7 @@ __global__ __launch_bounds__(kMfBlock) void MfBf16Kernel(
     if (cl != cls) {
       if (cls >= 0) __syncthreads();
       // B1 and B2 of the class: bstride 16-bit words, a multiple of 8
-      CopyToLds(lds_raw, bmat + (int64_t)cl * bstride, (int)(bstride / 8));
+      CopyToLds<kMfBlock>(lds_raw, bmat + (int64_t)cl * bstride, (int)(bstride / 8));
       __syncthreads();
       cls = cl;
     }
@@ -482,7 +409,7 @@ __global__ __launch_bounds__(kMfBlock) void MfRefKernel(
     if (c != cls) {
       if (cls >= 0) __syncthreads();
       // sstride * sizeof(T) is a multiple of 16 bytes
-      CopyToLds(ls, smat + (int64_t)c * sstride, (int)(sstride * sizeof(T) / 16));
+      CopyToLds<kMfBlock>(ls, smat + (int64_t)c * sstride, (int)(sstride * sizeof(T) / 16));
       __syncthreads();
       cls = c;
     }
@@ -601,7 +528,7 @@ __global__ __launch_bounds__(kMfBlock) void MfRef16Kernel(
     if (cl != cls) {
       if (cls >= 0) __syncthreads();
       // sstride 16-bit words, a multiple of 8
-      CopyToLds(lds_raw, smat + (int64_t)cl * sstride, (int)(sstride / 8));
+      CopyToLds<kMfBlock>(lds_raw, smat + (int64_t)cl * sstride, (int)(sstride / 8));
       __syncthreads();
       cls = cl;
     }
@@ -770,7 +697,7 @@ __global__ __launch_bounds__(kMfBlock) void MfFacKernel(
     while (s_round0[c + 1] <= rd) c++;
     if (c != cls) {
       if (cls >= 0) __syncthreads();
-      CopyToLds(ls, fmat + (int64_t)c * fstride, (int)(fstride * sizeof(T) / 16));
+      CopyToLds<kMfBlock>(ls, fmat + (int64_t)c * fstride, (int)(fstride * sizeof(T) / 16));
       __syncthreads();
       cls = c;
     }
@@ -1665,6 +1592,14 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
   kappa.alloc(ne_global);
   kappa.upload(kap.data(), ne_global);
 
+  // patch kernels where every class is a relabelling of the first one
+  // (NGSAMD_MF_PATCH=0: the general gather, =1: patches whatever the size, for
+  // comparison)
+  const char* penv = getenv("NGSAMD_MF_PATCH");
+  if (fac_kernel && scat == NGSAMD_SCATTER_GATHER && PatchShape(dim, nd, fac_kg) && !(penv && std::string(penv) == "0"))
+    patch.ok = patch.Build(dim, nd, ndof, half, prec == NGSAMD_PREC_F64, ks1, fstride * (half ? 2 : prec == NGSAMD_PREC_F64 ? 8 : 4),
+                           classes, S, hdofs, hmetric, el.data(), DeviceMaxLds(),
+                           penv && std::string(penv) == "1" ? 1 : 8192);
   std::vector<int> gather_slots;  // element-major slots in gather order (kept for the tile-major copy)
   // dof -> contribution slots, ascending slot order (the order of each sum)
   std::vector<int> cnt(ndof + 1, 0);
@@ -1685,7 +1620,7 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
     // among a dof's contributions, so the dofs reading one 16-element line
     // are gathered together (BF16 apply with FP64 vectors 75 -> 71 us, split
     // FP16 with FP32 vectors 56 -> 54 us at 32^3 p=4)
-    const bool tiled16 = use_mfma && fac_kernel && half;
+    const bool tiled16 = use_mfma && fac_kernel && half && !patch.ok;
     int64_t kmax = ne_global;
     std::vector<int> rowkey;
     if (tiled16) {
@@ -1700,27 +1635,32 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
       }
       kmax = tb * nd * 16;
     }
-    std::vector<int> key(ndof, (int)kmax);
-    for (int64_t i = 0; i < nel * nd; i++)
-      key[hdofs[i]] = std::min(key[hdofs[i]], tiled16 ? rowkey[i] : el[i / nd]);
-    std::vector<int> kc(kmax + 2, 0);
-    for (int64_t d = 0; d < ndof; d++) kc[key[d] + 1]++;
-    for (int64_t k = 0; k <= kmax; k++) kc[k + 1] += kc[k];
     std::vector<int> order(ndof);
-    for (int64_t d = 0; d < ndof; d++) order[kc[key[d]]++] = (int)d;
-    // Inside each workgroup's range of the gather kernel (the launch grid
-    // depends on ndof only), dofs by decreasing contribution count (stable):
-    // the wavefronts of a range then hold dofs of like count, so a vertex dof
-    // (up to 24 contributions on tets) no longer holds up a wavefront of
-    // edge, face and cell dofs (2 to 6).  Which dofs a workgroup gathers and
-    // each dof's summation order are unchanged.
-    if (ndof > 0) {
-      const int64_t grid = GridFor(ndof, kGatherBlock, kMaxWideBlocks);
-      const int64_t per = (ndof + grid - 1) / grid;
-      for (int64_t a = 0; a < ndof; a += per) {
-        const int64_t b = std::min<int64_t>(ndof, a + per);
-        std::stable_sort(order.begin() + a, order.begin() + b,
-                         [&](int u, int v) { return cnt[u + 1] - cnt[u] > cnt[v + 1] - cnt[v]; });
+    // (with patches only the diagonal and the linear form gather this way: by number)
+    if (patch.ok) {
+      for (int64_t d = 0; d < ndof; d++) order[d] = (int)d;
+    } else {
+      std::vector<int> key(ndof, (int)kmax);
+      for (int64_t i = 0; i < nel * nd; i++)
+        key[hdofs[i]] = std::min(key[hdofs[i]], tiled16 ? rowkey[i] : el[i / nd]);
+      std::vector<int> kc(kmax + 2, 0);
+      for (int64_t d = 0; d < ndof; d++) kc[key[d] + 1]++;
+      for (int64_t k = 0; k <= kmax; k++) kc[k + 1] += kc[k];
+      for (int64_t d = 0; d < ndof; d++) order[kc[key[d]]++] = (int)d;
+      // Inside each workgroup's range of the gather kernel (the launch grid
+      // depends on ndof only), dofs by decreasing contribution count (stable):
+      // the wavefronts of a range then hold dofs of like count, so a vertex dof
+      // (up to 24 contributions on tets) no longer holds up a wavefront of
+      // edge, face and cell dofs (2 to 6).  Which dofs a workgroup gathers and
+      // each dof's summation order are unchanged.
+      if (ndof > 0) {
+        const int64_t grid = GridFor(ndof, kGatherBlock, kMaxWideBlocks);
+        const int64_t per = (ndof + grid - 1) / grid;
+        for (int64_t a = 0; a < ndof; a += per) {
+          const int64_t b = std::min<int64_t>(ndof, a + per);
+          std::stable_sort(order.begin() + a, order.begin() + b,
+                           [&](int u, int v) { return cnt[u + 1] - cnt[u] > cnt[v + 1] - cnt[v]; });
+        }
       }
     }
     std::vector<int> prp(ndof + 1, 0), psl(sl.size());
@@ -1767,7 +1707,7 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
   // tile-major tables of the factored kernels: a wavefront's load of one dof
   // row (or metric component) of its 16 elements covers one or two lines
   // instead of 16
-  if (fac_kernel) {
+  if (fac_kernel && !patch.ok) {
     std::vector<int> tb(nclass + 1, 0);
     for (int c = 0; c < nclass; c++) tb[c + 1] = tb[c] + (int)((off[c + 1] - off[c] + 15) / 16);
     const int64_t nt = tb[nclass];
@@ -1822,6 +1762,10 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
   LaunchElements<1, double>(*this, nullptr, nullptr, 1.0, nullptr, nullptr, true);
   LaunchElements<0, float>(*this, nullptr, nullptr, 1.0, nullptr, nullptr, true);
   LaunchElements<1, float>(*this, nullptr, nullptr, 1.0, nullptr, nullptr, true);
+  if (patch.ok) {
+    PatchApply<double>(*this, nullptr, nullptr, 1.0, 0, nullptr, nullptr, nullptr, true);
+    PatchApply<float>(*this, nullptr, nullptr, 1.0, 0, nullptr, nullptr, nullptr, true);
+  }
   NGSAMD_HIP(hipStreamSynchronize(Stream()));
 }
 
@@ -2200,6 +2144,31 @@ int MatFreeOp::Apply(double s, const V* x, V* y, bool accumulate, const int* sto
     }
     LaunchElements<1, V>(*this, x, y, s, stop, st, false);
     return 0;
+  }
+  if (patch.ok) {
+    // x and y overlap: from a copy (the general gather reads all of x first)
+    if (x < y + height && y < x + height) {
+      V* copy;
+      if constexpr (sizeof(V) == 8) copy = reinterpret_cast<V*>(contrib64.p);
+      else copy = reinterpret_cast<V*>(contrib32.p);
+      NGSAMD_HIP(hipMemcpyAsync(copy, x, sizeof(V) * height, hipMemcpyDeviceToDevice, st));
+      x = copy;
+    }
+    const bool dot = partials && !accumulate && s == 1.0;
+    double* wgsum = dot ? (wide ? wide : State().wide_partials) : nullptr;
+    const int nsum = patch.Grid(sizeof(V) == 8);
+    PatchApply<V>(*this, x, y, s, accumulate ? 1 : 0, stop, st, wgsum, false);
+    if (patch.nshared > 0) {
+      const int ng = GridFor(patch.nshared, kGatherBlock, kMaxWideBlocks);
+      MfGatherKernel<double, V, false><<<ng, kGatherBlock, 0, st>>>(
+          patch.s_rowptr.p, patch.s_slots.p, patch.s_order.p, patch.part.p, y, patch.nshared, s, accumulate ? 1 : 0,
+          stop, nullptr, nullptr, wgsum, nsum, partials);
+      NGSAMD_CHECK_LAUNCH();
+      return dot ? std::min(kFoldedPartials, ng) : 0;
+    }
+    if (!dot) return 0;
+    LaunchFoldPartials(wgsum, nsum, partials, stop, st);
+    return kFoldedPartials;
   }
   // contribution buffers are allocated by the constructor: nothing here
   // allocates, so the apply can be captured into a graph

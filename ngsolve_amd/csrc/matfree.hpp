@@ -11,7 +11,47 @@ struct MfClass {
   int64_t begin = 0, end = 0;  // element range in the (class-sorted) tables
 };
 
+// The patch kernels' tables (mfpatch.hip): elements in patches of 16 * waves
+// of one reference class, per patch its dofs in groups of 64 with the LDS
+// positions of their contributions, and the gather of the dofs that several
+// patches share.
+struct MfPatchPlan {
+  bool ok = false;
+  int waves = 0, npatch = 0;
+  int nx = 0;               // x entries of a patch in LDS
+  size_t lds = 0;
+  mutable int occ[2] = {1, 1};  // resident workgroups per CU [FP64 vectors]
+  int64_t nshared = 0;      // dofs of several patches
+  DevBuf<int4> d_hdr;
+  DevBuf<int> d_xdof, d_elnr;
+  DevBuf<int2> d_grp;
+  DevBuf<uint16_t> d_js, d_jx, d_lidx;
+  DevBuf<double> d_metric;
+  DevBuf<int> s_rowptr, s_slots, s_order;  // shared dofs: their partial sums
+  DevBuf<double> part;
+  // false: fewer than min_elements, some class is no relabelling of class 0, a dof belongs to no
+  // element, or a patch does not fit into LDS
+  bool Build(int dim, int nd, int64_t ndof, bool half, bool f64, int ks1, int64_t fbytes,
+             const std::vector<MfClass>& classes, const std::vector<double>& S, const int* dofs, const double* metric,
+             const int* elnr, int max_lds, int64_t min_elements);
+  int Grid(bool f64_vectors) const {
+    const int64_t resident = (int64_t)DeviceCUs() * occ[f64_vectors ? 1 : 0];
+    return (int)(npatch < resident ? npatch : resident);
+  }
+};
+
+struct MatFreeOp;
+// shapes with an instance of the patch kernels
+bool PatchShape(int dim, int nd, int kg);
+// y = (accumulate ? y : 0) + s A x on the inner dofs, partial sums of the
+// shared ones; with partials one partial of <x, A x> per workgroup.  prepare:
+// set up the kernel instance only.
+template <class V>
+void PatchApply(const MatFreeOp& A, const V* x, V* y, double s, int accumulate, const int* stop, hipStream_t st,
+                double* partials, bool prepare);
+
 struct MatFreeOp : ngsamd_op_s {
+  MfPatchPlan patch;
   int dim = 3, nd = 0, nq = 0, ncomp = 6;
   int ndp = 0;                // nd padded to a multiple of 4 (MFMA K)
   int nqp = 0;                // nq padded to a multiple of 16

@@ -1,0 +1,126 @@
+"""The matrix-free apply over element patches against the general gather
+(NGSAMD_MF_PATCH=0) and the oracle: every order, structured meshes whose
+element count leaves a partial tile, a partial patch or a single patch, 4- and
+8-tile patches, unstructured meshes, every precision, FP32 and FP64 vectors,
+accumulation, overlapping vectors, a changed coefficient, CG's inner product."""
+import numpy as np
+import pytest
+
+from oracle import fe_oracle as O
+from helpers import N, dvec, say
+
+pytestmark = pytest.mark.gpu
+
+import ngsolve_amd as ngs  # noqa: E402
+
+TOL = {"f64": 1e-14, "f32": 2e-6, "f16x3": 2e-6, "f16": 4e-3, "bf16": 3e-2}
+
+
+def build(monkeypatch, fes, kappa, precision, patch):
+    monkeypatch.setenv("NGSAMD_MF_PATCH", "1" if patch else "0")
+    u, v = fes.TnT()
+    return ngs.BilinearForm(ngs.ElementCoefficient(kappa) * ngs.grad(u) * ngs.grad(v) * ngs.dx,
+                            mf=ngs.MFOpts(precision=precision)).Assemble().mat
+
+
+def compare(monkeypatch, mesh, p, precision):
+    fes = ngs.H1(mesh, order=p, dirichlet=".*")
+    rng = np.random.default_rng(7)
+    kappa = np.exp(rng.standard_normal(mesh.ne))
+    A, B = build(monkeypatch, fes, kappa, precision, True), build(monkeypatch, fes, kappa, precision, False)
+    x = rng.uniform(-1, 1, fes.ndof)
+    out = []
+    for M in (A, B):
+        dx, dy = dvec(x), dvec(np.full(fes.ndof, 7.0))
+        M.op.mult(dx, dy)
+        y = dy.download()
+        M.op.mult(dx, dy)
+        assert np.array_equal(y, dy.download())  # same bits every time
+        fx, fy = dvec(x.astype(np.float32), 4), N.DeviceVector(fes.ndof, 4)
+        M.op.mult_f32(fx, fy)
+        y0 = rng.uniform(-1, 1, fes.ndof) if not out else out[0][3]
+        da = dvec(y0)
+        M.op.mult_add(-0.5, dx, da)
+        out.append((y, fy.download().astype(np.float64), da.download(), y0))
+    scale = np.abs(out[1][0]).max()
+    t = TOL[precision]
+    assert np.abs(out[0][0] - out[1][0]).max() <= t * scale
+    assert np.abs(out[0][1] - out[1][1]).max() <= max(t, 1e-6) * scale
+    assert np.abs(out[0][2] - out[1][2]).max() <= t * (scale + 1)
+    return fes, kappa, A, x, out[0][0]
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32", "f16x3", "f16", "bf16"])
+@pytest.mark.parametrize("dim,p", [(2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (3, 1), (3, 2), (3, 3), (3, 4)])
+def test_orders_and_precisions(device, monkeypatch, dim, p, precision):
+    say(f"[mfpatch] {dim}D p={p} {precision}")
+    mesh = ngs.MakeStructured2DMesh(nx=9, ny=7) if dim == 2 else ngs.MakeStructured3DMesh(nx=3, ny=4, nz=5)
+    compare(monkeypatch, mesh, p, precision)
+
+
+@pytest.mark.parametrize("cells", [(1, 1, 1), (2, 1, 1), (2, 2, 2), (5, 5, 5), (11, 3, 1)])
+def test_partial_tiles_and_patches(device, monkeypatch, cells):
+    # 6, 12, 48, 750 and 198 elements
+    mesh = ngs.MakeStructured3DMesh(nx=cells[0], ny=cells[1], nz=cells[2])
+    for p in (1, 4):
+        compare(monkeypatch, mesh, p, "f64")
+
+
+def test_eight_tile_patches(device, monkeypatch):
+    # above 4 * 128 elements per CU: patches of 8 tiles
+    mesh = ngs.MakeStructured3DMesh(nx=29, ny=27, nz=29)
+    assert mesh.ne > 4 * 128 * 256
+    for precision in ("f64", "f16x3"):
+        compare(monkeypatch, mesh, 2, precision)
+
+
+@pytest.mark.parametrize("name,p", [("square", 3), ("square", 5), ("cube", 3), ("cube", 4)])
+def test_unstructured(device, monkeypatch, name, p):
+    import os
+    path = os.path.join(os.path.dirname(__file__), "golden", name + ".vol.gz")
+    fes, kappa, A, x, y = compare(monkeypatch, ngs.Mesh(path), p, "f64")
+    # the host assembly as an independent sum
+    u, v = fes.TnT()
+    a = ngs.BilinearForm(ngs.ElementCoefficient(kappa) * ngs.grad(u) * ngs.grad(v) * ngs.dx).Assemble().mat
+    ref = O.csr_matvec(a.rowptr, a.cols, a.vals, x) if hasattr(O, "csr_matvec") else None
+    if ref is None:
+        import scipy.sparse as sp
+        ref = sp.csr_matrix((a.vals, a.cols, a.rowptr)) @ x
+    assert np.abs(y - ref).max() <= 1e-13 * np.abs(ref).max()
+
+
+def test_overlapping_vectors_and_new_coefficient(device, monkeypatch):
+    mesh = ngs.MakeStructured3DMesh(nx=4, ny=4, nz=4)
+    fes, kappa, A, x, y = compare(monkeypatch, mesh, 3, "f64")
+    d = dvec(x)
+    A.op.mult(d, d)
+    assert np.array_equal(d.download(), y)
+    k2 = kappa[::-1].copy()
+    B = build(monkeypatch, fes, k2, "f64", False)
+    A.op.set_kappa(dvec(k2))
+    dx, dy, dz = dvec(x), N.DeviceVector(fes.ndof, 8), N.DeviceVector(fes.ndof, 8)
+    A.op.mult(dx, dy)
+    B.op.mult(dx, dz)
+    assert np.abs(dy.download() - dz.download()).max() <= 1e-14 * np.abs(dz.download()).max()
+
+
+@pytest.mark.parametrize("cells", [(1, 1, 1), (6, 5, 7)])
+def test_cg_inner_product(device, monkeypatch, cells):
+    """CG takes <s, A s> from the patch kernel's partial sums (with one patch:
+    no shared dofs)."""
+    mesh = ngs.MakeStructured3DMesh(nx=cells[0], ny=cells[1], nz=cells[2])
+    fes = ngs.H1(mesh, order=3, dirichlet=".*")
+    rng = np.random.default_rng(5)
+    kappa = np.exp(rng.standard_normal(mesh.ne))
+    f = dvec(rng.uniform(0.5, 1, fes.ndof))
+    sol, its = [], []
+    for patch in (True, False):
+        A = build(monkeypatch, fes, kappa, "f64", patch)
+        C = A.CreateSmoother(fes.FreeDofs)
+        u = N.DeviceVector(fes.ndof, 8)
+        it, _ = N.CGSolve(A.op, C.op, f, u, True, 1e-12, -1.0, 2000, 16)
+        sol.append(u.download())
+        its.append(it)
+    assert abs(its[0] - its[1]) <= 1
+    # both stop at 1e-12 in the preconditioned residual
+    assert np.linalg.norm(sol[0] - sol[1]) <= 1e-10 * max(np.linalg.norm(sol[1]), 1e-300)
