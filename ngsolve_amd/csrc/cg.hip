@@ -21,6 +21,8 @@
 // workgroup 0 of (3) also does the stopping test and keeps the iteration
 // count and the residual history.  The operator kernels write one partial
 // per workgroup of a wide grid; a small kernel folds them to 64 before (2).
+// A small CSR operator (FormsDirection) takes (3) with it: two kernels an
+// iteration.
 // With a block-Jacobi preconditioner, (2) does only the two updates and the
 // preconditioner's two kernels and a dot kernel for <w,d> follow it.  Every
 // workgroup sums the same partials
@@ -43,6 +45,7 @@
 #include <cmath>
 #include <vector>
 
+#include "cgstate.hpp"
 #include "common.hpp"
 #include "csr.hpp"
 #include "matfree.hpp"
@@ -103,33 +106,7 @@ void JacobiOp::Mult(const double* x, double* y, hipStream_t st) {
   NGSAMD_CHECK_LAUNCH();
 }
 
-// ---------------------------------------------------------- CG device state
-
-struct CGScalars {
-  double wdn[2];     // <w,d> of the current iteration, by iteration parity
-  double alpha, beta;
-  double final_res;  // stopping threshold
-  double tol, atol;  // tol < 0: not given; atol < 0: not given
-  int it;            // CheckResidual calls so far
-  int done;          // 0 running, 1 converged / maxiter, 2 breakdown
-  int maxiter;
-  int pad;
-};
-
-constexpr int kCgBlock = 256;
-
-__device__ __forceinline__ void CheckResidual(CGScalars* S, double* residuals, double res) {
-  S->it += 1;
-  if (S->it <= S->maxiter) residuals[S->it - 1] = res;
-  if (S->it == 1) {
-    if (S->tol < 0) S->final_res = S->atol;
-    else {
-      S->final_res = res * S->tol;
-      if (S->atol >= 0 && S->atol > S->final_res) S->final_res = S->atol;
-    }
-  }
-  if (S->it >= S->maxiter || res <= S->final_res) S->done = 1;
-}
+// ---------------------------------------------------------- CG kernels
 
 // w = C d (inv null: w already holds C d); s = w; partials of <w,d>
 template <class V>
@@ -216,6 +193,55 @@ __global__ __launch_bounds__(kCgBlock) void CgDirectionKernel(V* __restrict__ s,
   const V bv = (V)beta;
   for (int64_t i = blockIdx.x * (int64_t)kCgBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kCgBlock)
     s[i] = bv * s[i] + w[i];
+}
+
+// Start of a solve whose operator forms the direction: w = C d, pairs {0, w};
+// partials of <w,d>
+__global__ __launch_bounds__(kCgBlock) void CgInitPairKernel(const double* __restrict__ inv, const double* __restrict__ d,
+                                                             double* __restrict__ pair, int64_t n,
+                                                             double* __restrict__ partials) {
+  __shared__ double lds[kCgBlock / 64];
+  double acc = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)kCgBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kCgBlock) {
+    const double di = d[i];
+    const double wi = inv[i] * di;
+    pair[2 * i] = 0.0;
+    pair[2 * i + 1] = wi;
+    acc += wi * di;
+  }
+  StorePartial<kCgBlock>(acc, partials, lds);
+}
+
+// CgUpdateKernel for a solve whose operator forms the direction: s is the
+// first entry of the pairs, C d goes to the second (wd is wdn[P ^ 1], which
+// the operator kernel wrote).
+__global__ __launch_bounds__(kCgBlock) void CgUpdatePairKernel(const double* __restrict__ inv, double* __restrict__ u,
+                                                               double* __restrict__ d, const double* __restrict__ w,
+                                                               double* __restrict__ pair, int64_t n, CGScalars* S, int P,
+                                                               const double* __restrict__ pa, int na,
+                                                               double* __restrict__ pw) {
+  if (S->done) return;
+  __shared__ double lds[kCgBlock / 64 + 1];
+  const double as_s = SumPartialsAll<kCgBlock>(pa, na, lds);
+  const double wd = S->wdn[P ^ 1];
+  if (as_s == 0.0 || wd == 0.0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 2;
+    return;
+  }
+  const double alpha = wd / as_s;
+  if (blockIdx.x == 0 && threadIdx.x == 0) S->alpha = alpha;
+  const double alv = alpha;
+  double acc = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)kCgBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kCgBlock) {
+    const double si = pair[2 * i], wi = w[i];
+    u[i] += alv * si;
+    const double di = d[i] - alv * wi;
+    d[i] = di;
+    const double zi = inv[i] * di;
+    pair[2 * i + 1] = zi;
+    acc += zi * di;
+  }
+  StorePartial<kCgBlock>(acc, pw, lds);
 }
 
 // partials of <x,y> (FP64 accumulation), skipped when *done
@@ -337,18 +363,48 @@ static void EnqueueIteration(ngsamd_op_t A, const V* inv, ngsamd_op_t pre, V* u,
   NGSAMD_CHECK_LAUNCH();
 }
 
+// Whether the operator forms the direction itself (one kernel less an
+// iteration): CSR in the runs layout where no fold kernel follows the product
+// (64^2 p=3: 14.2 -> 12.6 us an iteration, the direction kernel's 4.4 us less
+// the second gathered vector; up to 1024 workgroups).  Not the patch kernels:
+// every patch of a dof then stores it (32^3 p=4 refinement 24.5 -> 27.8 ms).
+template <class V>
+static bool FormsDirection(ngsamd_op_t A, const V* inv, int64_t n) {
+  if constexpr (sizeof(V) == 8)
+    return inv && n > 0 && A->kind == OpKind::CSR && static_cast<CsrOp*>(A)->FormsDirection();
+  return false;
+}
+
+// One such iteration of parity P: w = A s with the new s, then the update.
+static void EnqueuePairIteration(ngsamd_op_t A, const double* inv, double* u, double* d, double* w, double* pair0,
+                                 double* pair1, int64_t n,
+                                 CGScalars* dS, double* residuals, int P, hipStream_t st,
+                                 const CgPartials& B = LibraryPartials()) {
+  const int g = CgGrid(n);
+  double* next = P ? pair0 : pair1;
+  const CgDirection D{P ? pair1 : pair0, next, dS, B.w, g, P, residuals};
+  const int na = static_cast<CsrOp*>(A)->MultDotDirection(D, w, B.a, &dS->done, st);
+  CgUpdatePairKernel<<<g, kCgBlock, 0, st>>>(inv, u, d, w, next, n, dS, P, B.a, na, B.w);
+  NGSAMD_CHECK_LAUNCH();
+}
+
 struct CgResult {
   int iterations = 0;
   int done = 0;
 };
 
 // Work vectors and device scalars of one CG instance.
+// pairs: the operator forms the direction (FormsDirection), {s, z} pairs in
+// two buffers instead of s.
 template <class V>
 struct CgWork {
-  DevBuf<V> d, w, s;
+  bool pairs;
+  DevBuf<V> d, w, s, pair0, pair1;
   DevBuf<double> residuals;
   DevBuf<CGScalars> S;
-  CgWork(int64_t n, int maxiter) : d(n), w(n), s(n), residuals(maxiter), S(1) {}
+  CgWork(int64_t n, int maxiter, bool pairs_)
+      : pairs(pairs_), d(n), w(n), s(pairs_ ? 0 : n), pair0(pairs_ ? 2 * n : 0), pair1(pairs_ ? 2 * n : 0),
+        residuals(maxiter), S(1) {}
 };
 
 // A captured graph of `chunk` CG iterations.  The kernels read the
@@ -392,11 +448,25 @@ static CgResult IterateCg(ngsamd_op_t A, const V* inv, ngsamd_op_t pre, V* u, Cg
   hS.maxiter = maxiter;
   NGSAMD_HIP(hipMemcpyAsync(W.S.p, &hS, sizeof(CGScalars), hipMemcpyHostToDevice, st));
   const int g = CgGrid(n);
-  if (!inv) EnqueuePrecond<V>(pre, W.d.p, W.w.p, nullptr, st);
-  CgInitKernel<V><<<g, kCgBlock, 0, st>>>(inv, W.d.p, W.w.p, W.s.p, n, LibraryPartials().w);
-  NGSAMD_CHECK_LAUNCH();
-  CgInitCheckKernel<<<1, kCgBlock, 0, st>>>(LibraryPartials().w, g, W.S.p, W.residuals.p);
-  NGSAMD_CHECK_LAUNCH();
+  auto iteration = [&](int P) {
+    if constexpr (sizeof(V) == 8)
+      if (W.pairs)
+        return EnqueuePairIteration(A, inv, u, W.d.p, W.w.p, W.pair0.p, W.pair1.p, n, W.S.p, W.residuals.p, P, st);
+    EnqueueIteration<V>(A, inv, pre, u, W.d.p, W.w.p, W.s.p, n, W.S.p, W.residuals.p, P, st);
+  };
+  if (W.pairs) {
+    // the first operator kernel does the first check
+    if constexpr (sizeof(V) == 8) {
+      CgInitPairKernel<<<g, kCgBlock, 0, st>>>(inv, W.d.p, W.pair0.p, n, LibraryPartials().w);
+      NGSAMD_CHECK_LAUNCH();
+    }
+  } else {
+    if (!inv) EnqueuePrecond<V>(pre, W.d.p, W.w.p, nullptr, st);
+    CgInitKernel<V><<<g, kCgBlock, 0, st>>>(inv, W.d.p, W.w.p, W.s.p, n, LibraryPartials().w);
+    NGSAMD_CHECK_LAUNCH();
+    CgInitCheckKernel<<<1, kCgBlock, 0, st>>>(LibraryPartials().w, g, W.S.p, W.residuals.p);
+    NGSAMD_CHECK_LAUNCH();
+  }
 
   // graphs hold an even number of iterations so that every replay starts
   // at parity 0
@@ -411,8 +481,7 @@ static CgResult IterateCg(ngsamd_op_t A, const V* inv, ngsamd_op_t pre, V* u, Cg
     if (e == hipSuccess) {
       bool ok = true;
       try {
-        for (int k = 0; k < chunk; k++)
-          EnqueueIteration<V>(A, inv, pre, u, W.d.p, W.w.p, W.s.p, n, W.S.p, W.residuals.p, k & 1, st);
+        for (int k = 0; k < chunk; k++) iteration(k & 1);
       } catch (...) {
         ok = false;
       }
@@ -435,14 +504,15 @@ static CgResult IterateCg(ngsamd_op_t A, const V* inv, ngsamd_op_t pre, V* u, Cg
   long long enqueued = 0;  // iterations enqueued without a graph (parity)
   auto enqueue = [&](int slot) {
     if (use_graph) NGSAMD_HIP(hipGraphLaunch(exec, st));
-    else
-      EnqueueIteration<V>(A, inv, pre, u, W.d.p, W.w.p, W.s.p, n, W.S.p, W.residuals.p, (int)(enqueued++ & 1), st);
+    else iteration((int)(enqueued++ & 1));
     NGSAMD_HIP(hipMemcpyAsync(&pin[slot], W.S.p, sizeof(CGScalars), hipMemcpyDeviceToHost, st));
   };
 
-  NGSAMD_HIP(hipMemcpyAsync(&pin[0], W.S.p, sizeof(CGScalars), hipMemcpyDeviceToHost, st));
-  NGSAMD_HIP(hipStreamSynchronize(st));
-  if (!pin[0].done) {
+  if (!W.pairs) {
+    NGSAMD_HIP(hipMemcpyAsync(&pin[0], W.S.p, sizeof(CGScalars), hipMemcpyDeviceToHost, st));
+    NGSAMD_HIP(hipStreamSynchronize(st));
+  }
+  if (W.pairs || !pin[0].done) {
     // keep two launches in flight; poll the older one
     enqueue(0);
     NGSAMD_HIP(hipEventRecord(ev[0], st));
@@ -569,12 +639,12 @@ extern "C" int ngsamd_cg_solve(ngsamd_op_t A, ngsamd_op_t pre, const double* f, 
     NGSAMD_REQUIRE(maxiter >= 1, "cg: maxiter must be >= 1");
     const int64_t n = A->height;
     hipStream_t st = Stream();
-    CgWork<double> W(n, maxiter);
+    const double* inv = pre->kind == OpKind::Jacobi ? static_cast<JacobiOp*>(pre)->invdiag.p : nullptr;
+    CgWork<double> W(n, maxiter, FormsDirection<double>(A, inv, n));
     // d = f - A u
     if (initialize) LaunchFill(u, n, 0.0, st);
     if (n) NGSAMD_HIP(hipMemcpyAsync(W.d.p, f, n * sizeof(double), hipMemcpyDeviceToDevice, st));
     if (!initialize) A->MultAdd(-1.0, u, W.d.p, st);
-    const double* inv = pre->kind == OpKind::Jacobi ? static_cast<JacobiOp*>(pre)->invdiag.p : nullptr;
     CgResult r = IterateCg<double>(A, inv, pre, u, W, n, tol, atol, maxiter, chunk, st);
     if (h_iterations) *h_iterations = r.iterations;
     if (h_residuals && r.iterations > 0) {
@@ -637,7 +707,7 @@ extern "C" int ngsamd_ir_cg_solve(ngsamd_op_t A, ngsamd_op_t inner, ngsamd_op_t 
     // FP32 copy of the Jacobi inverse diagonal
     const double* inv64 = static_cast<JacobiOp*>(pre)->invdiag.p;
     ngsamd_vec_f64_to_f32(n, inv64, inv32.p);
-    CgWork<float> W(n, max_inner);
+    CgWork<float> W(n, max_inner, false);
 
     // residual norms over the free dofs (where the Jacobi inverse is nonzero)
     DevBuf<double> sq(1);

@@ -3,6 +3,7 @@
 #pragma once
 #include <vector>
 
+#include "cgstate.hpp"
 #include "common.hpp"
 
 namespace ngsamd {
@@ -51,6 +52,10 @@ struct CsrOp : ngsamd_op_s {
   // library's)
   int MultDot(const double* x, double* y, double* partials, const int* d_stop, hipStream_t st,
               double* wide = nullptr);
+  // MultDot with the direction step (CgDirection): w = A s for the new s,
+  // whose entries the kernel forms and stores
+  bool FormsDirection() const;
+  int MultDotDirection(const CgDirection& D, double* w, double* partials, const int* d_stop, hipStream_t st);
   // Y = A X for K vectors stored interleaved ([n][K]); the matrix is read
   // once for all K in the runs layout
   // (all kernels return at once when *stop != 0, stop may be null)

@@ -242,11 +242,26 @@ __device__ __forceinline__ void LoadPair(const double* p, double& a, double& b) 
   b = t.y;
 }
 
+// The single vector x of the runs kernel: plain, or formed from {s, z} pairs
+// (CgDirection) as beta s + z.
+struct PlainX {
+  const double* __restrict__ x;
+  __device__ __forceinline__ double operator()(int i) const { return x[i]; }
+};
+struct PairX {
+  const double2* __restrict__ pair;
+  double beta;
+  __device__ __forceinline__ double operator()(int i) const {
+    const double2 t = pair[i];
+    return __builtin_fma(beta, t.x, t.y);
+  }
+};
+
 // acc[q][j] = this lane's share of row q of its run (first column c0, first
 // value v0, L slots) times component j0 + j of the K-vector x
-template <int R, int KC, int U>
+template <int R, int KC, int U, class X>
 __device__ __forceinline__ void RunPartials(const int* __restrict__ rcols, const double* __restrict__ rvals,
-                                            const double* __restrict__ x, int K, int j0, int c0, int v0, int L, int l,
+                                            const X& x, int K, int j0, int c0, int v0, int L, int l,
                                             int G, double (&acc)[R][KC]) {
 #pragma unroll
   for (int q = 0; q < R; q++)
@@ -267,11 +282,13 @@ __device__ __forceinline__ void RunPartials(const int* __restrict__ rcols, const
     }
 #pragma unroll
     for (int i = 0; i < U; i++) {
-      const double* xp = x + ((int64_t)c[i] * K + j0);
-      if constexpr (KC == 1) xv[i][0] = xp[0];
-      else {
+      if constexpr (std::is_same<X, PlainX>::value || std::is_same<X, PairX>::value) {
+        xv[i][0] = x(c[i]);
+      } else {
+        const double* xp = x + ((int64_t)c[i] * K + j0);
+        if constexpr (KC == 1) xv[i][0] = xp[0];
 #pragma unroll
-        for (int j = 0; j < KC; j += 2) LoadPair(xp + j, xv[i][j], xv[i][j + 1]);
+        for (int j = 0; j + 1 < KC; j += 2) LoadPair(xp + j, xv[i][j], xv[i][j + 1]);
       }
     }
 #pragma unroll
@@ -335,10 +352,11 @@ __device__ __forceinline__ void WalkRunTasks(const int4* __restrict__ tasks, int
 
 // The task's rows: y[r] = (ACCUM ? y[r] : 0) + s * (A x)[r]; with DOT the
 // lane's sum of x[r] * (A x)[r] is added to dotacc.
-template <int R, int U, bool ACCUM, bool DOT>
+template <int R, int U, bool ACCUM, bool DOT, class X>
 __device__ __forceinline__ void RunTaskRows(const RunHead& h, const int* __restrict__ rcols,
-                                            const double* __restrict__ rvals, const double* __restrict__ x,
-                                            double* __restrict__ y, double s, double& dotacc) {
+                                            const double* __restrict__ rvals, const X& x,
+                                            double* __restrict__ y, double s, double& dotacc,
+                                            double* __restrict__ next) {
   const int4 t = h.t;
   const int n = t.w & 0xff, lg = (t.w >> 16) & 0xff;
   const int lane = threadIdx.x & 63, G = 1 << lg;
@@ -356,7 +374,11 @@ __device__ __forceinline__ void RunTaskRows(const RunHead& h, const int* __restr
   if (g < n && l < R) {
     const int r = t.z + g * R + l;
     if (ACCUM) y[r] += s * mine; else y[r] = s * mine;
-    if (DOT) dotacc += x[r] * mine;
+    if (DOT) {
+      const double xr = x(r);
+      dotacc += xr * mine;
+      if (std::is_same<X, PairX>::value) next[2 * (int64_t)r] = xr;
+    }
   }
 }
 
@@ -377,21 +399,33 @@ __device__ __forceinline__ void RunTaskRows(const RunHead& h, const int* __restr
 // per value), us per apply: 32^3 p=4 (159M nonzeros) 389 -> 298 (4.3 TB/s of
 // values alone, 5.2 TB/s with the shared columns), 20x16x24 p=4 97 -> 64,
 // 61x67 p=3 6.0 -> 4.3.
-template <bool ACCUM, bool DOT>
-__global__ __launch_bounds__(kStreamBlock, 6) void CsrRunsKernel(
+// DIR (with DOT): x is the new search direction, formed from the pairs of D
+// and stored by the rows' owners (CgDirection).
+template <bool ACCUM, bool DOT, bool DIR>
+__global__ __launch_bounds__(kStreamBlock, DIR ? 4 : 6) void CsrRunsKernel(
     const int4* __restrict__ tasks, int ntasks, const int* __restrict__ run_ptr,
-    const int* __restrict__ rcols, const double* __restrict__ rvals, const double* __restrict__ x,
-    double* __restrict__ y, double s, double* __restrict__ partials, const int* __restrict__ stop_flag, int reverse) {
+    const int* __restrict__ rcols, const double* __restrict__ rvals, const double* __restrict__ xv,
+    double* __restrict__ y, double s, double* __restrict__ partials, const int* __restrict__ stop_flag, int reverse,
+    CgDirection D) {
   if (stop_flag && *stop_flag) return;
+  static_assert(kStreamBlock == kCgBlock, "DirectionBeta");
+  __shared__ double lds[kStreamBlock / 64 + 1];
+  typename std::conditional<DIR, PairX, PlainX>::type x;
+  if constexpr (DIR) {
+    x.beta = DirectionBeta(D, lds);
+    x.pair = reinterpret_cast<const double2*>(D.pair);
+  } else {
+    x.x = xv;
+  }
   const int lx = XcdContiguousBlock(blockIdx.x, gridDim.x);
   double dotacc = 0.0;
   WalkRunTasks(tasks, ntasks, run_ptr, reverse ? (int)gridDim.x - 1 - lx : lx, gridDim.x, reverse, [&](const RunHead& h) __attribute__((always_inline)) {
     ForRunShape<1>((h.t.w >> 8) & 0xff, h.t.w >> 24, [&](auto r, auto u) __attribute__((always_inline)) {
-      RunTaskRows<decltype(r)::value, decltype(u)::value, ACCUM, DOT>(h, rcols, rvals, x, y, s, dotacc);
+      RunTaskRows<decltype(r)::value, decltype(u)::value, ACCUM, DOT>(h, rcols, rvals, x, y, s, dotacc, D.next);
     });
   });
   if (DOT) {
-    __shared__ double lds[kStreamBlock / 64];
+    __syncthreads();
     StorePartial<kStreamBlock>(dotacc, partials, lds);
   }
 }
@@ -772,8 +806,8 @@ template <bool ACCUM, bool DOT>
 static int LaunchRuns(const CsrOp& A, double s, const double* x, double* y, hipStream_t st, double* partials,
                       const int* stop, int reverse) {
   const int wg = RunsGrid(A, DOT ? RunsDotCap(A) : A.max_grid);
-  CsrRunsKernel<ACCUM, DOT><<<wg, kStreamBlock, 0, st>>>(A.tasks.p, A.ntasks, A.run_ptr.p, A.rcols.p, A.rvals.p, x,
-                                                         y, s, partials, stop, reverse);
+  CsrRunsKernel<ACCUM, DOT, false><<<wg, kStreamBlock, 0, st>>>(A.tasks.p, A.ntasks, A.run_ptr.p, A.rcols.p,
+                                                                A.rvals.p, x, y, s, partials, stop, reverse, {});
   NGSAMD_CHECK_LAUNCH();
   return wg;
 }
@@ -827,6 +861,17 @@ int CsrOp::MultDot(const double* x, double* y, double* partials, const int* d_st
   const int np = LaunchSpmv<false, true>(*this, 1.0, x, y, st, wide, d_stop);
   LaunchFoldPartials(wide, np, partials, d_stop, st);
   return kFoldedPartials;
+}
+
+bool CsrOp::FormsDirection() const { return algo == 2 && width > 0 && DotWorkgroups(*this) <= 1024; }
+
+int CsrOp::MultDotDirection(const CgDirection& D, double* w, double* partials, const int* stop,
+                            hipStream_t st) {
+  const int wg = RunsGrid(*this, RunsDotCap(*this));
+  CsrRunsKernel<false, true, true><<<wg, kStreamBlock, 0, st>>>(tasks.p, ntasks, run_ptr.p, rcols.p, rvals.p, nullptr,
+                                                                w, 1.0, partials, stop, 0, D);
+  NGSAMD_CHECK_LAUNCH();
+  return wg;
 }
 
 __global__ void CsrDiagKernel(const int* __restrict__ rowptr, const int* __restrict__ cols,

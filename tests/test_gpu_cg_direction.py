@@ -1,0 +1,54 @@
+"""CG on a small CSR operator, whose kernel forms the search direction (two
+kernels an iteration): iteration counts, residual history and solutions against
+the oracle's PCG where the first check, the iteration limit or the breakdown
+test ends the loop, with and without an initial guess, with graphs of 2 and 16
+iterations and without."""
+import numpy as np
+import pytest
+
+import oracle
+from oracle import fe_oracle as O
+from helpers import N, dvec, problem, say
+
+pytestmark = pytest.mark.gpu
+
+
+def pcg(P, inv, f, u0, tol, maxiter):
+    A = lambda t: oracle.spmv(P["rowptr"], P["cols"], P["vals"], t)  # noqa: E731
+    g = f - A(u0)
+    u, its, res = O.pcg(A, inv, g, tol=tol, maxiter=maxiter)
+    return u0 + u, its, res
+
+
+@pytest.mark.parametrize("dim,n,p", [(2, 2, 2), (2, 9, 3), (2, 20, 5), (3, 4, 3)])
+@pytest.mark.parametrize("maxiter", [1, 2, 3, 17, 2000])
+@pytest.mark.parametrize("chunk", [0, 2, 16])
+def test_against_oracle(device, dim, n, p, maxiter, chunk):
+    say(f"[cg direction] {dim}D {n} p={p} maxiter={maxiter} chunk={chunk}")
+    P = problem(dim, n, p, seed_kappa=4)
+    A = N.CreateCSR(P["ndof"], P["ndof"], P["rowptr"], P["cols"], P["vals"])
+    free = P["fes"].freedofs.astype(np.uint8)
+    diag, inv = O.jacobi_invdiag(P["rowptr"], P["cols"], P["vals"], free)
+    C = N.CreateJacobi(diag, free)
+    rng = np.random.default_rng(8)
+    f = np.where(free != 0, rng.uniform(-1, 1, P["ndof"]), 0.0)
+    for u0 in (None, rng.uniform(-1, 1, P["ndof"])):
+        start = np.zeros(P["ndof"]) if u0 is None else u0
+        ref, its_ref, res_ref = pcg(P, inv, f, start, 1e-10, maxiter)
+        du = dvec(start)
+        its, res = N.CGSolve(A, C, dvec(f), du, u0 is None, 1e-10, -1.0, maxiter, chunk)
+        assert abs(its - its_ref) <= (1 if its_ref < maxiter else 0)
+        assert np.allclose(res[:3], res_ref[:3], rtol=1e-9, atol=0)
+        if its == its_ref:
+            assert np.abs(du.download() - ref).max() <= 1e-9 * max(np.abs(ref).max(), 1e-300)
+
+
+def test_zero_right_hand_side(device):
+    P = problem(2, 6, 2, seed_kappa=1)
+    A = N.CreateCSR(P["ndof"], P["ndof"], P["rowptr"], P["cols"], P["vals"])
+    free = P["fes"].freedofs.astype(np.uint8)
+    diag, _ = O.jacobi_invdiag(P["rowptr"], P["cols"], P["vals"], free)
+    C = N.CreateJacobi(diag, free)
+    du = dvec(np.full(P["ndof"], 3.0))
+    its, res = N.CGSolve(A, C, dvec(np.zeros(P["ndof"])), du, True, 1e-10, -1.0, 100, 16)
+    assert its == 1 and res[0] == 0.0 and not du.download().any()
