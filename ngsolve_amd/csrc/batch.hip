@@ -14,11 +14,13 @@
 // the stream SpMV never straddle two problems, so each block's <s, A s>
 // partial belongs to one problem; vectors are cut into chunks of at most
 // kChunk dofs inside one problem for the update kernels.  Per-problem sums
-// are formed by one workgroup per problem over its contiguous range of
-// partials (deterministic).
+// are formed over the problem's contiguous range of partials, in one order
+// (deterministic): by every chunk's workgroup that needs the sum, so that an
+// iteration is three kernels (product, update, direction).
 //
-// Tiles: the nonzeros per row block (1024/2048/4096) are picked when the
-// operator is created by timing each candidate on the device.
+// Tiles: the nonzeros per row block, or per wavefront of the runs kernel
+// (1024/2048/4096), are picked when the operator is created by timing each
+// candidate on the device.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -29,6 +31,7 @@
 #include "csr.hpp"
 #include "reduce.hpp"
 #include "runs.hpp"
+#include "runsdev.hpp"
 #include "runtime_state.hpp"
 
 namespace ngsamd {
@@ -76,7 +79,8 @@ struct BatchOp : ngsamd_op_s {
   // column numbers; blocks never straddle two problems
   bool use_runs = false;
   bool has_f32 = false;
-  DevBuf<int> run_row, run_ptr, val_ptr, rcols, blk_run, blk_len;
+  DevBuf<int> run_ptr, rcols;
+  DevBuf<int4> blk_info;  // two records per block (BatchRunsBlock)
   DevBuf<double> rvals;
   DevBuf<float> rvals32;
   int nseg = 0;
@@ -87,7 +91,8 @@ struct BatchOp : ngsamd_op_s {
   int nchunks = 0;
   DevBuf<int64_t> chunk_start;
   DevBuf<int> chunk_seg, seg_chunk;
-  DevBuf<double> partials;
+  DevBuf<double> partials;   // per row block (the other sums: per chunk or problem)
+  DevBuf<double> cpartials;  // per chunk, of the update kernel
   // autotune: ms per apply of each candidate block size (1024, 2048, 4096),
   // empty when a single size was forced
   std::vector<float> tuned_ms;
@@ -196,112 +201,89 @@ __global__ __launch_bounds__(kBatchBlock) void BatchSpmvKernel(
                                           lds);
 }
 
-// Runs-layout form of BatchSpmvKernel (the runs kernel of spmv.hip with the
-// frozen-problem skip and one partial per block).
-// Block b of the runs layout (prod / lds as in BatchSpmvBlock).
-template <int NNZ, class V, class M, bool ACCUM, bool DOT>
-__device__ __forceinline__ void BatchRunsBlock(const int* __restrict__ run_row, const int* __restrict__ run_ptr,
-                                               const int* __restrict__ val_ptr, const int* __restrict__ rcols,
-                                               const M* __restrict__ rvals, const V* __restrict__ x,
-                                               V* __restrict__ y, double s, const int* __restrict__ blk_run,
-                                               const int* __restrict__ blk_len, const int* __restrict__ blk_seg,
-                                               const int* __restrict__ done, double* __restrict__ partials, int b,
-                                               double* prod, double* lds) {
-  static_assert(NNZ <= 4096, "RunDiv is exact below 4096");
-  constexpr int PER = NNZ / kBatchBlock;
-  const int tid = threadIdx.x;
-  {
-    if (done && done[blk_seg[b]]) {
-      if (DOT && tid == 0) partials[b] = 0.0;
-      return;
-    }
-    const int u0 = blk_run[b], u1 = blk_run[b + 1];
-    const int R = blk_len[b];
-    const int inv = (65536 + R - 1) / R;
-    const int c0 = run_ptr[u0];
-    const int vb = val_ptr[u0];
-    const int nv = val_ptr[u1] - vb;
-    double dotacc = 0.0;
-    if (nv > NNZ) {
-      // one long row (R = 1): the whole workgroup strides over it
-      double a = 0.0;
-      for (int k = tid; k < nv; k += kBatchBlock)
-        a += (double)__builtin_nontemporal_load(&rvals[vb + k]) * (double)x[__builtin_nontemporal_load(&rcols[c0 + k])];
-      a = BlockSum<kBatchBlock>(a, lds);
-      if (tid == 0) {
-        const int r = run_row[u0];
-        if (ACCUM) y[r] = (V)((double)y[r] + s * a); else y[r] = (V)(s * a);
-        if (DOT) partials[b] = (double)x[r] * a;
-      }
-      return;
-    }
-    int c[PER];
-    double v[PER], xv[PER];
+// x(i) in FP64 for RunPartials
+template <class V>
+struct BatchX {
+  const V* __restrict__ x;
+  __device__ __forceinline__ double operator()(int i) const { return (double)x[i]; }
+};
+
+// The runs of one block (one problem and one R): 64 >> lg at a time, the next
+// ones' extent loaded meanwhile.
+template <int R, int U, class V, class M, bool ACCUM, bool DOT>
+__device__ __forceinline__ void BatchRunRows(const int* __restrict__ run_ptr, const int* __restrict__ rcols,
+                                             const M* __restrict__ rvals, const V* __restrict__ x,
+                                             V* __restrict__ y, double s, int u0, int nr, int c00, int vb, int row0,
+                                             int lg, double& dotacc) {
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> lg, l = lane & ((1 << lg) - 1);
+  const int step = 64 >> lg;
+  int u = min(g, nr - 1);
+  int c0 = run_ptr[u0 + u], c1 = run_ptr[u0 + u + 1];
+  for (int t = 0; t < nr; t += step) {
+    const int un = min(t + step + g, nr - 1);
+    const int n0 = run_ptr[u0 + un], n1 = run_ptr[u0 + un + 1];
+    double acc[R][1];
+    RunPartials<R, 1, U>(rcols, rvals, BatchX<V>{x}, 1, 0, c0, vb + (c0 - c00) * R, c1 - c0, l, 1 << lg, acc);
+    double mine = 0.0;
 #pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int k = tid + i * kBatchBlock;
-      const int kk = k < nv ? k : 0;
-      c[i] = __builtin_nontemporal_load(&rcols[c0 + RunDiv(kk, inv)]);
-      v[i] = (double)__builtin_nontemporal_load(&rvals[vb + kk]);
+    for (int q = 0; q < R; q++) {
+      const double sum = GroupSum(acc[q][0], lg);
+      mine = l == q ? sum : mine;
     }
-#pragma unroll
-    for (int i = 0; i < PER; i++) xv[i] = (double)x[c[i]];
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int k = tid + i * kBatchBlock;
-      prod[k] = k < nv ? v[i] * xv[i] : 0.0;
+    if (t + g < nr && l < R) {
+      const int r = row0 + u * R + l;
+      if (ACCUM) y[r] = (V)((double)y[r] + s * mine); else y[r] = (V)(s * mine);
+      if (DOT) dotacc += (double)x[r] * mine;
     }
-    __syncthreads();
-    const int row0 = run_row[u0];
-    const int nr = (u1 - u0) * R;
-    int tpr = 64;
-    while (tpr > 1 && tpr * nr > kBatchBlock) tpr >>= 1;
-    const int l = tid & (tpr - 1);
-    for (int j0 = 0; j0 < nr; j0 += kBatchBlock / tpr) {
-      const int j = j0 + tid / tpr;
-      double sum = 0.0;
-      if (j < nr) {
-        const int run = RunDiv(j, inv), q = j - run * R;
-        const int s0 = run_ptr[u0 + run] - c0, s1 = run_ptr[u0 + run + 1] - c0;
-        double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-        int k = s0 + l;
-        for (; k + 3 * tpr < s1; k += 4 * tpr) {
-          a0 += prod[k * R + q];
-          a1 += prod[(k + tpr) * R + q];
-          a2 += prod[(k + 2 * tpr) * R + q];
-          a3 += prod[(k + 3 * tpr) * R + q];
-        }
-        for (; k < s1; k += tpr) a0 += prod[k * R + q];
-        sum = (a0 + a1) + (a2 + a3);
-      }
-      for (int off = tpr / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-      if (j < nr && l == 0) {
-        if (ACCUM) y[row0 + j] = (V)((double)y[row0 + j] + s * sum); else y[row0 + j] = (V)(s * sum);
-        if (DOT) dotacc += (double)x[row0 + j] * sum;
-      }
-    }
-    if (DOT) {
-      dotacc = BlockSum<kBatchBlock>(dotacc, lds);
-      if (tid == 0) partials[b] = dotacc;
-    }
-    __syncthreads();
+    u = un;
+    c0 = n0;
+    c1 = n1;
   }
 }
 
-template <int NNZ, class V, class M, bool ACCUM, bool DOT>
-__global__ __launch_bounds__(kBatchBlock) void BatchRunsKernel(
-    const int* __restrict__ run_row, const int* __restrict__ run_ptr, const int* __restrict__ val_ptr,
-    const int* __restrict__ rcols, const M* __restrict__ rvals, const V* __restrict__ x, V* __restrict__ y, double s,
-    const int* __restrict__ blk_run, const int* __restrict__ blk_len, const int* __restrict__ blk_seg, int nblocks,
-    int blocks_per_wg, const int* __restrict__ done, double* __restrict__ partials) {
-  __shared__ double prod[NNZ];
-  __shared__ double lds[kBatchBlock / 64];
+// Runs-layout form of BatchSpmvKernel (the runs kernel of spmv.hip with the
+// frozen-problem skip and one partial per block): one block of up to 1024
+// values per wavefront, row sums in registers, neither LDS nor barriers.
+// What bounds it is the chain block record, run extent, columns, x: 48 2D
+// problems (32584 blocks, FP64, about 290 MB) take 0.106 ms, 0.128 with a
+// block per workgroup.
+// info[b]: {first run, runs, first column, first value},
+//          {first row, rows per run | log2(lanes per run) << 8, slots, problem}
+template <class V, class M, bool ACCUM, bool DOT>
+__device__ __forceinline__ void BatchRunsBlock(const int4* __restrict__ info, const int* __restrict__ run_ptr,
+                                               const int* __restrict__ rcols, const M* __restrict__ rvals,
+                                               const V* __restrict__ x, V* __restrict__ y, double s,
+                                               const int* __restrict__ done, double* __restrict__ partials, int b) {
+  const int4 a = info[2 * b], e = info[2 * b + 1];
+  const int nr = __builtin_amdgcn_readfirstlane(a.y), slots = __builtin_amdgcn_readfirstlane(e.z);
+  const int R = __builtin_amdgcn_readfirstlane(e.y & 255), lg = __builtin_amdgcn_readfirstlane(e.y >> 8);
+  if (done && done[e.w]) {
+    if (DOT && (threadIdx.x & 63) == 0) partials[b] = 0.0;
+    return;
+  }
+  const int m = max(1, (slots + (nr << lg) - 1) / (nr << lg));
+  double dotacc = 0.0;
+  ForRunShape<1>(R, m, [&](auto r, auto u) __attribute__((always_inline)) {
+    BatchRunRows<decltype(r)::value, decltype(u)::value, V, M, ACCUM, DOT>(run_ptr, rcols, rvals, x, y, s, a.x, nr,
+                                                                          a.z, a.w, e.x, lg, dotacc);
+  });
+  if (DOT) {
+    dotacc = GroupSum(dotacc, 6);
+    if ((threadIdx.x & 63) == 0) partials[b] = dotacc;
+  }
+}
+
+template <class V, class M, bool ACCUM, bool DOT>
+__global__ __launch_bounds__(kBatchBlock, 6) void BatchRunsKernel(
+    const int4* __restrict__ info, const int* __restrict__ run_ptr, const int* __restrict__ rcols,
+    const M* __restrict__ rvals, const V* __restrict__ x, V* __restrict__ y, double s, int nblocks,
+    int blocks_per_wave, const int* __restrict__ done, double* __restrict__ partials) {
   const int lb = XcdBlock(blockIdx.x, gridDim.x);
-  const int b0 = lb * blocks_per_wg;
-  const int b1 = min(b0 + blocks_per_wg, nblocks);
+  const int b0 = (lb * (kBatchBlock / 64) + (threadIdx.x >> 6)) * blocks_per_wave;
+  const int b1 = min(b0 + blocks_per_wave, nblocks);
   for (int b = b0; b < b1; b++)
-    BatchRunsBlock<NNZ, V, M, ACCUM, DOT>(run_row, run_ptr, val_ptr, rcols, rvals, x, y, s, blk_run, blk_len,
-                                          blk_seg, done, partials, b, prod, lds);
+    BatchRunsBlock<V, M, ACCUM, DOT>(info, run_ptr, rcols, rvals, x, y, s, done, partials, b);
 }
 
 template <class V, class M, bool ACCUM, bool DOT>
@@ -314,15 +296,15 @@ static void LaunchBatchSpmv(const BatchOp& A, const M* vals, const V* x, V* y, d
     if constexpr (sizeof(M) == 8) rv = A.rvals.p;
     else rv = A.rvals32.p;
     (void)vals;
-    int64_t wg = A.nblocks < 16384 ? A.nblocks : 16384;
-    if (wg > 8) wg &= ~int64_t(7);
+    // block_nnz / 1024 blocks per wavefront, workgroups in whole rounds of
+    // the XCDs
+    constexpr int waves = kBatchBlock / 64;
+    const int per = block_nnz / 1024;
+    int64_t wg = (A.nblocks + waves * per - 1) / (waves * per);
+    if (wg > 8) wg = (wg + 7) & ~int64_t(7);
     if (wg < 1) wg = 1;
-    const int per = (int)((A.nblocks + wg - 1) / wg);
-    auto rk = block_nnz == 1024   ? BatchRunsKernel<1024, V, M, ACCUM, DOT>
-              : block_nnz == 4096 ? BatchRunsKernel<4096, V, M, ACCUM, DOT>
-                                  : BatchRunsKernel<2048, V, M, ACCUM, DOT>;
-    rk<<<(int)wg, kBatchBlock, 0, st>>>(A.run_row.p, A.run_ptr.p, A.val_ptr.p, A.rcols.p, rv, x, y, s, A.blk_run.p,
-                                       A.blk_len.p, A.blk_seg.p, A.nblocks, per, done, A.partials.p);
+    BatchRunsKernel<V, M, ACCUM, DOT><<<(int)wg, kBatchBlock, 0, st>>>(A.blk_info.p, A.run_ptr.p, A.rcols.p, rv, x, y,
+                                                                        s, A.nblocks, per, done, A.partials.p);
     NGSAMD_CHECK_LAUNCH();
     return;
   }
@@ -384,14 +366,8 @@ BatchOp::BatchOp(int64_t n, const int64_t* rp, const int* c, const double* v, in
     const int64_t nsh = BuildRuns(n, rp, c, v, 1024, rr, rpp, vp, rc, rv, br, bl, seg, ns, &bs);
     if (4 * nsh <= 3 * nnz) {
       use_runs = true;
-      block_nnz = 1024;
-      nblocks = (int)br.size() - 1;
-      run_row.alloc(rr.size());
-      run_row.upload(rr.data(), rr.size());
       run_ptr.alloc(rpp.size());
       run_ptr.upload(rpp.data(), rpp.size());
-      val_ptr.alloc(vp.size());
-      val_ptr.upload(vp.data(), vp.size());
       rcols.alloc(nsh + 4);
       rcols.upload(rc.data(), nsh);
       rcols.upload_at(zc, nsh, 4);
@@ -415,29 +391,39 @@ BatchOp::BatchOp(int64_t n, const int64_t* rp, const int* c, const double* v, in
           rseg[u] = q;
         }
       }
-      auto set_blocks = [&](int bn) {
-        GroupRunBlocks(rr, vp, rseg, bn, br, bl, &bs);
-        nblocks = (int)br.size() - 1;
-        blk_run.alloc(br.size());
-        blk_run.upload(br.data(), br.size());
-        blk_len.alloc(std::max<size_t>(bl.size(), 1));
-        blk_len.upload(bl.data(), bl.size());
-        blk_seg.alloc(std::max<size_t>(bs.size(), 1));
-        blk_seg.upload(bs.data(), bs.size());
-        // first block of each problem (blocks are in problem order)
-        std::vector<int> sb(ns + 1);
-        int b = 0;
-        for (int q = 0; q <= ns; q++) {
-          while (b < nblocks && bs[b] < q) b++;
-          sb[q] = b;
-        }
-        seg_blk.alloc(sb.size());
-        seg_blk.upload(sb.data(), sb.size());
-        partials.alloc(std::max<size_t>({(size_t)nblocks, (size_t)ns, (size_t)1}));
-        NGSAMD_HIP(hipStreamSynchronize(Stream()));
-      };
-      // autotune the values per block of the runs kernel: each candidate
-      // timed on the device (three applies), the fastest kept
+      // lanes per run (log2) of each problem's runs of R rows, from their mean
+      // length: a row's sum is the same for every block size
+      std::vector<int64_t> cnt(9 * ns, 0), slots(9 * ns, 0);
+      for (int u = 0; u < nruns; u++) {
+        const int k = 9 * rseg[u] + rr[u + 1] - rr[u];
+        cnt[k]++;
+        slots[k] += rpp[u + 1] - rpp[u];
+      }
+      nblocks = (int)br.size() - 1;
+      std::vector<int4> info(2 * std::max(nblocks, 1), make_int4(0, 0, 0, 0));
+      for (int b = 0; b < nblocks; b++) {
+        const int k = 9 * bs[b] + bl[b], u0 = br[b], u1 = br[b + 1];
+        const int lg = RunGroupLog2(bl[b], (int)((slots[k] + cnt[k] - 1) / cnt[k]));
+        info[2 * b] = make_int4(u0, u1 - u0, rpp[u0], vp[u0]);
+        info[2 * b + 1] = make_int4(rr[u0], bl[b] | lg << 8, rpp[u1] - rpp[u0], bs[b]);
+      }
+      blk_info.alloc(info.size());
+      blk_info.upload(info.data(), info.size());
+      blk_seg.alloc(std::max<size_t>(bs.size(), 1));
+      blk_seg.upload(bs.data(), bs.size());
+      // first block of each problem (blocks are in problem order)
+      std::vector<int> sb(ns + 1);
+      for (int q = 0, b = 0; q <= ns; q++) {
+        while (b < nblocks && bs[b] < q) b++;
+        sb[q] = b;
+      }
+      seg_blk.alloc(sb.size());
+      seg_blk.upload(sb.data(), sb.size());
+      partials.alloc(std::max<size_t>({(size_t)nblocks, (size_t)ns, (size_t)1}));
+      NGSAMD_HIP(hipStreamSynchronize(Stream()));
+      // autotune the values per workgroup of the runs kernel (a block holds
+      // up to 1024, so that sums do not depend on it): each candidate timed
+      // on the device (three applies), the fastest kept
       const char* benv = getenv("NGSAMD_SPMV_NNZ");
       std::vector<int> cand = benv ? std::vector<int>{atoi(benv)} : std::vector<int>{1024, 2048, 4096};
       int best = cand[0];
@@ -450,7 +436,6 @@ BatchOp::BatchOp(int64_t n, const int64_t* rp, const int* c, const double* v, in
         NGSAMD_HIP(hipEventCreate(&e0));
         NGSAMD_HIP(hipEventCreate(&e1));
         for (int bn : cand) {
-          set_blocks(bn);
           LaunchBatchSpmv<double, double, false, true>(*this, rvals.p, tx.p, ty.p, 1.0, nullptr, st, bn);
           NGSAMD_HIP(hipEventRecord(e0, st));
           for (int k = 0; k < 3; k++)
@@ -467,7 +452,6 @@ BatchOp::BatchOp(int64_t n, const int64_t* rp, const int* c, const double* v, in
       }
       NGSAMD_REQUIRE(best == 1024 || best == 2048 || best == 4096, "NGSAMD_SPMV_NNZ must be 1024, 2048 or 4096");
       block_nnz = best;
-      set_blocks(best);
     }
   }
   if (!use_runs) {
@@ -508,6 +492,7 @@ BatchOp::BatchOp(int64_t n, const int64_t* rp, const int* c, const double* v, in
   chunk_seg.upload(csg.data(), csg.size());
   seg_chunk.alloc(sgc.size());
   seg_chunk.upload(sgc.data(), sgc.size());
+  cpartials.alloc(std::max(nchunks, 1));
 
   if (use_runs) {
     partials.alloc(std::max<size_t>({(size_t)nblocks, (size_t)nchunks, (size_t)1}));
@@ -586,6 +571,7 @@ static void Fill(T* x, int64_t n, T a, hipStream_t st) {
 
 struct BatchState {
   double* wdn;
+  double* wd;         // <w, d> before the last update
   double* alpha;
   double* beta;
   double* final_res;
@@ -599,13 +585,13 @@ struct BatchState {
 
 struct BatchWork {
   int nseg;
-  DevBuf<double> wdn, alpha, beta, final_res, tol, last_res;
+  DevBuf<double> wdn, wd, alpha, beta, final_res, tol, last_res;
   DevBuf<long long> finish;
   DevBuf<int> it, done;
   explicit BatchWork(int n)
-      : nseg(n), wdn(n), alpha(n), beta(n), final_res(n), tol(n), last_res(n), finish(n), it(n), done(n) {}
+      : nseg(n), wdn(n), wd(n), alpha(n), beta(n), final_res(n), tol(n), last_res(n), finish(n), it(n), done(n) {}
   BatchState state(int maxiter) {
-    return BatchState{wdn.p, alpha.p, beta.p, final_res.p, tol.p, last_res.p, finish.p, it.p, done.p, maxiter};
+    return BatchState{wdn.p, wd.p, alpha.p, beta.p, final_res.p, tol.p, last_res.p, finish.p, it.p, done.p, maxiter};
   }
 };
 
@@ -657,9 +643,11 @@ __device__ __forceinline__ void BatchCheck(BatchState& S, int p, double res) {
 
 // one workgroup per problem: sum of partials[first[p] .. first[p+1])
 __device__ __forceinline__ double SegmentSum(const double* partials, const int* first, int p, double* lds) {
-  double v = 0.0;
-  for (int i = first[p] + threadIdx.x; i < first[p + 1]; i += kBatchBlock) v += partials[i];
-  return BlockSum<kBatchBlock>(v, lds);
+  return SumPartials<kBatchBlock>(partials + first[p], first[p + 1] - first[p], lds);
+}
+// the same for every thread (lds: kBatchBlock / 64 + 1 doubles)
+__device__ __forceinline__ double SegmentSumAll(const double* partials, const int* first, int p, double* lds) {
+  return SumPartialsAll<kBatchBlock>(partials + first[p], first[p + 1] - first[p], lds);
 }
 
 __global__ __launch_bounds__(kBatchBlock) void BatchInitCheckKernel(const double* __restrict__ partials,
@@ -691,12 +679,6 @@ __device__ __forceinline__ void BatchAlphaProblem(const double* __restrict__ par
   }
 }
 
-__global__ __launch_bounds__(kBatchBlock) void BatchAlphaKernel(const double* __restrict__ partials,
-                                                                const int* __restrict__ seg_blk, BatchState S) {
-  __shared__ double lds[kBatchBlock / 64];
-  BatchAlphaProblem(partials, seg_blk, S, blockIdx.x, lds);
-}
-
 // u += al s, d -= al w, w = C d over dofs [i0, i1); returns this thread's
 // part of <w, d>
 template <class V>
@@ -723,22 +705,49 @@ __device__ __forceinline__ void BatchDirectionRange(V* __restrict__ s, const V* 
   for (int64_t i = i0 + threadIdx.x; i < i1; i += kBatchBlock) s[i] = beta * s[i] + w[i];
 }
 
+// alpha of the chunk's problem from its row blocks' partials bpart (every
+// workgroup of the problem forms the same bits; the problem's first one keeps
+// its state), the updates, the chunk's part of <w, d> into cpart.  Taking
+// alpha and, in the direction kernel, the stopping test and beta along saves
+// two kernels of one workgroup per problem (4.4 us each) an iteration.
 template <class V>
 __global__ __launch_bounds__(kBatchBlock) void BatchUpdateKernel(const V* __restrict__ inv, V* __restrict__ u,
                                                                  V* __restrict__ d, V* __restrict__ w,
                                                                  const V* __restrict__ s,
                                                                  const int64_t* __restrict__ cstart,
                                                                  const int* __restrict__ cseg, BatchState S,
-                                                                 double* __restrict__ partials) {
-  __shared__ double lds[kBatchBlock / 64];
+                                                                 const double* __restrict__ bpart,
+                                                                 const int* __restrict__ seg_blk,
+                                                                 const int* __restrict__ seg_chunk,
+                                                                 double* __restrict__ cpart) {
+  __shared__ double lds[kBatchBlock / 64 + 1];
+  __shared__ int stopped;
   const int c = blockIdx.x;
   const int p = cseg[c];
-  if (S.done[p]) {
-    if (threadIdx.x == 0) partials[c] = 0.0;
+  if (threadIdx.x == 0) stopped = S.done[p];  // one read: another workgroup may set it now
+  __syncthreads();
+  if (stopped) {
+    if (threadIdx.x == 0) cpart[c] = 0.0;
     return;
   }
-  const double acc = BatchUpdateRange<V>(inv, u, d, w, s, cstart[c], cstart[c + 1], (V)S.alpha[p]);
-  StorePartial<kBatchBlock>(acc, partials, lds);
+  const double as_s = SegmentSumAll(bpart, seg_blk, p, lds);
+  const double wd = S.wdn[p];
+  const bool first = c == seg_chunk[p] && threadIdx.x == 0;
+  if (as_s == 0.0 || wd == 0.0) {
+    if (threadIdx.x == 0) cpart[c] = 0.0;
+    if (first) {
+      S.done[p] = 2;
+      S.finish[p] = DeviceClock();
+    }
+    return;
+  }
+  const double alpha = wd / as_s;
+  if (first) {
+    S.alpha[p] = alpha;
+    S.wd[p] = wd;
+  }
+  const double acc = BatchUpdateRange<V>(inv, u, d, w, s, cstart[c], cstart[c + 1], (V)alpha);
+  StorePartial<kBatchBlock>(acc, cpart, lds);
 }
 
 // <w, d> of problem p from its chunks' partials, the stopping test and
@@ -756,20 +765,30 @@ __device__ __forceinline__ void BatchCheckProblem(const double* __restrict__ par
   }
 }
 
-__global__ __launch_bounds__(kBatchBlock) void BatchCheckKernel(const double* __restrict__ partials,
-                                                                const int* __restrict__ seg_chunk, BatchState S) {
-  __shared__ double lds[kBatchBlock / 64];
-  BatchCheckProblem(partials, seg_chunk, S, blockIdx.x, lds);
-}
-
+// beta of the chunk's problem from its chunks' partials, s = beta s + w; the
+// problem's first workgroup does the stopping test (the others may already
+// see it stopped: s is not used any more then)
 template <class V>
 __global__ __launch_bounds__(kBatchBlock) void BatchDirectionKernel(V* __restrict__ s, const V* __restrict__ w,
                                                                     const int64_t* __restrict__ cstart,
-                                                                    const int* __restrict__ cseg, BatchState S) {
+                                                                    const int* __restrict__ cseg, BatchState S,
+                                                                    const double* __restrict__ cpart,
+                                                                    const int* __restrict__ seg_chunk) {
+  __shared__ double lds[kBatchBlock / 64 + 1];
+  __shared__ int stopped;
   const int c = blockIdx.x;
   const int p = cseg[c];
-  if (S.done[p]) return;
-  BatchDirectionRange<V>(s, w, cstart[c], cstart[c + 1], (V)S.beta[p]);
+  if (threadIdx.x == 0) stopped = S.done[p];  // one read: another workgroup may set it now
+  __syncthreads();
+  if (stopped) return;
+  const double wdn = SegmentSumAll(cpart, seg_chunk, p, lds);
+  const double beta = wdn / S.wd[p];
+  if (c == seg_chunk[p] && threadIdx.x == 0) {
+    S.wdn[p] = wdn;
+    S.beta[p] = beta;
+    BatchCheck(S, p, sqrt(fabs(wdn)));
+  }
+  BatchDirectionRange<V>(s, w, cstart[c], cstart[c + 1], (V)beta);
 }
 
 // all problems done?  one workgroup
@@ -838,13 +857,10 @@ struct PersistentArgs {
   const double* vals;
   const int* blk_row;
   // runs layout
-  const int* run_row;
   const int* run_ptr;
-  const int* val_ptr;
   const int* rcols;
   const double* rvals;
-  const int* blk_run;
-  const int* blk_len;
+  const int4* blk_info;
   // blocks and chunks
   const int* blk_seg;
   const int* seg_blk;
@@ -870,7 +886,7 @@ struct PersistentArgs {
 
 template <int NNZ, bool RUNS>
 __global__ __launch_bounds__(kBatchBlock) void BatchCgPersistentKernel(PersistentArgs P) {
-  __shared__ double prod[NNZ];
+  __shared__ double prod[RUNS ? 1 : NNZ];
   __shared__ double lds[kBatchBlock / 64 + 1];
   __shared__ int flag;
   const int G = gridDim.x;
@@ -886,12 +902,13 @@ __global__ __launch_bounds__(kBatchBlock) void BatchCgPersistentKernel(Persisten
     __syncthreads();
     if (lds[kBatchBlock / 64] == 0.0) break;
     // (S) w = A s, <s, A s> per row block
-    for (int b = lb; b < P.nblocks; b += G) {
-      if constexpr (RUNS)
-        BatchRunsBlock<NNZ, double, double, false, true>(P.run_row, P.run_ptr, P.val_ptr, P.rcols, P.rvals, P.s, P.w,
-                                                         1.0, P.blk_run, P.blk_len, P.blk_seg, S.done, P.bpart, b,
-                                                         prod, lds);
-      else
+    if constexpr (RUNS) {
+      constexpr int waves = kBatchBlock / 64;
+      for (int b = lb * waves + (threadIdx.x >> 6); b < P.nblocks; b += G * waves)
+        BatchRunsBlock<double, double, false, true>(P.blk_info, P.run_ptr, P.rcols, P.rvals, P.s, P.w, 1.0, S.done,
+                                                    P.bpart, b);
+    } else {
+      for (int b = lb; b < P.nblocks; b += G)
         BatchSpmvBlock<NNZ, double, double, false, true>(P.rowptr, P.cols, P.vals, P.s, P.w, 1.0, P.blk_row,
                                                          P.blk_seg, S.done, P.bpart, b, prod, lds);
     }
@@ -922,18 +939,13 @@ __global__ __launch_bounds__(kBatchBlock) void BatchCgPersistentKernel(Persisten
 
 template <class V, class M>
 static void EnqueueBatchIteration(BatchOp& A, const M* vals, const V* inv, V* u, V* d, V* w, V* s, BatchState S,
-                                  int* all_done, hipStream_t st) {
+                                  hipStream_t st) {
   LaunchBatchSpmv<V, M, false, true>(A, vals, s, w, 1.0, S.done, st, A.block_nnz);
-  BatchAlphaKernel<<<A.nseg, kBatchBlock, 0, st>>>(A.partials.p, A.seg_blk.p, S);
-  NGSAMD_CHECK_LAUNCH();
   BatchUpdateKernel<V><<<A.nchunks, kBatchBlock, 0, st>>>(inv, u, d, w, s, A.chunk_start.p, A.chunk_seg.p, S,
-                                                           A.partials.p);
+                                                           A.partials.p, A.seg_blk.p, A.seg_chunk.p, A.cpartials.p);
   NGSAMD_CHECK_LAUNCH();
-  BatchCheckKernel<<<A.nseg, kBatchBlock, 0, st>>>(A.partials.p, A.seg_chunk.p, S);
-  NGSAMD_CHECK_LAUNCH();
-  BatchDirectionKernel<V><<<A.nchunks, kBatchBlock, 0, st>>>(s, w, A.chunk_start.p, A.chunk_seg.p, S);
-  NGSAMD_CHECK_LAUNCH();
-  BatchAllDoneKernel<<<1, kBatchBlock, 0, st>>>(S.done, A.nseg, all_done);
+  BatchDirectionKernel<V><<<A.nchunks, kBatchBlock, 0, st>>>(s, w, A.chunk_start.p, A.chunk_seg.p, S, A.cpartials.p,
+                                                              A.seg_chunk.p);
   NGSAMD_CHECK_LAUNCH();
 }
 
@@ -974,13 +986,10 @@ static void RunPersistent(BatchOp& A, const double* inv, double* u, double* d, d
   P.cols = A.cols.p;
   P.vals = A.vals.p;
   P.blk_row = A.blk_row.p;
-  P.run_row = A.run_row.p;
   P.run_ptr = A.run_ptr.p;
-  P.val_ptr = A.val_ptr.p;
   P.rcols = A.rcols.p;
   P.rvals = A.rvals.p;
-  P.blk_run = A.blk_run.p;
-  P.blk_len = A.blk_len.p;
+  P.blk_info = A.blk_info.p;
   P.blk_seg = A.blk_seg.p;
   P.seg_blk = A.seg_blk.p;
   P.nblocks = A.nblocks;
@@ -1001,9 +1010,7 @@ static void RunPersistent(BatchOp& A, const double* inv, double* u, double* d, d
   P.err = err.p;
   if (A.nblocks > 0 || A.nchunks > 0) {
     if (A.use_runs) {
-      if (A.block_nnz == 1024) LaunchPersistent<1024, true>(P, st);
-      else if (A.block_nnz == 4096) LaunchPersistent<4096, true>(P, st);
-      else LaunchPersistent<2048, true>(P, st);
+      LaunchPersistent<1024, true>(P, st);
     } else {
       if (A.block_nnz == 1024) LaunchPersistent<1024, false>(P, st);
       else if (A.block_nnz == 4096) LaunchPersistent<4096, false>(P, st);
@@ -1045,8 +1052,12 @@ static long long RunBatchCg(BatchOp& A, const M* vals, const V* inv, const V* rh
   } else {
     NGSAMD_REQUIRE(chunk >= 0, "batch cg: the persistent form is FP64 only");
   }
-  BatchAllDoneKernel<<<1, kBatchBlock, 0, st>>>(S.done, A.nseg, all.p);
-  NGSAMD_CHECK_LAUNCH();
+  // the flag that the host polls, once per launch
+  auto all_done = [&] {
+    BatchAllDoneKernel<<<1, kBatchBlock, 0, st>>>(S.done, A.nseg, all.p);
+    NGSAMD_CHECK_LAUNCH();
+  };
+  all_done();
 
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -1056,7 +1067,8 @@ static long long RunBatchCg(BatchOp& A, const M* vals, const V* inv, const V* rh
     if (e == hipSuccess) {
       bool ok = true;
       try {
-        for (int k = 0; k < chunk; k++) EnqueueBatchIteration<V, M>(A, vals, inv, u, d.p, w.p, s.p, S, all.p, st);
+        for (int k = 0; k < chunk; k++) EnqueueBatchIteration<V, M>(A, vals, inv, u, d.p, w.p, s.p, S, st);
+        all_done();
       } catch (...) {
         ok = false;
       }
@@ -1097,7 +1109,10 @@ static long long RunBatchCg(BatchOp& A, const M* vals, const V* inv, const V* rh
   long long launched = 0;
   auto enqueue = [&](int slot) {
     if (use_graph) NGSAMD_HIP(hipGraphLaunch(exec, st));
-    else EnqueueBatchIteration<V, M>(A, vals, inv, u, d.p, w.p, s.p, S, all.p, st);
+    else {
+      EnqueueBatchIteration<V, M>(A, vals, inv, u, d.p, w.p, s.p, S, st);
+      all_done();
+    }
     launched += per;
     NGSAMD_HIP(hipMemcpyAsync(&pin[slot], all.p, sizeof(int), hipMemcpyDeviceToHost, st));
     NGSAMD_HIP(hipEventRecord(ev[slot], st));
@@ -1342,13 +1357,12 @@ __global__ __launch_bounds__(kBatchBlock) void IrAllFrozenKernel(const int* __re
 struct IrDeviceWork {
   DevBuf<double> r, fnorm, rnorm, inv_rnorm, itol, relres;
   DevBuf<float> inv32, c32, d, w, s;
-  // all: every problem finished; inner_all: the inner iterations' own
-  // all-stopped flag (not used by the refinement)
-  DevBuf<int> frozen, pending, skip, restart, outer, inner_sum, all, inner_all;
+  // all: every problem finished
+  DevBuf<int> frozen, pending, skip, restart, outer, inner_sum, all;
   DevBuf<long long> finish;
   IrDeviceWork(int64_t n, int ns)
       : r(n), fnorm(ns), rnorm(ns), inv_rnorm(ns), itol(ns), relres(ns), inv32(n), c32(n), d(n), w(n), s(n),
-        frozen(ns), pending(ns), skip(ns), restart(ns), outer(ns), inner_sum(ns), all(1), inner_all(1), finish(ns) {}
+        frozen(ns), pending(ns), skip(ns), restart(ns), outer(ns), inner_sum(ns), all(1), finish(ns) {}
 };
 
 // one outer block: the steps of every problem whose inner solve stopped
@@ -1412,7 +1426,7 @@ static void RunBatchIrDevice(BatchOp& A, const double* inv, const double* f, dou
   auto enqueue_iterations = [&](int count) {
     for (int k = 0; k < count; k++) {
       EnqueueBatchIteration<float, float>(A, A.vals32.p, W.inv32.p, W.c32.p, W.d.p, W.w.p, W.s.p, S,
-                                          W.inner_all.p, st);
+                                          st);
       if ((k + 1) % kIrOuterEvery == 0) EnqueueOuterBlock(A, f, u, inv, W, S, tol, inner_tol, max_outer, st);
     }
   };
