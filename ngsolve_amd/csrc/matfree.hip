@@ -23,9 +23,10 @@
 // nd padded to 4, one pad word per point against LDS bank conflicts) is loaded
 // into LDS once per workgroup; every wavefront then walks element tiles.
 //
-// Scatter: GATHER (default) writes each element's result row to a
-// contribution buffer; a second kernel sums, per dof, the contributions in a
-// fixed order (deterministic, no atomics).  ATOMIC adds the element results
+// Scatter: GATHER (default) sums per element patch in LDS from 8192 elements
+// on (mfpatch.hip); on smaller meshes each element's result row goes to a
+// contribution buffer and a second kernel sums, per dof, the contributions in
+// a fixed order (both deterministic, no atomics).  ATOMIC adds the element results
 // with hardware floating-point atomics, as the reference kernel does.
 #include <algorithm>
 #include <climits>

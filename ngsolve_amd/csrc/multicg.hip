@@ -11,14 +11,19 @@
 // beta_j = 0) where the reference divides 0 by 0.
 //
 // The operator product reads the matrix once for all K components
-// (CsrOp::MultMulti); the vector kernels handle all components of a dof in
-// one thread, the update kernel forming the partials of the new w.d as it
-// writes w and d; inner products are per-workgroup partials folded in a
-// fixed order (deterministic).  The stopping test runs on the device: every
-// kernel returns at once after it has stopped, and the host enqueues 16
-// iterations at a time, reading the control word once per chunk.
+// (CsrOp::MultMulti).  An iteration is four kernels: the product, the partials
+// of <s_j, A s_j>, the update with the partials of the new w.d, the direction;
+// every workgroup of the last two sums the K x kMcGrid partials itself, in one
+// order (deterministic; a small L2 read against 4.4 us for each kernel of one
+// workgroup).  A thread keeps one component, so that a wavefront's accesses are
+// contiguous.  3D p=4 with K = 4: 82 us an iteration, 107 with a fold kernel
+// per product, three one-thread test kernels and a thread per dof.  The stopping
+// test runs on the device: every kernel returns at once after it has stopped,
+// and the host enqueues 16 iterations at a time, reading the control word once
+// per chunk.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <utility>
 #include <vector>
@@ -34,38 +39,83 @@ constexpr int kMcBlock = 256;
 constexpr int kMcGrid = 1024;  // workgroups of the dot kernels (fixed: same sums for every run)
 constexpr int kMaxRhs = 8;
 
-// partials[w K + j] = sum over the dofs of workgroup w of a[i K + j] b[i K + j]
+// A thread's entries of a vector of K components: component j of dofs i,
+// i + step, ..; threads past the last whole dof of the workgroup have none.
+struct McPart {
+  int j, rows;  // component; dofs a workgroup covers at once
+  int64_t i, step;
+  __device__ McPart(int64_t n, int K) : j(threadIdx.x % K), rows(kMcBlock / K) {
+    const int r = threadIdx.x / K;
+    i = r < rows ? blockIdx.x * (int64_t)rows + r : n;
+    step = (int64_t)gridDim.x * rows;
+  }
+};
+static int McGrid(int64_t n, int K) {
+  const int64_t rows = kMcBlock / K;
+  return (int)std::max<int64_t>(1, std::min<int64_t>((n + rows - 1) / rows, kMcGrid));
+}
+
+// partials[w K + j] = sum of v over the threads of component j
+__device__ __forceinline__ void StoreMcPartials(double v, const McPart& t, int K, double* __restrict__ partials) {
+  __shared__ double lds[kMcBlock], part[16 * kMaxRhs];
+  lds[threadIdx.x] = v;
+  __syncthreads();
+  if (threadIdx.x < 16 * K) {
+    double s = 0.0;
+    for (int r = threadIdx.x / K; r < t.rows; r += 16) s += lds[r * K + t.j];
+    part[threadIdx.x] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < K) {
+    double s = 0.0;
+    for (int r = 0; r < 16; r++) s += part[r * K + threadIdx.x];
+    partials[(int64_t)blockIdx.x * K + threadIdx.x] = s;
+  }
+}
+
+// out[j] (LDS) = sum over w < nwg of partials[w K + j], for every thread
+__device__ __forceinline__ void FoldMcPartials(const double* __restrict__ partials, int nwg, int K, double* out) {
+  __shared__ double lds[kMcBlock], part[16 * kMaxRhs];
+  const int rows = kMcBlock / K, j = threadIdx.x % K;
+  double v = 0.0;
+  if (threadIdx.x < rows * K)
+#pragma unroll 4
+    for (int k = threadIdx.x; k < nwg * K; k += rows * K) v += partials[k];
+  lds[threadIdx.x] = v;
+  __syncthreads();
+  if (threadIdx.x < 16 * K) {
+    double s = 0.0;
+    for (int r = threadIdx.x / K; r < rows; r += 16) s += lds[r * K + j];
+    part[threadIdx.x] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < K) {
+    double s = 0.0;
+    for (int r = 0; r < 16; r++) s += part[r * K + threadIdx.x];
+    out[threadIdx.x] = s;
+  }
+  __syncthreads();
+}
+
+// the partials of <a_j, b_j>
 __global__ __launch_bounds__(kMcBlock) void MultiDotPartialsKernel(const double* __restrict__ a,
                                                                    const double* __restrict__ b, int64_t n, int K,
                                                                    double* __restrict__ partials,
                                                                    const int* __restrict__ stop) {
   if (stop && *stop) return;
-  __shared__ double lds[kMcBlock / 64];
-  double acc[kMaxRhs];
-#pragma unroll
-  for (int j = 0; j < kMaxRhs; j++) acc[j] = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)kMcBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMcBlock) {
-#pragma unroll
-    for (int j = 0; j < kMaxRhs; j++)
-      if (j < K) acc[j] += a[i * K + j] * b[i * K + j];
-  }
-  for (int j = 0; j < K; j++) {
-    const double v = BlockSum<kMcBlock>(acc[j], lds);
-    if (threadIdx.x == 0) partials[(int64_t)blockIdx.x * K + j] = v;
-  }
+  const McPart t(n, K);
+  double acc = 0.0;
+#pragma unroll 4
+  for (int64_t i = t.i; i < n; i += t.step) acc += a[i * K + t.j] * b[i * K + t.j];
+  StoreMcPartials(acc, t, K, partials);
 }
 
-// out[j] = sum over w < nwg of partials[w K + j], one workgroup, fixed order
+// out[j] = <a_j, b_j> from its partials (one workgroup)
 __global__ __launch_bounds__(kMcBlock) void MultiDotFoldKernel(const double* __restrict__ partials, int nwg, int K,
-                                                               double* __restrict__ out, const int* __restrict__ stop) {
-  if (stop && *stop) return;
-  __shared__ double lds[kMcBlock / 64];
-  for (int j = 0; j < K; j++) {
-    double v = 0.0;
-    for (int w = threadIdx.x; w < nwg; w += kMcBlock) v += partials[(int64_t)w * K + j];
-    v = BlockSum<kMcBlock>(v, lds);
-    if (threadIdx.x == 0) out[j] = v;
-  }
+                                                               double* __restrict__ out) {
+  __shared__ double sum[kMaxRhs];
+  FoldMcPartials(partials, nwg, K, sum);
+  if (threadIdx.x < K) out[threadIdx.x] = sum[threadIdx.x];
 }
 
 __device__ __forceinline__ double SafeDiv(double a, double b) { return b != 0.0 ? a / b : 0.0; }
@@ -80,97 +130,96 @@ __global__ __launch_bounds__(kMcBlock) void MultiPrecondKernel(const double* __r
   }
 }
 
-// alpha_j = wd_j / kss_j;  u += alpha s;  d -= alpha w;  w = C d, and the
-// workgroup partials of the new <w_j, d_j> (launched on the dot kernels'
-// grid, so the sums are those MultiDotPartialsKernel would form)
-__global__ __launch_bounds__(kMcBlock) void MultiCgUpdateKernel(double* __restrict__ u, double* __restrict__ d,
-                                                                double* __restrict__ w,
-                                                                const double* __restrict__ s,
-                                                                const double* __restrict__ inv, int64_t n, int K,
-                                                                const double* __restrict__ wd,
-                                                                const double* __restrict__ kss,
-                                                                double* __restrict__ partials,
-                                                                const int* __restrict__ stop) {
-  if (*stop) return;
-  __shared__ double lds[kMcBlock / 64];
-  double al[kMaxRhs], acc[kMaxRhs];
-#pragma unroll
-  for (int j = 0; j < kMaxRhs; j++) {
-    al[j] = j < K ? SafeDiv(wd[j], kss[j]) : 0.0;
-    acc[j] = 0.0;
-  }
-  for (int64_t i = blockIdx.x * (int64_t)kMcBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMcBlock) {
-    const double c = inv ? inv[i] : 1.0;
-#pragma unroll
-    for (int j = 0; j < kMaxRhs; j++) {
-      if (j >= K) break;
-      const int64_t k = i * K + j;
-      u[k] += al[j] * s[k];
-      const double dk = d[k] - al[j] * w[k];
-      d[k] = dk;
-      const double wk = inv ? c * dk : dk;
-      w[k] = wk;
-      acc[j] += wk * dk;
-    }
-  }
-  for (int j = 0; j < K; j++) {
-    const double v = BlockSum<kMcBlock>(acc[j], lds);
-    if (threadIdx.x == 0) partials[(int64_t)blockIdx.x * K + j] = v;
-  }
-}
-
-// beta_j = wdn_j / wd_j;  s = beta s + w
-__global__ __launch_bounds__(kMcBlock) void MultiCgDirectionKernel(double* __restrict__ s,
-                                                                   const double* __restrict__ w, int64_t n, int K,
-                                                                   const double* __restrict__ wd,
-                                                                   const double* __restrict__ wdn,
-                                                                   const int* __restrict__ stop) {
-  if (*stop) return;
-  double be[kMaxRhs];
-#pragma unroll
-  for (int j = 0; j < kMaxRhs; j++) be[j] = j < K ? SafeDiv(wdn[j], wd[j]) : 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)kMcBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kMcBlock) {
-#pragma unroll
-    for (int j = 0; j < kMaxRhs; j++) {
-      if (j >= K) break;
-      const int64_t k = i * K + j;
-      s[k] = s[k] * be[j] + w[k];
-    }
-  }
-}
-
 __device__ double NormK(const double* v, int K) {
   double s = 0.0;
   for (int j = 0; j < K; j++) s += v[j] * v[j];
   return sqrt(s);
 }
 
+// kss_j = <s_j, A s_j> from its partials pk; <s, A s> = 0 for every component:
+// stop before the update (steps = it).  alpha_j = wd_j / kss_j;
+// u += alpha s;  d -= alpha w;  w = C d, and the partials pw of the new
+// <w_j, d_j>.  ctl[0] = stop flag, ctl[1] = steps: whether a workgroup sees the
+// flag or the zero sum, it returns.
+__global__ __launch_bounds__(kMcBlock) void MultiCgUpdateKernel(double* __restrict__ u, double* __restrict__ d,
+                                                                double* __restrict__ w,
+                                                                const double* __restrict__ s,
+                                                                const double* __restrict__ inv, int64_t n, int K,
+                                                                const double* __restrict__ wd,
+                                                                const double* __restrict__ pk,
+                                                                double* __restrict__ pw, int it,
+                                                                int* __restrict__ ctl) {
+  __shared__ double kss[kMaxRhs];
+  __shared__ int stopped;
+  if (threadIdx.x == 0) stopped = ctl[0];
+  __syncthreads();
+  if (stopped) return;
+  FoldMcPartials(pk, gridDim.x, K, kss);
+  if (NormK(kss, K) == 0.0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      ctl[0] = 1;
+      ctl[1] = it;
+    }
+    return;
+  }
+  const McPart t(n, K);
+  const double al = SafeDiv(wd[t.j], kss[t.j]);
+  double acc = 0.0;
+#pragma unroll 2
+  for (int64_t i = t.i; i < n; i += t.step) {
+    const int64_t k = i * K + t.j;
+    u[k] += al * s[k];
+    const double dk = d[k] - al * w[k];
+    d[k] = dk;
+    const double wk = inv ? inv[i] * dk : dk;
+    w[k] = wk;
+    acc += wk * dk;
+  }
+  StoreMcPartials(acc, t, K, pw);
+}
+
 // The loop test at the head of iteration it (1-based): go on while
 // it - 1 < maxiter and ||wdn|| > err; else stop with steps = it.
-// ctl[0] = stop flag, ctl[1] = steps.
+__device__ __forceinline__ void MultiCgHead(double norm, double err, int it, int maxiter, int* __restrict__ ctl) {
+  if (!(it - 1 < maxiter && norm > err)) {
+    ctl[0] = 1;
+    ctl[1] = it;
+  }
+}
 __global__ void MultiCgHeadKernel(const double* __restrict__ wdn, int K, double err, int it, int maxiter,
                                   int* __restrict__ ctl) {
-  if (threadIdx.x != 0 || ctl[0]) return;
-  if (!(it - 1 < maxiter && NormK(wdn, K) > err)) {
-    ctl[0] = 1;
-    ctl[1] = it;
-  }
+  if (threadIdx.x == 0) MultiCgHead(NormK(wdn, K), err, it, maxiter, ctl);
 }
 
-// <s, A s> = 0 for every component: stop before the update (steps = it)
-__global__ void MultiCgKssKernel(const double* __restrict__ kss, int K, int it, int* __restrict__ ctl) {
-  if (threadIdx.x != 0 || ctl[0]) return;
-  if (NormK(kss, K) == 0.0) {
-    ctl[0] = 1;
-    ctl[1] = it;
+// wdn from its partials pw (kept by the first workgroup, with
+// hist[it] = sqrt(||wdn||) and the head test of iteration it + 1);
+// beta_j = wdn_j / wd_j;  s = beta s + w
+__global__ __launch_bounds__(kMcBlock) void MultiCgDirectionKernel(double* __restrict__ s,
+                                                                   const double* __restrict__ w, int64_t n, int K,
+                                                                   const double* __restrict__ wd,
+                                                                   double* __restrict__ wdn,
+                                                                   const double* __restrict__ pw, double err, int it,
+                                                                   int maxiter, int* __restrict__ ctl,
+                                                                   double* __restrict__ hist) {
+  __shared__ double sum[kMaxRhs];
+  __shared__ int stopped;
+  if (threadIdx.x == 0) stopped = ctl[0];  // set by this kernel too: s is not used any more then
+  __syncthreads();
+  if (stopped) return;
+  FoldMcPartials(pw, gridDim.x, K, sum);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int j = 0; j < K; j++) wdn[j] = sum[j];
+    const double norm = NormK(sum, K);
+    hist[it] = sqrt(norm);
+    MultiCgHead(norm, err, it + 1, maxiter, ctl);
   }
-}
-
-// end of iteration it: hist[it] = sqrt(||wdn||)
-__global__ void MultiCgTailKernel(const double* __restrict__ wdn, int K, int it, const int* __restrict__ ctl,
-                                  double* __restrict__ hist) {
-  if (threadIdx.x != 0 || ctl[0]) return;
-  hist[it] = sqrt(NormK(wdn, K));
+  const McPart t(n, K);
+  const double be = SafeDiv(sum[t.j], wd[t.j]);
+#pragma unroll 4
+  for (int64_t i = t.i; i < n; i += t.step) {
+    const int64_t k = i * K + t.j;
+    s[k] = s[k] * be + w[k];
+  }
 }
 
 // d = f - d (initial residual with d = A u on entry)
@@ -209,20 +258,13 @@ extern "C" int ngsamd_cg_solve_multi(ngsamd_op_t mat, ngsamd_op_t pre, int nrhs,
     hipStream_t st = Stream();
     *h_steps = 0;
     if (n == 0) return;
-    DevBuf<double> d(m), w(m), s(m), partials((size_t)kMcGrid * K), dots(3 * K);
+    DevBuf<double> d(m), w(m), s(m), pk((size_t)kMcGrid * K), pw((size_t)kMcGrid * K), dots(2 * K);
     double* wd = dots.p;
     double* wdn = dots.p + K;
-    double* kss = dots.p + 2 * K;
-    const int grid = GridFor(n, kMcBlock, kMcGrid);
+    const int grid = McGrid(n, K);
     DevBuf<int> ctl(2);
     DevBuf<double> hist((size_t)maxiter + 1);
     NGSAMD_HIP(hipMemsetAsync(ctl.p, 0, sizeof(int) * 2, st));
-    auto dot = [&](const double* a, const double* b, double* out, const int* stop) {
-      MultiDotPartialsKernel<<<grid, kMcBlock, 0, st>>>(a, b, n, K, partials.p, stop);
-      NGSAMD_CHECK_LAUNCH();
-      MultiDotFoldKernel<<<1, kMcBlock, 0, st>>>(partials.p, grid, K, out, stop);
-      NGSAMD_CHECK_LAUNCH();
-    };
     // d = f (u = 0) or f - A u
     if (initialize) {
       LaunchFill(d_sol, m, 0.0, st);
@@ -235,7 +277,10 @@ extern "C" int ngsamd_cg_solve_multi(ngsamd_op_t mat, ngsamd_op_t pre, int nrhs,
     MultiPrecondKernel<<<GridFor(n, kMcBlock, 8192), kMcBlock, 0, st>>>(d.p, inv, w.p, n, K);
     NGSAMD_CHECK_LAUNCH();
     NGSAMD_HIP(hipMemcpyAsync(s.p, w.p, sizeof(double) * m, hipMemcpyDeviceToDevice, st));
-    dot(w.p, d.p, wdn, nullptr);
+    MultiDotPartialsKernel<<<grid, kMcBlock, 0, st>>>(w.p, d.p, n, K, pw.p, nullptr);
+    NGSAMD_CHECK_LAUNCH();
+    MultiDotFoldKernel<<<1, kMcBlock, 0, st>>>(pw.p, grid, K, wdn);
+    NGSAMD_CHECK_LAUNCH();
     std::vector<double> h_wdn(K);
     NGSAMD_HIP(hipMemcpyAsync(h_wdn.data(), wdn, sizeof(double) * K, hipMemcpyDeviceToHost, st));
     NGSAMD_HIP(hipStreamSynchronize(st));
@@ -250,31 +295,26 @@ extern "C" int ngsamd_cg_solve_multi(ngsamd_op_t mat, ngsamd_op_t pre, int nrhs,
     // the host reads the control word once per chunk, not per iteration.
     constexpr int kChunkIts = 16;
     int it = 0, h_ctl[2] = {0, 0};
+    MultiCgHeadKernel<<<1, 64, 0, st>>>(wdn, K, err, 1, maxiter, ctl.p);
+    NGSAMD_CHECK_LAUNCH();
     while (true) {
-      for (int c = 0; c < kChunkIts && it <= maxiter; c++) {
+      for (int c = 0; c < kChunkIts && it < maxiter; c++) {
         ++it;
-        MultiCgHeadKernel<<<1, 64, 0, st>>>(wdn, K, err, it, maxiter, ctl.p);
-        NGSAMD_CHECK_LAUNCH();
         A.MultMulti(K, s.p, w.p, st, ctl.p);  // w = A s
         std::swap(wd, wdn);                    // wd = wdn
-        dot(s.p, w.p, kss, ctl.p);
-        MultiCgKssKernel<<<1, 64, 0, st>>>(kss, K, it, ctl.p);
+        MultiDotPartialsKernel<<<grid, kMcBlock, 0, st>>>(s.p, w.p, n, K, pk.p, ctl.p);
         NGSAMD_CHECK_LAUNCH();
-        MultiCgUpdateKernel<<<grid, kMcBlock, 0, st>>>(d_sol, d.p, w.p, s.p, inv, n, K, wd, kss, partials.p,
-                                                       ctl.p);
+        MultiCgUpdateKernel<<<grid, kMcBlock, 0, st>>>(d_sol, d.p, w.p, s.p, inv, n, K, wd, pk.p, pw.p, it, ctl.p);
         NGSAMD_CHECK_LAUNCH();
-        MultiDotFoldKernel<<<1, kMcBlock, 0, st>>>(partials.p, grid, K, wdn, ctl.p);
-        NGSAMD_CHECK_LAUNCH();
-        MultiCgDirectionKernel<<<GridFor(n, kMcBlock, 8192), kMcBlock, 0, st>>>(s.p, w.p, n, K, wd, wdn, ctl.p);
-        NGSAMD_CHECK_LAUNCH();
-        MultiCgTailKernel<<<1, 64, 0, st>>>(wdn, K, it, ctl.p, hist.p);
+        MultiCgDirectionKernel<<<grid, kMcBlock, 0, st>>>(s.p, w.p, n, K, wd, wdn, pw.p, err, it, maxiter, ctl.p,
+                                                           hist.p);
         NGSAMD_CHECK_LAUNCH();
       }
       NGSAMD_HIP(hipMemcpyAsync(h_ctl, ctl.p, sizeof(int) * 2, hipMemcpyDeviceToHost, st));
       NGSAMD_HIP(hipStreamSynchronize(st));
       // the head test of iteration maxiter + 1 always stops
       if (h_ctl[0]) break;
-      NGSAMD_REQUIRE(it <= maxiter, "ngsamd_cg_solve_multi: internal error (no stop after maxiter)");
+      NGSAMD_REQUIRE(it < maxiter, "ngsamd_cg_solve_multi: internal error (no stop after maxiter)");
     }
     *h_steps = h_ctl[1];
     if (h_residuals) {

@@ -1,6 +1,7 @@
 // Wavefront / workgroup reductions.  Grid-wide sums are two-stage: every
-// workgroup stores its partial sum with a plain store, and a one-workgroup
-// kernel launched next on the same stream sums the partials in index order.
+// workgroup stores its partial sum with a plain store, and the kernel launched
+// next on the same stream sums the partials in index order: one workgroup, or
+// every workgroup that needs the sum (all form the same bits).
 // The kernel boundary makes the partials visible; no grid-wide fence is
 // needed (on a multi-XCD device an agent-scope release writes back L2, which
 // is far too expensive to do once per workgroup).  For a fixed launch shape

@@ -1,7 +1,8 @@
 // Pattern-runs layout of a CSR matrix, shared by the single and the batched
 // SpMV: up to kMaxRun consecutive rows with one column list store that list
 // once and their values column by column ([L][R]); runs are grouped into
-// blocks of equal run length with at most max_vals values and max_vals rows.
+// blocks of equal run length with at most max_vals values and max_vals rows
+// (the batched kernel's work units; the single one cuts its own tasks).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -11,7 +11,7 @@
 // or cell of an H1 space) form a run that stores the list once and its values
 // column by column.  Values still stream once (8 B per nonzero) but the column
 // numbers drop to 4 B per run entry and each gathered x entry serves the
-// whole run.
+// whole run.  A group of lanes per run keeps the run's row sums in registers.
 //
 // stream: int32 row pointers, int32 column numbers, FP64 values (12 B per
 // nonzero streamed once); the rows are cut on the host into blocks of consecutive
@@ -505,8 +505,7 @@ CsrOp::CsrOp(int64_t h, int64_t w, const int64_t* rp, const int* c, const double
   block_nnz = nnz_env ? atoi(nnz_env) : 0;
   NGSAMD_REQUIRE(block_nnz == 0 || block_nnz == 1024 || block_nnz == 2048 || block_nnz == 4096,
                  "NGSAMD_SPMV_NNZ must be 1024, 2048 or 4096");
-  // grid of the stream/runs applies: 16384 measured best at 32^3 p=4 (runs
-  // kernel 395 us; 8192 405, 4096 418, 65536 494)
+  // largest grid of the stream applies: 16384 measured best at 32^3 p=4
   max_grid = 16384;
   const char* grid_env = getenv("NGSAMD_SPMV_GRID");
   if (grid_env) {
@@ -518,12 +517,8 @@ CsrOp::CsrOp(int64_t h, int64_t w, const int64_t* rp, const int* c, const double
   NGSAMD_REQUIRE(algo_name.empty() || algo_name == "rowgroup" || algo_name == "stream" || algo_name == "runs",
                  "NGSAMD_SPMV must be rowgroup, stream or runs");
   if (algo_name.empty() || algo_name == "runs") {
-    // measured on the 32^3 p=4 matrix (us per apply, grid 16384 / 4096
-    // workgroups): 2048 values per block 395 / 418, 4096 466 / 423
+    // in the runs layout block_nnz bounds the values of one run
     const int saved = block_nnz;
-    // below a million nonzeros (cache-resident, few blocks) 1024-value
-    // blocks give twice the workgroups: 6.1 vs 7.1 us on the 64^2 p=3
-    // triangle matrix (0.63M nonzeros)
     if (block_nnz == 0) block_nnz = nnz < (int64_t(1) << 20) ? 1024 : 2048;
     // the runs layout pays when it saves at least a quarter of the column
     // numbers (H1 matrices of order >= 2 share patterns between the dofs of
