@@ -23,8 +23,8 @@
 // nd padded to 4, one pad word per point against LDS bank conflicts) is loaded
 // into LDS once per workgroup; every wavefront then walks element tiles.
 //
-// Scatter: GATHER (default) sums per element patch in LDS from 8192 elements
-// on (mfpatch.hip); on smaller meshes each element's result row goes to a
+// Scatter: GATHER (default) sums per element patch in LDS on larger meshes
+// (mfpatch.hip); on smaller meshes each element's result row goes to a
 // contribution buffer and a second kernel sums, per dof, the contributions in
 // a fixed order (both deterministic, no atomics).  ATOMIC adds the element results
 // with hardware floating-point atomics, as the reference kernel does.
@@ -1597,10 +1597,17 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
   // (NGSAMD_MF_PATCH=0: the general gather, =1: patches whatever the size, for
   // comparison)
   const char* penv = getenv("NGSAMD_MF_PATCH");
-  if (fac_kernel && scat == NGSAMD_SCATTER_GATHER && PatchShape(dim, nd, fac_kg) && !(penv && std::string(penv) == "0"))
+  const bool pforce = penv && std::string(penv) == "1", pnever = penv && std::string(penv) == "0";
+  // From where they are the faster form (us per apply, gather / patches): in
+  // 3D 8192 elements (FP64 p=2 9K 9.4 / 8.9, p=4 17.3 / 15.6), 16-bit 16384
+  // (p=4 9K 12.3 / 12.9, 16K 14.5 / 13.4); in 2D 240K element dofs (FP64 p=3
+  // 9K elements 7.4 / 8.1, 30K 10.1 / 8.8), 16-bit 480K (p=4 16K 8.2 / 8.7,
+  // 60K 13.2 / 10.6), never for p=1 (150K 12.0 / 13.3).
+  const int64_t pmin = dim == 3 ? (half ? 16384 : 8192) : (half ? 480000 : 240000) / nd;
+  if (fac_kernel && scat == NGSAMD_SCATTER_GATHER && PatchShape(dim, nd, fac_kg) && !pnever &&
+      (pforce || dim == 3 || nd > 3))
     patch.ok = patch.Build(dim, nd, ndof, half, prec == NGSAMD_PREC_F64, ks1, fstride * (half ? 2 : prec == NGSAMD_PREC_F64 ? 8 : 4),
-                           classes, S, hdofs, hmetric, el.data(), DeviceMaxLds(),
-                           penv && std::string(penv) == "1" ? 1 : 8192);
+                           classes, S, hdofs, hmetric, el.data(), DeviceMaxLds(), pforce ? 1 : (int)pmin);
   std::vector<int> gather_slots;  // element-major slots in gather order (kept for the tile-major copy)
   // dof -> contribution slots, ascending slot order (the order of each sum)
   std::vector<int> cnt(ndof + 1, 0);

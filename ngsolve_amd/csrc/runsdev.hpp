@@ -69,6 +69,24 @@ __device__ __forceinline__ void LoadPair(const double* p, double& a, double& b) 
   b = t.y;
 }
 
+// R adjacent floats in 16-, 8- and 4-byte loads, aligned like a float
+typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+template <int R>
+__device__ __forceinline__ void LoadFloats(const float* p, double* v) {
+  constexpr int n4 = R / 4 * 4, n2 = n4 + (R % 4) / 2 * 2;
+#pragma unroll
+  for (int q = 0; q < n4; q += 4) {
+    const float4u t = *reinterpret_cast<const float4u*>(p + q);
+    v[q] = t.x, v[q + 1] = t.y, v[q + 2] = t.z, v[q + 3] = t.w;
+  }
+  if constexpr (n2 > n4) {
+    const float2u t = *reinterpret_cast<const float2u*>(p + n4);
+    v[n4] = t.x, v[n4 + 1] = t.y;
+  }
+  if constexpr (R > n2) v[n2] = p[n2];
+}
+
 // acc[q][j] = this lane's share of row q of its run (first column c0, first
 // value v0, L slots) times component j0 + j of the K-vector x (a pointer), or
 // times x(column) (KC = 1)
@@ -94,8 +112,7 @@ __device__ __forceinline__ void RunPartials(const int* __restrict__ rcols, const
         for (int q = 0; q + 1 < R; q += 2) LoadPair(vp + q, v[i][q], v[i][q + 1]);
         if constexpr (R % 2 == 1) v[i][R - 1] = vp[R - 1];
       } else {
-#pragma unroll
-        for (int q = 0; q < R; q++) v[i][q] = (double)vp[q];
+        LoadFloats<R>(vp, v[i]);
       }
     }
 #pragma unroll
