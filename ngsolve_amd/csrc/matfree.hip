@@ -41,6 +41,7 @@
 #include "half.hpp"
 #include "matfree.hpp"
 #include "mfdev.hpp"
+#include "mfpart.hpp"
 #include "reduce.hpp"
 #include "runtime_state.hpp"
 
@@ -1205,90 +1206,6 @@ static bool SupportedFac16(int dim, int ks1, int mt, int kg, int nd) {
   return is(1, 1, 1, 4) || is(1, 1, 1, 10) || is(1, 2, 3, 20) || is(2, 3, 5, 35);
 }
 
-// Factor of each class's reference matrices (see MfFacKernel): the rows
-// Bw[(d,i)][q] = b_{q,i,d} sqrt(w_q) are orthonormalised by Gram-Schmidt with
-// pivoting on the largest remaining row (each new vector orthogonalised twice
-// against the basis), stopping when every remaining row is below 1e-10 of
-// the largest row; D[(d,i)][k] = Bw[(d,i)] . phi_k.  Returns the largest rank
-// over the classes (D has that many columns, zero beyond a class's own rank),
-// or 0 if a weight is not positive or D Phi misses Bw by more than 1e-12
-// relative.  D is [class][d][i][rank].
-static int FactorGradients(int dim, int nd, int nq, int nclass, const double* bmat, const double* w,
-                           std::vector<double>& D) {
-  for (int q = 0; q < nq; q++)
-    if (!(w[q] > 0.0)) return 0;
-  const int nr = dim * nd;
-  const size_t bsz = (size_t)nq * nd * dim;
-  std::vector<std::vector<double>> phis(nclass);
-  std::vector<double> Bw((size_t)nr * nq);
-  int rank = 0;
-  auto dot = [&](const double* a, const double* b) {
-    double t = 0.0;
-    for (int q = 0; q < nq; q++) t += a[q] * b[q];
-    return t;
-  };
-  for (int c = 0; c < nclass; c++) {
-    for (int d = 0; d < dim; d++)
-      for (int i = 0; i < nd; i++)
-        for (int q = 0; q < nq; q++)
-          Bw[((size_t)d * nd + i) * nq + q] = bmat[c * bsz + ((size_t)q * nd + i) * dim + d] * std::sqrt(w[q]);
-    std::vector<double> res(Bw);
-    std::vector<double>& phi = phis[c];
-    double norm0 = 0.0;
-    for (int r = 0; r < nr; r++) norm0 = std::max(norm0, std::sqrt(dot(&Bw[(size_t)r * nq], &Bw[(size_t)r * nq])));
-    if (norm0 == 0.0) continue;
-    for (int k = 0; k < std::min(nr, nq); k++) {
-      int best = -1;
-      double bn = 0.0;
-      for (int r = 0; r < nr; r++) {
-        const double t = std::sqrt(dot(&res[(size_t)r * nq], &res[(size_t)r * nq]));
-        if (t > bn) bn = t, best = r;
-      }
-      if (best < 0 || bn <= 1e-10 * norm0) break;
-      std::vector<double> v(res.begin() + (size_t)best * nq, res.begin() + (size_t)(best + 1) * nq);
-      for (int pass = 0; pass < 2; pass++) {
-        for (size_t j = 0; j < phi.size() / nq; j++) {
-          const double t = dot(v.data(), &phi[j * nq]);
-          for (int q = 0; q < nq; q++) v[q] -= t * phi[j * nq + q];
-        }
-        const double vn = std::sqrt(dot(v.data(), v.data()));
-        for (int q = 0; q < nq; q++) v[q] /= vn;
-      }
-      phi.insert(phi.end(), v.begin(), v.end());
-      for (int r = 0; r < nr; r++) {
-        double* rr = &res[(size_t)r * nq];
-        const double t = dot(rr, v.data());
-        for (int q = 0; q < nq; q++) rr[q] -= t * v[q];
-      }
-    }
-    rank = std::max(rank, (int)(phi.size() / nq));
-  }
-  if (rank == 0) return 0;
-  D.assign((size_t)nclass * nr * rank, 0.0);
-  for (int c = 0; c < nclass; c++) {
-    const std::vector<double>& phi = phis[c];
-    const int rc = (int)(phi.size() / nq);
-    double norm0 = 0.0, err = 0.0;
-    for (int d = 0; d < dim; d++)
-      for (int i = 0; i < nd; i++) {
-        std::vector<double> row(nq), rec(nq, 0.0);
-        for (int q = 0; q < nq; q++) row[q] = bmat[c * bsz + ((size_t)q * nd + i) * dim + d] * std::sqrt(w[q]);
-        double* Dr = &D[((size_t)c * nr + (size_t)d * nd + i) * rank];
-        for (int k = 0; k < rc; k++) {
-          Dr[k] = dot(row.data(), &phi[(size_t)k * nq]);
-          for (int q = 0; q < nq; q++) rec[q] += Dr[k] * phi[(size_t)k * nq + q];
-        }
-        for (int q = 0; q < nq; q++) {
-          norm0 = std::max(norm0, std::fabs(row[q]));
-          err = std::max(err, std::fabs(row[q] - rec[q]));
-        }
-      }
-    if (err > 1e-12 * norm0) return 0;
-  }
-  return rank;
-}
-
-
 template <int MODE, class V>
 static void LaunchElements(const MatFreeOp& A, const V* x, V* out, double s, const int* stop, hipStream_t st,
                            bool prepare);
@@ -1437,9 +1354,9 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
   }
   // factored kernels (default where an instance exists; NGSAMD_MF_KERNEL=ref
   // keeps the sum over S_c)
+  std::vector<double> D;  // their factors, [class][d][i][fac_rank]
   if (ref_kernel && nclass <= kMaxLdsClasses && !(getenv("NGSAMD_MF_KERNEL") &&
                                                   std::string(getenv("NGSAMD_MF_KERNEL")) == "ref")) {
-    std::vector<double> D;
     const int rank = FactorGradients(dim, nd, nq, nclass, bmat, w, D);
     const int kg = (rank + 3) / 4;
     const int nsl = dim * kg;
@@ -1606,8 +1523,8 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
   const int64_t pmin = dim == 3 ? (half ? 16384 : 8192) : (half ? 480000 : 240000) / nd;
   if (fac_kernel && scat == NGSAMD_SCATTER_GATHER && PatchShape(dim, nd, fac_kg) && !pnever &&
       (pforce || dim == 3 || nd > 3))
-    patch.ok = patch.Build(dim, nd, ndof, half, prec == NGSAMD_PREC_F64, ks1, fstride * (half ? 2 : prec == NGSAMD_PREC_F64 ? 8 : 4),
-                           classes, S, hdofs, hmetric, el.data(), DeviceMaxLds(), pforce ? 1 : (int)pmin);
+    patch.ok = patch.Build(dim, nd, ndof, prec, ks1, fstride * (half ? 2 : prec == NGSAMD_PREC_F64 ? 8 : 4), classes, S,
+                           D, fac_rank, hdofs, hmetric, el.data(), DeviceMaxLds(), pforce ? 1 : (int)pmin);
   std::vector<int> gather_slots;  // element-major slots in gather order (kept for the tile-major copy)
   // dof -> contribution slots, ascending slot order (the order of each sum)
   std::vector<int> cnt(ndof + 1, 0);

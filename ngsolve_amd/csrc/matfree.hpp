@@ -29,11 +29,13 @@ struct MfPatchPlan {
   DevBuf<double> d_metric;
   DevBuf<int> s_rowptr, s_slots, s_order;  // shared dofs: their partial sums
   DevBuf<double> part;
-  // false: fewer than min_elements, some class is no relabelling of class 0, a dof belongs to no
-  // element, or a patch does not fit into LDS
-  bool Build(int dim, int nd, int64_t ndof, bool half, bool f64, int ks1, int64_t fbytes,
-             const std::vector<MfClass>& classes, const std::vector<double>& S, const int* dofs, const double* metric,
-             const int* elnr, int max_lds, int64_t min_elements);
+  // S, D: the classes' reference matrices and their factors of rank `rank`.
+  // false: fewer than min_elements, some class is no relabelling of class 0
+  // (FP16 / BF16: its rounded factor is none), a dof belongs to no element, or
+  // a patch does not fit into LDS
+  bool Build(int dim, int nd, int64_t ndof, int prec, int ks1, int64_t fbytes, const std::vector<MfClass>& classes,
+             const std::vector<double>& S, const std::vector<double>& D, int rank, const int* dofs,
+             const double* metric, const int* elnr, int max_lds, int64_t min_elements);
   int Grid(bool f64_vectors) const {
     const int64_t resident = (int64_t)DeviceCUs() * occ[f64_vectors ? 1 : 0];
     return (int)(npatch < resident ? npatch : resident);

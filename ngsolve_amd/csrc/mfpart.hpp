@@ -143,6 +143,125 @@ inline bool MapClass(int dim, int nd, const double* S0, const double* Sc, ClassM
   return false;
 }
 
+// Factor of each class's reference matrices (see MfFacKernel): the rows
+// Bw[(d,i)][q] = b_{q,i,d} sqrt(w_q) are orthonormalised by Gram-Schmidt with
+// pivoting on the largest remaining row (each new vector orthogonalised twice
+// against the basis), stopping when every remaining row is below 1e-10 of
+// the largest row; D[(d,i)][k] = Bw[(d,i)] . phi_k.  Returns the largest rank
+// over the classes (D has that many columns, zero beyond a class's own rank),
+// or 0 if a weight is not positive or D Phi misses Bw by more than 1e-12
+// relative.  D is [class][d][i][rank].
+inline int FactorGradients(int dim, int nd, int nq, int nclass, const double* bmat, const double* w,
+                           std::vector<double>& D) {
+  for (int q = 0; q < nq; q++)
+    if (!(w[q] > 0.0)) return 0;
+  const int nr = dim * nd;
+  const size_t bsz = (size_t)nq * nd * dim;
+  std::vector<std::vector<double>> phis(nclass);
+  std::vector<double> Bw((size_t)nr * nq);
+  int rank = 0;
+  auto dot = [&](const double* a, const double* b) {
+    double t = 0.0;
+    for (int q = 0; q < nq; q++) t += a[q] * b[q];
+    return t;
+  };
+  for (int c = 0; c < nclass; c++) {
+    for (int d = 0; d < dim; d++)
+      for (int i = 0; i < nd; i++)
+        for (int q = 0; q < nq; q++)
+          Bw[((size_t)d * nd + i) * nq + q] = bmat[c * bsz + ((size_t)q * nd + i) * dim + d] * std::sqrt(w[q]);
+    std::vector<double> res(Bw);
+    std::vector<double>& phi = phis[c];
+    double norm0 = 0.0;
+    for (int r = 0; r < nr; r++) norm0 = std::max(norm0, std::sqrt(dot(&Bw[(size_t)r * nq], &Bw[(size_t)r * nq])));
+    if (norm0 == 0.0) continue;
+    for (int k = 0; k < std::min(nr, nq); k++) {
+      int best = -1;
+      double bn = 0.0;
+      for (int r = 0; r < nr; r++) {
+        const double t = std::sqrt(dot(&res[(size_t)r * nq], &res[(size_t)r * nq]));
+        if (t > bn) bn = t, best = r;
+      }
+      if (best < 0 || bn <= 1e-10 * norm0) break;
+      std::vector<double> v(res.begin() + (size_t)best * nq, res.begin() + (size_t)(best + 1) * nq);
+      for (int pass = 0; pass < 2; pass++) {
+        for (size_t j = 0; j < phi.size() / nq; j++) {
+          const double t = dot(v.data(), &phi[j * nq]);
+          for (int q = 0; q < nq; q++) v[q] -= t * phi[j * nq + q];
+        }
+        const double vn = std::sqrt(dot(v.data(), v.data()));
+        for (int q = 0; q < nq; q++) v[q] /= vn;
+      }
+      phi.insert(phi.end(), v.begin(), v.end());
+      for (int r = 0; r < nr; r++) {
+        double* rr = &res[(size_t)r * nq];
+        const double t = dot(rr, v.data());
+        for (int q = 0; q < nq; q++) rr[q] -= t * v[q];
+      }
+    }
+    rank = std::max(rank, (int)(phi.size() / nq));
+  }
+  if (rank == 0) return 0;
+  D.assign((size_t)nclass * nr * rank, 0.0);
+  for (int c = 0; c < nclass; c++) {
+    const std::vector<double>& phi = phis[c];
+    const int rc = (int)(phi.size() / nq);
+    double norm0 = 0.0, err = 0.0;
+    for (int d = 0; d < dim; d++)
+      for (int i = 0; i < nd; i++) {
+        std::vector<double> row(nq), rec(nq, 0.0);
+        for (int q = 0; q < nq; q++) row[q] = bmat[c * bsz + ((size_t)q * nd + i) * dim + d] * std::sqrt(w[q]);
+        double* Dr = &D[((size_t)c * nr + (size_t)d * nd + i) * rank];
+        for (int k = 0; k < rc; k++) {
+          Dr[k] = dot(row.data(), &phi[(size_t)k * nq]);
+          for (int q = 0; q < nq; q++) rec[q] += Dr[k] * phi[(size_t)k * nq + q];
+        }
+        for (int q = 0; q < nq; q++) {
+          norm0 = std::max(norm0, std::fabs(row[q]));
+          err = std::max(err, std::fabs(row[q] - rec[q]));
+        }
+      }
+    if (err > 1e-12 * norm0) return 0;
+  }
+  return rank;
+}
+
+// Whether the factor of class c is the one of class 0 relabelled, entry by entry
+// in the operand format that `bits` rounds to: the directions permuted and
+// turned by A, the dofs by the class map, the rank columns in some order
+// and with some signs.  D0, Dc [d][i][rank] (FactorGradients).
+template <class F>
+inline bool SameRoundedFactor(int dim, int nd, int rank, const double* D0, const double* Dc, const ClassMap& m, F bits) {
+  std::vector<int> pi(dim, -1), sd(dim, 0);
+  for (int d = 0; d < dim; d++) {  // column d of A: one entry, +-1
+    for (int r = 0; r < dim; r++)
+      if (m.A[r * dim + d] != 0.0) {
+        if (pi[d] >= 0) return false;
+        pi[d] = r;
+        sd[d] = m.A[r * dim + d] > 0 ? 1 : -1;
+      }
+    if (pi[d] < 0) return false;
+  }
+  std::vector<char> used(rank, 0);
+  for (int k = 0; k < rank; k++) {
+    auto same = [&](int q, int s) {
+      for (int d = 0; d < dim; d++)
+        for (int i = 0; i < nd; i++) {
+          const double a = Dc[((size_t)d * nd + i) * rank + k];
+          const double b = s * sd[d] * m.sign[i] * D0[((size_t)pi[d] * nd + m.perm[i]) * rank + q];
+          if (bits(a) != bits(b) && !(std::fabs(a) + std::fabs(b) < 1e-12)) return false;
+        }
+      return true;
+    };
+    int found = -1;
+    for (int q = 0; q < rank && found < 0; q++)
+      if (!used[q] && (same(q, 1) || same(q, -1))) found = q;
+    if (found < 0) return false;
+    used[found] = 1;
+  }
+  return true;
+}
+
 // Elements around each of the first nv dofs of the elements (the vertices of an
 // H1 element): adj[ptr[d] .. ptr[d + 1]).
 inline void VertexElements(int64_t nel, int nd, int nv, int64_t ndof, const int* dofs, std::vector<int>& ptr,

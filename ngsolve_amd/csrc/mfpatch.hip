@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "half.hpp"
 #include "matfree.hpp"
 #include "mfdev.hpp"
 #include "mfpart.hpp"
@@ -496,9 +497,12 @@ static void InThreads(int64_t n, int64_t grain, F f) {
     if (e) std::rethrow_exception(e);
 }
 
-bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, bool half_, bool f64_, int ks1_, int64_t fbytes,
-                        const std::vector<MfClass>& classes, const std::vector<double>& S, const int* dofs,
-                        const double* metric, const int* elnr, int max_lds, int64_t min_elements) {
+bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64_t fbytes,
+                        const std::vector<MfClass>& classes, const std::vector<double>& S,
+                        const std::vector<double>& D, int rank, const int* dofs, const double* metric, const int* elnr,
+                        int max_lds, int64_t min_elements) {
+  const bool f64_ = prec == NGSAMD_PREC_F64;
+  const bool half_ = prec == NGSAMD_PREC_BF16 || prec == NGSAMD_PREC_F16 || prec == NGSAMD_PREC_F16X3;
   const int nclass = (int)classes.size(), nc = dim * (dim + 1) / 2;
   const int64_t nel = nclass ? classes.back().end : 0;
   // Below 8192 elements (128 patches) a patch's chain of phases is longer
@@ -509,6 +513,15 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, bool half_, bool f64_, in
   const size_t ssz = (size_t)nc * nd * nd;
   for (int c = 0; c < nclass; c++)
     if (!MapClass(dim, nd, S.data(), S.data() + c * ssz, map[c])) return false;
+  // One 16-bit term: a class's results change with the rounding of its factor (3D
+  // p=4 structured meshes: one class of three maps with A = (1 0 0; -1 -1 -1;
+  // 0 1 0), BF16 results 4e-4 apart), so that the first class's must be the same
+  // rounded numbers.  Split FP16 and FP32 differ by less than their sums' rounding.
+  if (half_ && prec != NGSAMD_PREC_F16X3)
+    for (int c = 0; c < nclass; c++) {
+      const double* Dc = D.data() + (size_t)c * dim * nd * rank;
+      if (!SameRoundedFactor(dim, nd, rank, D.data(), Dc, map[c], prec == NGSAMD_PREC_F16 ? ToF16 : ToBf16)) return false;
+    }
   // elements by number: neighbours in the mesh are mostly near each other
   int64_t kmax = 0;
   for (int64_t e = 0; e < nel; e++) kmax = std::max<int64_t>(kmax, elnr[e]);

@@ -124,3 +124,25 @@ def test_cg_inner_product(device, monkeypatch, cells):
     assert abs(its[0] - its[1]) <= 1
     # both stop at 1e-12 in the preconditioned residual
     assert np.linalg.norm(sol[0] - sol[1]) <= 1e-10 * max(np.linalg.norm(sol[1]), 1e-300)
+
+
+@pytest.mark.parametrize("precision", ["f16", "bf16"])
+@pytest.mark.parametrize("dim,p", [(2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (3, 1), (3, 2), (3, 3), (3, 4)])
+def test_16bit_rounding_of_every_class(device, monkeypatch, dim, p, precision):
+    """One 16-bit term: each element class keeps the rounding of its own factor,
+    with patches or not.  The same 16-bit operands leave the order of the FP32
+    sums; where one turns the rounding of a second operand (about 1e-3 of them,
+    by 2^-11 or 2^-8 of it), results move by some 1e-6.  Another class's rounded
+    factor (3D p=4) moved them by 4e-5 (FP16) and 4e-4 (BF16)."""
+    say(f"[mfpatch 16-bit] {dim}D p={p} {precision}")
+    mesh = ngs.MakeStructured2DMesh(nx=31, ny=17) if dim == 2 else ngs.MakeStructured3DMesh(nx=5, ny=6, nz=7)
+    fes = ngs.H1(mesh, order=p, dirichlet=".*")
+    rng = np.random.default_rng(11)
+    kappa, x = np.exp(rng.standard_normal(mesh.ne)), rng.uniform(-1, 1, fes.ndof)
+    out = []
+    for patch in (True, False):
+        M = build(monkeypatch, fes, kappa, precision, patch)
+        dx, dy = dvec(x), N.DeviceVector(fes.ndof, 8)
+        M.op.mult(dx, dy)
+        out.append(dy.download())
+    assert np.linalg.norm(out[0] - out[1]) <= 1e-5 * np.linalg.norm(out[1])

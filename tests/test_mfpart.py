@@ -1,0 +1,133 @@
+"""Host planning of the matrix-free element patches
+(ngsolve_amd/csrc/mfpart.hpp): every vertex order of a triangle or tetrahedron
+mapped to the first one, and whether its rounded factor is the first one's
+relabelled."""
+import itertools
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from helpers import N
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROG = r"""
+#include <cstdio>
+#include "half.hpp"
+#include "mfpart.hpp"
+using namespace ngsamd;
+// in: dim, nd, nq, classes, weights, gradients [class][q][i][d]; out: rank,
+// factors, per class: found, same as BF16 / FP16, dofs, signs, A
+int main(int argc, char** argv) {
+  FILE* f = std::fopen(argv[1], "rb");
+  FILE* o = std::fopen(argv[2], "wb");
+  int h[4];
+  if (std::fread(h, 4, 4, f) != 4) return 1;
+  const int dim = h[0], nd = h[1], nq = h[2], nc = h[3], ncomp = dim * (dim + 1) / 2;
+  std::vector<double> w(nq), b((size_t)nc * nq * nd * dim), D, S((size_t)nc * ncomp * nd * nd, 0.0);
+  if (std::fread(w.data(), 8, nq, f) != (size_t)nq || std::fread(b.data(), 8, b.size(), f) != b.size()) return 1;
+  const int c3[6][2] = {{0, 0}, {1, 1}, {2, 2}, {0, 1}, {0, 2}, {1, 2}}, c2[3][2] = {{0, 0}, {1, 1}, {0, 1}};
+  for (int c = 0; c < nc; c++)
+    for (int k = 0; k < ncomp; k++)
+      for (int q = 0; q < nq; q++)
+        for (int i = 0; i < nd; i++)
+          for (int j = 0; j < nd; j++) {
+            const int x = dim == 3 ? c3[k][0] : c2[k][0], y = dim == 3 ? c3[k][1] : c2[k][1];
+            const double* g = &b[((size_t)c * nq + q) * nd * dim];
+            S[(((size_t)c * ncomp + k) * nd + i) * nd + j] +=
+                w[q] * (x == y ? g[i * dim + x] * g[j * dim + x]
+                               : g[i * dim + x] * g[j * dim + y] + g[i * dim + y] * g[j * dim + x]);
+          }
+  const int rank = FactorGradients(dim, nd, nq, nc, b.data(), w.data(), D);
+  std::fwrite(&rank, 4, 1, o);
+  std::fwrite(D.data(), 8, D.size(), o);
+  for (int c = 0; c < nc; c++) {
+    ClassMap m;
+    int r[3] = {MapClass(dim, nd, S.data(), &S[(size_t)c * ncomp * nd * nd], m), 0, 0};
+    if (r[0]) {
+      const double* Dc = &D[(size_t)c * dim * nd * rank];
+      r[1] = SameRoundedFactor(dim, nd, rank, D.data(), Dc, m, ToBf16);
+      r[2] = SameRoundedFactor(dim, nd, rank, D.data(), Dc, m, ToF16);
+    }
+    m.perm.resize(nd), m.sign.resize(nd);
+    std::fwrite(r, 4, 3, o);
+    std::fwrite(m.perm.data(), 4, nd, o);
+    std::fwrite(m.sign.data(), 1, nd, o);
+    std::fwrite(m.A, 8, dim * dim, o);
+  }
+  std::fclose(f);
+  std::fclose(o);
+  return 0;
+}
+"""
+
+
+def compile_host(d, prog):
+    src, exe = d / "t.cpp", d / "t"
+    src.write_text(prog)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-I", os.path.join(ROOT, "ngsolve_amd", "csrc"),
+                    str(src), "-o", str(exe)], check=True)
+    return exe
+
+
+@pytest.fixture(scope="module")
+def mapper(tmp_path_factory):
+    d = tmp_path_factory.mktemp("mfpart")
+    exe = compile_host(d, PROG)
+
+    def run(dim, w, b):
+        nc, nq, nd, _ = b.shape
+        (d / "in").write_bytes(np.int32([dim, nd, nq, nc]).tobytes() + w.tobytes() + np.ascontiguousarray(b).tobytes())
+        subprocess.run([str(exe), str(d / "in"), str(d / "out")], check=True)
+        raw = (d / "out").read_bytes()
+        rank = int(np.frombuffer(raw, np.int32, 1)[0])
+        D = np.frombuffer(raw, np.float64, nc * dim * nd * rank, 4).reshape(nc, dim, nd, rank)
+        kind = np.dtype([("r", "<i4", 3), ("perm", "<i4", nd), ("sign", "i1", nd), ("A", "<f8", (dim, dim))])
+        return D, np.frombuffer(raw, kind, nc, 4 + D.size * 8)
+
+    return run
+
+
+def gradients(dim, p, orders):
+    ir = N.TrigRule(max(2 * p - 2, 1)) if dim == 2 else N.TetRule(max(2 * p - 2, 1))
+    pts, w = np.asarray(ir.points), np.ascontiguousarray(ir.weights)
+    b = np.stack([np.asarray(N.ReferenceShapes(dim, p, list(o), np.ascontiguousarray(pts[:, :dim]))[1]) for o in orders])
+    return w, b
+
+
+@pytest.mark.parametrize("dim,p", [(2, 1), (2, 2), (2, 3), (2, 4), (2, 5), (3, 1), (3, 2), (3, 3), (3, 4)])
+def test_every_vertex_order_maps_to_the_first(mapper, dim, p):
+    orders = list(itertools.permutations(range(dim + 1)))
+    w, b = gradients(dim, p, orders)
+    D, maps = mapper(dim, w, b)
+    G = np.array([[1.3, 0.2, -0.4], [0.2, 0.9, 0.1], [-0.4, 0.1, 2.1]])[:dim, :dim]
+
+    def form(c, G):
+        return np.einsum("q,qid,de,qje->ij", w, b[c], G, b[c])
+
+    for c, m in enumerate(maps):
+        assert m["r"][0], orders[c]
+        K0 = form(0, m["A"] @ G @ m["A"].T)[np.ix_(m["perm"], m["perm"])] * np.outer(m["sign"], m["sign"])
+        K = form(c, G)
+        assert np.abs(K - K0).max() <= 1e-10 * np.abs(K).max()
+        # FP16: the rounded factors give the same matrices to the last bits where they are called the same
+        if m["r"][2]:
+            h0, hc = (np.asarray(D[k], np.float16).astype(np.float64) for k in (0, c))
+            R = np.einsum("dik,de,ejk->ij", hc, G, hc)
+            R0 = np.einsum("dik,de,ejk->ij", h0, m["A"] @ G @ m["A"].T, h0)[np.ix_(m["perm"], m["perm"])]
+            assert np.abs(R - R0 * np.outer(m["sign"], m["sign"])).max() <= 1e-13 * np.abs(R).max()
+    assert maps[0]["r"].all()
+
+
+@pytest.mark.parametrize("p,same", [(1, True), (2, True), (3, True), (4, False)])
+def test_structured_3d_classes_of_one_rounded_factor(mapper, p, same):
+    """Of the three vertex orders of a structured 3D mesh at p=4 one maps with
+    directions mixed: its factor rounds to other numbers."""
+    fes = N.H1Space(N.MakeStructured3DMesh(3, 3, 3), p, 1)
+    ir = N.TetRule(max(2 * p - 2, 1))
+    b = np.stack([np.asarray(c["bmat"]) for c in N.BuildClasses(fes, ir)])
+    _, maps = mapper(3, np.ascontiguousarray(ir.weights), b)
+    assert len(maps) == 3 and maps["r"][:, 0].all()
+    assert bool(maps["r"][:, 1].all()) == same and bool(maps["r"][:, 2].all()) == same
