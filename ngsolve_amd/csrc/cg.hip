@@ -147,9 +147,10 @@ __global__ __launch_bounds__(kCgBlock) void CgUpdateKernel(const V* __restrict__
                                                            const V* __restrict__ s, int64_t n, CGScalars* S, int P,
                                                            const double* __restrict__ pa, int na,
                                                            double* __restrict__ pw) {
-  if (S->done) return;
-  __shared__ double lds[kCgBlock / 64 + 1];
-  const double as_s = SumPartialsAll<kCgBlock>(pa, na, lds);
+  __shared__ double lds[kCgBlock / 64 + 2];
+  bool stopped;
+  const double as_s = SumPartialsUnless<kCgBlock>(&S->done, stopped, pa, na, lds);
+  if (stopped) return;
   const double wd = S->wdn[P];
   if (as_s == 0.0 || wd == 0.0) {
     if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 2;
@@ -181,9 +182,10 @@ template <class V>
 __global__ __launch_bounds__(kCgBlock) void CgDirectionKernel(V* __restrict__ s, const V* __restrict__ w, int64_t n,
                                                               CGScalars* S, int P, const double* __restrict__ pw,
                                                               int nw, double* residuals) {
-  if (S->done) return;
-  __shared__ double lds[kCgBlock / 64 + 1];
-  const double wdn = SumPartialsAll<kCgBlock>(pw, nw, lds);
+  __shared__ double lds[kCgBlock / 64 + 2];
+  bool stopped;
+  const double wdn = SumPartialsUnless<kCgBlock>(&S->done, stopped, pw, nw, lds);
+  if (stopped) return;
   const double beta = wdn / S->wdn[P];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     S->wdn[P ^ 1] = wdn;
@@ -220,9 +222,10 @@ __global__ __launch_bounds__(kCgBlock) void CgUpdatePairKernel(const double* __r
                                                                double* __restrict__ pair, int64_t n, CGScalars* S, int P,
                                                                const double* __restrict__ pa, int na,
                                                                double* __restrict__ pw) {
-  if (S->done) return;
-  __shared__ double lds[kCgBlock / 64 + 1];
-  const double as_s = SumPartialsAll<kCgBlock>(pa, na, lds);
+  __shared__ double lds[kCgBlock / 64 + 2];
+  bool stopped;
+  const double as_s = SumPartialsUnless<kCgBlock>(&S->done, stopped, pa, na, lds);
+  if (stopped) return;
   const double wd = S->wdn[P ^ 1];
   if (as_s == 0.0 || wd == 0.0) {
     if (blockIdx.x == 0 && threadIdx.x == 0) S->done = 2;
@@ -383,7 +386,7 @@ static void EnqueuePairIteration(ngsamd_op_t A, const double* inv, double* u, do
   const int g = CgGrid(n);
   double* next = P ? pair0 : pair1;
   const CgDirection D{P ? pair1 : pair0, next, dS, B.w, g, P, residuals};
-  const int na = static_cast<CsrOp*>(A)->MultDotDirection(D, w, B.a, &dS->done, st);
+  const int na = static_cast<CsrOp*>(A)->MultDotDirection(D, w, B.a, st);
   CgUpdatePairKernel<<<g, kCgBlock, 0, st>>>(inv, u, d, w, next, n, dS, P, B.a, na, B.w);
   NGSAMD_CHECK_LAUNCH();
 }

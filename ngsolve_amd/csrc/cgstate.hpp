@@ -51,9 +51,11 @@ struct CgDirection {
 // beta = <w,d> / previous <w,d> (0 in the first iteration), the same bits in
 // every workgroup; workgroup 0 also keeps <w,d> for the update kernel and does
 // the stopping test (the others may go on: their results are not used once
-// the loop has stopped).  lds: kCgBlock / 64 + 1 doubles.
-__device__ __forceinline__ double DirectionBeta(const CgDirection& D, double* lds) {
-  const double wdn = SumPartialsAll<kCgBlock>(D.pw, D.nw, lds);
+// the loop has stopped).  stopped: the loop had stopped before this kernel, or
+// workgroup 0 has seen it stop.  lds: kCgBlock / 64 + 2 doubles.
+__device__ __forceinline__ double DirectionBeta(const CgDirection& D, bool& stopped, double* lds) {
+  const double wdn = SumPartialsUnless<kCgBlock>(&D.S->done, stopped, D.pw, D.nw, lds);
+  if (stopped) return 0.0;
   const double wd = D.S->wdn[D.P];
   const double beta = wd == 0.0 ? 0.0 : wdn / wd;
   if (blockIdx.x == 0 && threadIdx.x == 0) {

@@ -55,7 +55,7 @@ struct CsrOp : ngsamd_op_s {
   // MultDot with the direction step (CgDirection): w = A s for the new s,
   // whose entries the kernel forms and stores
   bool FormsDirection() const;
-  int MultDotDirection(const CgDirection& D, double* w, double* partials, const int* d_stop, hipStream_t st);
+  int MultDotDirection(const CgDirection& D, double* w, double* partials, hipStream_t st);
   // Y = A X for K vectors stored interleaved ([n][K]); the matrix is read
   // once for all K in the runs layout
   // (all kernels return at once when *stop != 0, stop may be null)

@@ -72,4 +72,23 @@ __device__ __forceinline__ double SumPartialsAll(const double* partials, int cou
   return lds[BLOCK / 64];
 }
 
+// SumPartialsAll of a kernel that ends at once when *stop != 0 and whose grid
+// may set it: the workgroup reads the flag once (stopped), so that its
+// wavefronts, which start at different times, all go on or all return; the sum
+// of a stopped workgroup is not used.  The flag shares the sum's last barrier.
+// lds must hold BLOCK/64 + 2 doubles.
+template <int BLOCK>
+__device__ __forceinline__ double SumPartialsUnless(const int* stop, bool& stopped, const double* partials, int count,
+                                                    double* lds) {
+  const int flag = threadIdx.x == 0 ? *stop : 0;
+  const double v = SumPartials<BLOCK>(partials, count, lds);
+  if (threadIdx.x == 0) {
+    lds[BLOCK / 64] = v;
+    lds[BLOCK / 64 + 1] = flag;
+  }
+  __syncthreads();
+  stopped = lds[BLOCK / 64 + 1] != 0.0;
+  return lds[BLOCK / 64];
+}
+
 }  // namespace ngsamd

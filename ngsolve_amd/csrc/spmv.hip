@@ -294,21 +294,23 @@ __device__ __forceinline__ void RunTaskRows(const RunHead& h, const int* __restr
 // values alone, 5.2 TB/s with the shared columns), 20x16x24 p=4 97 -> 64,
 // 61x67 p=3 6.0 -> 4.3.
 // DIR (with DOT): x is the new search direction, formed from the pairs of D
-// and stored by the rows' owners (CgDirection).
+// and stored by the rows' owners (CgDirection, which holds the stop flag).
 template <bool ACCUM, bool DOT, bool DIR>
 __global__ __launch_bounds__(kStreamBlock, DIR ? 4 : 6) void CsrRunsKernel(
     const int4* __restrict__ tasks, int ntasks, const int* __restrict__ run_ptr,
     const int* __restrict__ rcols, const double* __restrict__ rvals, const double* __restrict__ xv,
     double* __restrict__ y, double s, double* __restrict__ partials, const int* __restrict__ stop_flag, int reverse,
     CgDirection D) {
-  if (stop_flag && *stop_flag) return;
   static_assert(kStreamBlock == kCgBlock, "DirectionBeta");
-  __shared__ double lds[kStreamBlock / 64 + 1];
+  __shared__ double lds[kStreamBlock / 64 + 2];
   typename std::conditional<DIR, PairX, PlainX>::type x;
   if constexpr (DIR) {
-    x.beta = DirectionBeta(D, lds);
+    bool stopped;
+    x.beta = DirectionBeta(D, stopped, lds);
+    if (stopped) return;
     x.pair = reinterpret_cast<const double2*>(D.pair);
   } else {
+    if (stop_flag && *stop_flag) return;
     x.x = xv;
   }
   const int lx = XcdContiguousBlock(blockIdx.x, gridDim.x);
@@ -743,11 +745,10 @@ int CsrOp::MultDot(const double* x, double* y, double* partials, const int* d_st
 
 bool CsrOp::FormsDirection() const { return algo == 2 && width > 0 && DotWorkgroups(*this) <= 1024; }
 
-int CsrOp::MultDotDirection(const CgDirection& D, double* w, double* partials, const int* stop,
-                            hipStream_t st) {
+int CsrOp::MultDotDirection(const CgDirection& D, double* w, double* partials, hipStream_t st) {
   const int wg = RunsGrid(*this, RunsDotCap(*this));
   CsrRunsKernel<false, true, true><<<wg, kStreamBlock, 0, st>>>(tasks.p, ntasks, run_ptr.p, rcols.p, rvals.p, nullptr,
-                                                                w, 1.0, partials, stop, 0, D);
+                                                                w, 1.0, partials, nullptr, 0, D);
   NGSAMD_CHECK_LAUNCH();
   return wg;
 }

@@ -52,3 +52,25 @@ def test_zero_right_hand_side(device):
     du = dvec(np.full(P["ndof"], 3.0))
     its, res = N.CGSolve(A, C, dvec(np.zeros(P["ndof"])), du, True, 1e-10, -1.0, 100, 16)
     assert its == 1 and res[0] == 0.0 and not du.download().any()
+
+
+@pytest.mark.parametrize("layout", ["runs", "stream"])
+@pytest.mark.parametrize("n,chunk", [(1, 0), (5000, 16), (250000, 0), (250000, 16)])
+def test_breakdown_leaves_the_solution(device, monkeypatch, layout, n, chunk):
+    """<s, A s> = 0 at the first step: every workgroup of the update sees it, or
+    the flag that the first one sets, and none of them touches u."""
+    say(f"[cg breakdown] {layout} n={n} chunk={chunk}")
+    monkeypatch.setenv("NGSAMD_SPMV", layout)
+    # pairs of rows with two columns each, all values 0
+    i = np.arange(n, dtype=np.int32)
+    cols = np.stack([i // 2 * 2, np.minimum(i // 2 * 2 + 1, n - 1)], 1)
+    cols = cols[:, :1] if n == 1 else cols
+    rp = np.arange(n + 1, dtype=np.int64) * cols.shape[1]
+    A = N.CreateCSR(n, n, rp, np.ascontiguousarray(cols.ravel()), np.zeros(cols.size))
+    C = N.CreateJacobi(np.full(n, 2.0), None)
+    u0 = np.random.default_rng(1).uniform(-1, 1, n)
+    for _ in range(3):
+        du = dvec(u0)
+        its, res = N.CGSolve(A, C, dvec(np.ones(n)), du, False, 1e-10, -1.0, 50, chunk)
+        assert its == 1 and res[0] == pytest.approx(np.sqrt(n / 2), rel=1e-12)
+        assert np.array_equal(du.download(), u0)
