@@ -263,14 +263,17 @@ inline bool SameRoundedFactor(int dim, int nd, int rank, const double* D0, const
 }
 
 // Elements around each of the first nv dofs of the elements (the vertices of an
-// H1 element): adj[ptr[d] .. ptr[d + 1]).
-inline void VertexElements(int64_t nel, int nd, int nv, int64_t ndof, const int* dofs, std::vector<int>& ptr,
+// H1 element): adj[ptr[d] .. ptr[d + 1]), d up to the largest of these dofs.
+inline void VertexElements(int64_t nel, int nd, int nv, const int* dofs, std::vector<int>& ptr,
                            std::vector<int>& adj) {
-  ptr.assign(ndof + 1, 0);
+  int last = -1;
+  for (int64_t e = 0; e < nel; e++)
+    for (int k = 0; k < nv; k++) last = std::max(last, dofs[e * nd + k]);
+  ptr.assign((size_t)last + 2, 0);
   for (int64_t e = 0; e < nel; e++)
     for (int k = 0; k < nv; k++) ptr[dofs[e * nd + k] + 1]++;
-  for (int64_t d = 0; d < ndof; d++) ptr[d + 1] += ptr[d];
-  adj.resize(ptr[ndof]);
+  for (int d = 0; d <= last; d++) ptr[d + 1] += ptr[d];
+  adj.resize(ptr.back());
   std::vector<int> pos(ptr.begin(), ptr.end() - 1);
   for (int64_t e = 0; e < nel; e++)
     for (int k = 0; k < nv; k++) adj[pos[dofs[e * nd + k]]++] = (int)e;
@@ -279,10 +282,13 @@ inline void VertexElements(int64_t nel, int nd, int nv, int64_t ndof, const int*
 // Cuts the elements e0 .. e1 - 1 into patches of `size` (the last one
 // smaller), order[e0 .. e1): each grows from a seed beside the previous patch by
 // the element sharing the most of its first nv dofs with the patch, the earliest
-// found first.
-inline void GrowPatches(int64_t e0, int64_t e1, int nd, int nv, int64_t ndof, const int* dofs,
-                        const std::vector<int>& ptr, const std::vector<int>& adj, int size, int* order) {
-  std::vector<int> stamp(ndof, -1), touched;
+// found first.  stamp: the last patch of each vertex dof, 0 at first, and
+// `patch` their number, kept from one call of a thread to the next (an array
+// per call would take the whole mesh's size for each piece of it: 96^3 cubes
+// p=4 39 s of set-up in place of 0.5).
+inline void GrowPatches(int64_t e0, int64_t e1, int nd, int nv, const int* dofs, const std::vector<int>& ptr,
+                        const std::vector<int>& adj, int size, std::vector<int>& stamp, int& patch, int* order) {
+  std::vector<int> touched;
   std::vector<unsigned char> score(e1 - e0, 0), taken(e1 - e0, 0);
   std::vector<std::vector<int>> q(nv + 1);
   std::vector<size_t> head(nv + 1, 0);
@@ -296,7 +302,8 @@ inline void GrowPatches(int64_t e0, int64_t e1, int nd, int nv, int64_t ndof, co
     return -1;
   };
   int seed = -1;
-  for (int patch = 0; n < e1; patch++) {
+  while (n < e1) {
+    patch++;
     for (int e : touched) score[e - e0] = 0;
     touched.clear();
     for (int s = 0; s <= nv; s++) {
@@ -326,5 +333,44 @@ inline void GrowPatches(int64_t e0, int64_t e1, int nd, int nv, int64_t ndof, co
     seed = pop();
   }
 }
+
+// Numbers the distinct values of a list in the order they are added: a table
+// of the list's size (the dofs of a patch), whatever the range of the values.
+class Numbering {
+ public:
+  explicit Numbering(size_t most) {
+    while (((size_t)1 << bits_) < 2 * most) bits_++;
+    key_.assign((size_t)1 << bits_, 0);
+    num_.resize(key_.size());
+    round_.assign(key_.size(), 0);
+  }
+  void Clear() {
+    n_ = 0;
+    cur_++;
+  }
+  // the number of v, given to it now if it has none (then it equals the former Size())
+  int Add(int v) {
+    size_t h = Slot(v);
+    if (round_[h] != cur_) {
+      round_[h] = cur_;
+      key_[h] = v;
+      num_[h] = n_++;
+    }
+    return num_[h];
+  }
+  int Size() const { return n_; }
+
+ private:
+  size_t Slot(int v) const {
+    const size_t mask = key_.size() - 1;
+    size_t h = ((uint32_t)v * 2654435769u) >> (32 - bits_);
+    while (round_[h] == cur_ && key_[h] != v) h = (h + 1) & mask;
+    return h;
+  }
+  int bits_ = 4, n_ = 0;
+  uint32_t cur_ = 1;
+  std::vector<int> key_, num_;
+  std::vector<uint32_t> round_;
+};
 
 }  // namespace ngsamd

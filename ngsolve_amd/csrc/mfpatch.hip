@@ -549,11 +549,14 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   {
     const int nv = std::min(dim + 1, nd);
     std::vector<int> vptr, vadj;
-    VertexElements(nel, nd, nv, ndof, sd.data(), vptr, vadj);
+    VertexElements(nel, nd, nv, sd.data(), vptr, vadj);
     const int64_t chunk = (int64_t)128 * size;
     InThreads((nel + chunk - 1) / chunk, 1, [&](int64_t a, int64_t b) {
+      std::vector<int> stamp(vptr.size(), 0);
+      int patch = 0;
       for (int64_t c = a; c < b; c++)
-        GrowPatches(c * chunk, std::min(nel, (c + 1) * chunk), nd, nv, ndof, sd.data(), vptr, vadj, size, order.data());
+        GrowPatches(c * chunk, std::min(nel, (c + 1) * chunk), nd, nv, sd.data(), vptr, vadj, size, stamp, patch,
+                    order.data());
     });
   }
 
@@ -597,21 +600,23 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   };
   std::vector<int> max_local(npatch, 0);
   InThreads(npatch, 16, [&](int64_t pa, int64_t pb) {
-    std::vector<int> at(ndof, -1), dl, c, o;
+    Numbering number((size_t)size * nd);
+    std::vector<int> at((size_t)size * nd), dl, c, o;  // at: number of each element dof among the patch's dl
     for (int64_t p = pa; p < pb; p++) {
       Patch& P = pt[p];
       const int64_t i0 = p * size, i1 = std::min<int64_t>(nel, i0 + size);
       dl.clear();
       c.clear();
+      number.Clear();
       for (int64_t i = i0; i < i1; i++)
         for (int k = 0; k < nd; k++) {
-          const int d = sd[(size_t)order[i] * nd + k];
-          if (at[d] < 0) {
-            at[d] = (int)dl.size();
+          const int d = sd[(size_t)order[i] * nd + k], a = number.Add(d);
+          at[(size_t)(i - i0) * nd + k] = a;
+          if (a == (int)dl.size()) {
             dl.push_back(d);
             c.push_back(0);
           }
-          c[at[d]]++;
+          c[a]++;
         }
       o.resize(dl.size());
       for (size_t q = 0; q < o.size(); q++) o[q] = (int)q;
@@ -644,7 +649,7 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
         const int e = row[order[i]];
         const ClassMap& m = map[cls[e]];
         for (int k = 0; k < nd; k++) {
-          const int a = at[sd[(size_t)order[i] * nd + k]], pl = place[a];
+          const int a = at[(size_t)(i - i0) * nd + k], pl = place[a];
           const uint16_t sg = m.sign[k] < 0 ? 0x8000 : 0;
           const int li = (int)(i - i0);
           const int sl = filled[a]++;
@@ -654,7 +659,6 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
           local[(size_t)i * nd + m.perm[k]] = (uint16_t)pl | sg;
         }
       }
-      for (int d : dl) at[d] = -1;
     }
   });
   nx = *std::max_element(max_local.begin(), max_local.end()) + 1;

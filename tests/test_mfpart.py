@@ -131,3 +131,103 @@ def test_structured_3d_classes_of_one_rounded_factor(mapper, p, same):
     _, maps = mapper(3, np.ascontiguousarray(ir.weights), b)
     assert len(maps) == 3 and maps["r"][:, 0].all()
     assert bool(maps["r"][:, 1].all()) == same and bool(maps["r"][:, 2].all()) == same
+
+
+GROW = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include <new>
+#include <random>
+#include "mfpart.hpp"
+static long long g_bytes = 0;
+void* operator new(std::size_t n) {
+  g_bytes += (long long)n;
+  void* p = std::malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+using namespace ngsamd;
+// in: elements, dofs per element, vertices per element, elements per patch and per
+// piece, dofs; out: bytes allocated by GrowPatches, by VertexElements, the order
+int main(int argc, char** argv) {
+  FILE* f = std::fopen(argv[1], "rb");
+  FILE* o = std::fopen(argv[2], "wb");
+  int h[5];
+  if (std::fread(h, 4, 5, f) != 5) return 1;
+  const int nel = h[0], nd = h[1], nv = h[2], size = h[3], piece = h[4];
+  std::vector<int> dofs((size_t)nel * nd), ptr, adj, order(nel, -1);
+  if (std::fread(dofs.data(), 4, dofs.size(), f) != dofs.size()) return 1;
+  long long bytes[2];
+  g_bytes = 0;
+  VertexElements(nel, nd, nv, dofs.data(), ptr, adj);
+  bytes[1] = g_bytes;
+  std::vector<int> stamp(ptr.size(), 0);
+  int patch = 0;
+  g_bytes = 0;
+  for (int e0 = 0; e0 < nel; e0 += piece)
+    GrowPatches(e0, std::min(nel, e0 + piece), nd, nv, dofs.data(), ptr, adj, size, stamp, patch, order.data());
+  bytes[0] = g_bytes;
+  // Numbering against a map
+  std::mt19937 rng(5);
+  Numbering number(600);
+  for (int t = 0; t < 200; t++) {
+    number.Clear();
+    std::map<int, int> m;
+    const int range = t % 3 == 0 ? 5 : t % 3 == 1 ? 700 : 0x7fffffff;
+    for (int k = 0; k < 600; k++) {
+      const int v = (int)(rng() % range), want = m.emplace(v, (int)m.size()).first->second;
+      if (number.Add(v) != want || number.Size() != (int)m.size()) return 2;
+    }
+  }
+  std::fwrite(bytes, 8, 2, o);
+  std::fwrite(order.data(), 4, nel, o);
+  std::fclose(o);
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def grower(tmp_path_factory):
+    d = tmp_path_factory.mktemp("grow")
+    exe = compile_host(d, GROW)
+
+    def run(dofs, nv, size, piece):
+        ne, nd = dofs.shape
+        (d / "in").write_bytes(np.int32([ne, nd, nv, size, piece]).tobytes() + dofs.astype(np.int32).tobytes())
+        subprocess.run([str(exe), str(d / "in"), str(d / "out")], check=True)
+        raw = (d / "out").read_bytes()
+        return np.frombuffer(raw, np.int64, 2), np.frombuffer(raw, np.int32, ne, 16)
+
+    return run
+
+
+@pytest.mark.parametrize("dim,n,p", [(2, (1, 1), 2), (2, (23, 31), 3), (3, (3, 5, 4), 1), (3, (8, 7, 9), 4)])
+@pytest.mark.parametrize("size,piece", [(64, 64), (64, 512), (128, 128 * 128)])
+def test_patches_partition_each_piece(grower, dim, n, p, size, piece):
+    mesh = N.MakeStructured2DMesh(*n) if dim == 2 else N.MakeStructured3DMesh(*n)
+    dofs = np.asarray(N.H1Space(mesh, p, 1).el_dofs)
+    (grow, around), order = grower(dofs, dim + 1, size, piece)
+    ne = len(dofs)
+    for e0 in range(0, ne, piece):
+        e1 = min(ne, e0 + piece)
+        assert np.array_equal(np.sort(order[e0:e1]), np.arange(e0, e1))
+    # neighbours: a patch has fewer vertices than its elements would apart
+    for i in range(0, ne - size + 1, size):
+        assert len(np.unique(dofs[order[i:i + size], :dim + 1])) < size * (dim + 1) / 2
+    # tables of the elements and of the vertices alone, however many pieces and dofs there are:
+    # two bytes and two numbers per element and, growing by doubling, the queues of one patch
+    # (at most 24 * size entries per vertex of an element)
+    pieces = -(-ne // piece)
+    assert grow <= 16 * ne + pieces * (8 * 24 * size * (dim + 1) * 4 + 1000)
+    assert around <= 4 * (3 * (dofs[:, :dim + 1].max() + 2) + (dim + 1) * ne)
+
+
+def test_patches_memory_independent_of_the_order(grower):
+    """High dof numbers of edges, faces and cells leave the growth's memory alone."""
+    mesh = N.MakeStructured3DMesh(8, 8, 8)
+    a, b = (grower(np.asarray(N.H1Space(mesh, p, 1).el_dofs), 4, 64, 256) for p in (1, 4))
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
