@@ -20,9 +20,7 @@
 // What bounds it: per patch two barriers and the chain dof list -> x -> LDS
 // -> MFMA -> LDS -> sums, overlapped between the workgroups of a CU.
 #include <algorithm>
-#include <exception>
-#include <system_error>
-#include <thread>
+#include <memory>
 #include <type_traits>
 #include <vector>
 
@@ -470,32 +468,21 @@ __global__ __launch_bounds__(64 * WAVES, 4) void MfPatch16Kernel(const uint16_t*
 
 // ----------------------------------------------------------------- host side
 
-// Runs f(first, last) over ranges of [0, n) on a few threads; an exception of
-// any of them is rethrown here.
-template <class F>
-static void InThreads(int64_t n, int64_t grain, F f) {
-  const int nt = (int)std::max<int64_t>(1, std::min<int64_t>({n / grain, (int64_t)std::thread::hardware_concurrency(), 16}));
-  std::vector<std::exception_ptr> failed(nt);
-  auto work = [&](int t) {
-    try {
-      f(n * t / nt, n * (t + 1) / nt);
-    } catch (...) {
-      failed[t] = std::current_exception();
-    }
-  };
-  std::vector<std::thread> th;
-  th.reserve(nt);
-  int started = 1;
-  try {
-    for (; started < nt; started++) th.emplace_back(work, started);
-  } catch (const std::system_error&) {  // no thread to be had: the rest runs here
-  }
-  work(0);
-  for (int t = started; t < nt; t++) work(t);
-  for (auto& t : th) t.join();
-  for (auto& e : failed)
-    if (e) std::rethrow_exception(e);
-}
+// A table that its loop fills whole: not cleared first, so that the threads that
+// write it take its pages in.
+template <class T>
+class HostTable {
+ public:
+  explicit HostTable(size_t n) : n_(n), p_(new T[n]) {}
+  T& operator[](size_t i) { return p_[i]; }
+  T* data() { return p_.get(); }
+  const T* data() const { return p_.get(); }
+  size_t size() const { return n_; }
+
+ private:
+  size_t n_;
+  std::unique_ptr<T[]> p_;
+};
 
 bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64_t fbytes,
                         const std::vector<MfClass>& classes, const std::vector<double>& S,
@@ -526,16 +513,14 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   int64_t kmax = 0;
   for (int64_t e = 0; e < nel; e++) kmax = std::max<int64_t>(kmax, elnr[e]);
   if (kmax >= 8 * nel + 1024) return false;
+  Workers workers(16);
   std::vector<int> cnt(kmax + 2, 0), cls(nel);
   for (int c = 0; c < nclass; c++)
     for (int64_t e = classes[c].begin; e < classes[c].end; e++) cls[e] = c;
   for (int64_t e = 0; e < nel; e++) cnt[elnr[e] + 1]++;
   for (int64_t k = 0; k <= kmax; k++) cnt[k + 1] += cnt[k];
-  std::vector<int> row(nel), sd((size_t)nel * nd);
+  std::vector<int> row(nel);
   for (int64_t e = 0; e < nel; e++) row[cnt[elnr[e]]++] = (int)e;
-  InThreads(nel, 8192, [&](int64_t a, int64_t b) {
-    for (int64_t i = a; i < b; i++) std::copy(dofs + (int64_t)row[i] * nd, dofs + (int64_t)row[i] * nd + nd, &sd[(size_t)i * nd]);
-  });
   // 8 tiles a patch (fewer shared dofs), 4 (more and smaller workgroups) where
   // 8 leave fewer than four patches per CU: 32^3 p=4 (1,536 patches of 8) FP64
   // 72 us against 89 with 4, split FP16 43 against 48 with FP32 vectors; 181x203
@@ -545,33 +530,37 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   const int size = 16 * waves;
   npatch = (int)((nel + size - 1) / size);
   // grown in chunks of 128 patches (whatever the number of threads)
-  std::vector<int> order(nel);
+  std::vector<int> order(nel);  // element rows, patch by patch
   {
     const int nv = std::min(dim + 1, nd);
-    std::vector<int> vptr, vadj;
-    VertexElements(nel, nd, nv, sd.data(), vptr, vadj);
+    std::vector<int> vptr, vadj, vd((size_t)nel * nv);  // vd: the elements' vertex dofs
+    for (int64_t i = 0; i < nel; i++) std::copy_n(dofs + (int64_t)row[i] * nd, nv, &vd[(size_t)i * nv]);
+    VertexElements(nel, nv, nv, vd.data(), vptr, vadj);
     const int64_t chunk = (int64_t)128 * size;
-    InThreads((nel + chunk - 1) / chunk, 1, [&](int64_t a, int64_t b) {
+    workers.Run((nel + chunk - 1) / chunk, 1, [&](Workers::Ranges& r) {
       std::vector<int> stamp(vptr.size(), 0);
       int patch = 0;
-      for (int64_t c = a; c < b; c++)
-        GrowPatches(c * chunk, std::min(nel, (c + 1) * chunk), nd, nv, sd.data(), vptr, vadj, size, stamp, patch,
-                    order.data());
+      for (int64_t c, c1; r.Next(c, c1);)
+        GrowPatches(c * chunk, std::min(nel, c1 * chunk), nv, nv, vd.data(), vptr, vadj, size, stamp, patch, order.data());
     });
+    for (int64_t i = 0; i < nel; i++) order[i] = row[order[i]];
   }
 
   // dofs of more than one patch (whichever thread meets a dof first owns it,
   // the flags come out the same)
   std::vector<int> owner(ndof, -1);
   std::vector<unsigned char> shared(ndof, 0);
-  InThreads(nel, 8192, [&](int64_t a, int64_t b) {
-    for (int64_t i = a; i < b; i++)
-      for (int k = 0; k < nd; k++) {
-        const int d = sd[(size_t)order[i] * nd + k], p = (int)(i / size);
-        int was = -1;
-        if (!__atomic_compare_exchange_n(&owner[d], &was, p, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED) && was != p)
-          __atomic_store_n(&shared[d], (unsigned char)1, __ATOMIC_RELAXED);
-      }
+  workers.Run(npatch, 32, [&](Workers::Ranges& r) {
+    r.Each([&](int64_t p) {
+      for (int64_t i = p * size; i < std::min(nel, (p + 1) * size); i++)
+        for (int k = 0; k < nd; k++) {
+          const int d = dofs[(int64_t)order[i] * nd + k];
+          int was = __atomic_load_n(&owner[d], __ATOMIC_RELAXED);
+          if (was < 0 && __atomic_compare_exchange_n(&owner[d], &was, (int)p, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED))
+            continue;
+          if (was != p) __atomic_store_n(&shared[d], (unsigned char)1, __ATOMIC_RELAXED);
+        }
+    });
   });
   for (int64_t d = 0; d < ndof; d++)
     if (owner[d] < 0) return false;  // a dof of no element: the general gather writes its 0
@@ -587,11 +576,10 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   std::vector<Patch> pt(npatch);
   const int ki = half_ ? 8 * ks1_ : ((nd + 3) / 4 + 3) / 4 * 4;
   const int ntile = npatch * waves;
-  std::vector<uint16_t> lidx((size_t)ntile * 64 * ki);
-  std::vector<double> tm((size_t)ntile * nc * 16, 0.0);
-  // lanes past the last element: metric 0, some element's coefficient
-  std::vector<int> te((size_t)ntile * 16, elnr[row[order[nel - 1]]]);
-  std::vector<uint16_t> local((size_t)nel * nd);  // position of each element dof in its patch's list
+  HostTable<uint16_t> lidx((size_t)ntile * 64 * ki);
+  HostTable<double> tm((size_t)ntile * nc * 16);
+  HostTable<int> te((size_t)ntile * 16);
+  HostTable<uint16_t> local((size_t)nel * nd);  // position of each element dof in its patch's list
   const int zero_cs = 16 * waves * nd;
   auto pos_of = [&](int k) {  // row order of the contributions in LDS (see the kernels)
     if (f64_ || (k & ~15) + 16 > nd) return k;
@@ -599,10 +587,14 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
     return (k & ~15) + 4 * (r % 4) + r / 4;
   };
   std::vector<int> max_local(npatch, 0);
-  InThreads(npatch, 16, [&](int64_t pa, int64_t pb) {
+  workers.Run(npatch, 8, [&](Workers::Ranges& r) {
     Numbering number((size_t)size * nd);
-    std::vector<int> at((size_t)size * nd), dl, c, o;  // at: number of each element dof among the patch's dl
-    for (int64_t p = pa; p < pb; p++) {
+    std::vector<int> at((size_t)size * nd), dl, c, place;  // at: number of each element dof among the patch's dl
+    std::vector<int> width, rows, filled;
+    std::vector<uint64_t> key;
+    std::vector<int> o;
+    KeySort sort;
+    r.Each([&](int64_t p) {
       Patch& P = pt[p];
       const int64_t i0 = p * size, i1 = std::min<int64_t>(nel, i0 + size);
       dl.clear();
@@ -610,7 +602,7 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
       number.Clear();
       for (int64_t i = i0; i < i1; i++)
         for (int k = 0; k < nd; k++) {
-          const int d = sd[(size_t)order[i] * nd + k], a = number.Add(d);
+          const int d = dofs[(int64_t)order[i] * nd + k], a = number.Add(d);
           at[(size_t)(i - i0) * nd + k] = a;
           if (a == (int)dl.size()) {
             dl.push_back(d);
@@ -618,15 +610,13 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
           }
           c[a]++;
         }
-      o.resize(dl.size());
-      for (size_t q = 0; q < o.size(); q++) o[q] = (int)q;
-      std::sort(o.begin(), o.end(), [&](int a, int b) {
-        if (shared[dl[a]] != shared[dl[b]]) return shared[dl[a]] < shared[dl[b]];
-        if (c[a] != c[b]) return c[a] > c[b];
-        return dl[a] < dl[b];
-      });
+      // inner before shared, then by falling count, then by number
+      key.resize(dl.size());
+      for (size_t q = 0; q < dl.size(); q++)
+        key[q] = (uint64_t)shared[dl[q]] << 63 | (uint64_t)(0x7fffffff - c[q]) << 32 | (uint32_t)dl[q];
+      sort(key, o);
       size_t q = 0;
-      std::vector<int> place(dl.size());  // padded position
+      place.resize(dl.size());  // padded position
       for (int part = 0; part < 2; part++) {
         while (P.xdof.size() % 64) P.xdof.push_back(-1);
         if (part == 1) P.nig = (int)P.xdof.size() / 64;
@@ -638,15 +628,16 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
       while (P.xdof.size() % 64) P.xdof.push_back(-1);
       max_local[p] = (int)P.xdof.size();
       const int ng = (int)P.xdof.size() / 64;
-      std::vector<int> width(ng, 0), rows(ng + 1, 0);
+      width.assign(ng, 0);
+      rows.assign(ng + 1, 0);
       for (size_t a = 0; a < dl.size(); a++) width[place[a] / 64] = std::max(width[place[a] / 64], c[a]);
       for (int g = 0; g < ng; g++) rows[g + 1] = rows[g] + std::max(0, (width[g] - 1) / 4);
       for (int g = 0; g < ng; g++) P.grp.push_back(make_int2(rows[g], width[g]));
       P.js.assign((size_t)ng * 256, (uint16_t)zero_cs);
       P.jx.assign((size_t)rows[ng] * 256, (uint16_t)zero_cs);
-      std::vector<int> filled(dl.size(), 0);
+      filled.assign(dl.size(), 0);
       for (int64_t i = i0; i < i1; i++) {
-        const int e = row[order[i]];
+        const int e = order[i];
         const ClassMap& m = map[cls[e]];
         for (int k = 0; k < nd; k++) {
           const int a = at[(size_t)(i - i0) * nd + k], pl = place[a];
@@ -659,7 +650,7 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
           local[(size_t)i * nd + m.perm[k]] = (uint16_t)pl | sg;
         }
       }
-    }
+    });
   });
   nx = *std::max_element(max_local.begin(), max_local.end()) + 1;
   if (nx > 0x7fff || zero_cs > 0x7fff) return false;
@@ -669,8 +660,8 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   lds = (lds + 15) / 16 * 16;
   if (lds + 1024 > (size_t)max_lds) return false;
 
-  InThreads(ntile, 64, [&](int64_t ta, int64_t tb) {
-    for (int64_t t = ta; t < tb; t++)
+  workers.Run(ntile, 64, [&](Workers::Ranges& r) {
+    r.Each([&](int64_t t) {
       for (int l = 0; l < 64; l++) {
         const int64_t i = t * 16 + l % 16;
         const int g = l / 16;
@@ -679,8 +670,13 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
           const int k = half_ ? 32 * (q / 8) + 8 * g + q % 8 : 4 * q + g;
           out[q] = i < nel && k < nd ? local[(size_t)i * nd + k] : (uint16_t)(nx - 1);
         }
-        if (g || i >= nel) continue;
-        const int e = row[order[i]];
+        if (g) continue;
+        if (i >= nel) {  // lanes past the last element: metric 0, some element's coefficient
+          for (int q = 0; q < nc; q++) tm[((size_t)t * nc + q) * 16 + l % 16] = 0.0;
+          te[(size_t)t * 16 + l % 16] = elnr[order[nel - 1]];
+          continue;
+        }
+        const int e = order[i];
         const double* A = map[cls[e]].A;
         const double* m = metric + (int64_t)e * nc;
         const double G3[9] = {m[0], m[nc > 3 ? 3 : 0], m[nc > 3 ? 4 : 0], m[nc > 3 ? 3 : 0], m[1], m[nc > 3 ? 5 : 0],
@@ -699,6 +695,7 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
         for (int q = 0; q < nc; q++) tm[((size_t)t * nc + q) * 16 + l % 16] = dim == 3 ? r3[q] : r2[q];
         te[(size_t)t * 16 + l % 16] = elnr[e];
       }
+    });
   });
 
   // concatenated tables, and the shared dofs' partial sums in patch order
@@ -713,18 +710,18 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
     b0 += (int64_t)(ng - pt[p].nig) * 64;
   }
   if (g0 * 64 >= (int64_t(1) << 31) || b0 >= (int64_t(1) << 31) || r0 >= (int64_t(1) << 31)) return false;
-  std::vector<int> xd((size_t)g0 * 64);
-  std::vector<int2> gp(g0);
-  std::vector<uint16_t> js((size_t)g0 * 256), jx((size_t)r0 * 256);
+  HostTable<int> xd((size_t)g0 * 64);
+  HostTable<int2> gp(g0);
+  HostTable<uint16_t> js((size_t)g0 * 256), jx((size_t)r0 * 256);
   std::vector<int64_t> roff(npatch + 1, 0);
   for (int p = 0; p < npatch; p++) roff[p + 1] = roff[p] + (int64_t)pt[p].jx.size();
-  InThreads(npatch, 64, [&](int64_t pa, int64_t pb) {
-    for (int64_t p = pa; p < pb; p++) {
-      std::copy(pt[p].xdof.begin(), pt[p].xdof.end(), xd.begin() + (size_t)hdr[p].x * 64);
-      std::copy(pt[p].grp.begin(), pt[p].grp.end(), gp.begin() + hdr[p].x);
-      std::copy(pt[p].js.begin(), pt[p].js.end(), js.begin() + (size_t)hdr[p].x * 256);
-      std::copy(pt[p].jx.begin(), pt[p].jx.end(), jx.begin() + roff[p]);
-    }
+  workers.Run(npatch, 64, [&](Workers::Ranges& r) {
+    r.Each([&](int64_t p) {
+      std::copy(pt[p].xdof.begin(), pt[p].xdof.end(), xd.data() + (size_t)hdr[p].x * 64);
+      std::copy(pt[p].grp.begin(), pt[p].grp.end(), gp.data() + hdr[p].x);
+      std::copy(pt[p].js.begin(), pt[p].js.end(), js.data() + (size_t)hdr[p].x * 256);
+      std::copy(pt[p].jx.begin(), pt[p].jx.end(), jx.data() + roff[p]);
+    });
   });
   // gather of the shared dofs: in the order their first partial sum appears
   std::vector<int> pc(ndof, 0), gorder, grow(1, 0), gslot(0);
@@ -749,7 +746,7 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
 
   auto up = [](auto& dev, const auto& host) {
     dev.alloc(std::max<size_t>(host.size(), 1));
-    if (!host.empty()) dev.upload(host.data(), host.size());
+    if (host.size()) dev.upload(host.data(), host.size());
   };
   up(d_hdr, hdr);
   up(d_xdof, xd);

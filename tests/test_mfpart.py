@@ -231,3 +231,91 @@ def test_patches_memory_independent_of_the_order(grower):
     mesh = N.MakeStructured3DMesh(8, 8, 8)
     a, b = (grower(np.asarray(N.H1Space(mesh, p, 1).el_dofs), 4, 64, 256) for p in (1, 4))
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+WORK = r"""
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <new>
+#include <random>
+#include <stdexcept>
+#include "mfpart.hpp"
+static std::atomic<int> g_left{-1};  // allocations until one fails, -1: none does
+void* operator new(std::size_t n) {
+  if (g_left.load() >= 0 && g_left.fetch_sub(1) == 0) throw std::bad_alloc();
+  void* p = std::malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+using namespace ngsamd;
+static int Check(Workers& w) {
+  for (int64_t n : {0, 1, 7, 64, 1000, 4097})
+    for (int64_t grain : {1, 3, 500}) {
+      std::vector<int> hit(n, 0);
+      w.Run(n, grain, [&](Workers::Ranges& r) {
+        for (int64_t a, b; r.Next(a, b);) for (int64_t i = a; i < b; i++) hit[i]++;
+      });
+      for (int v : hit) if (v != 1) return 1;
+    }
+  // any range may fail, the next loop runs whole again
+  for (int64_t bad : {0, 17, 99}) {
+    bool caught = false;
+    try {
+      w.Run(100, 1, [&](Workers::Ranges& r) {
+        for (int64_t a, b; r.Next(a, b);) if (a <= bad && bad < b) throw std::runtime_error("x");
+      });
+    } catch (const std::runtime_error&) {
+      caught = true;
+    }
+    if (!caught) return 2;
+  }
+  return 0;
+}
+int main() {
+  for (int t = 0; t < 20; t++) {
+    Workers w(1 + t % 9);
+    for (int k = 0; k < 5; k++) if (int r = Check(w)) return r;
+  }
+  // memory that runs out while the threads start leaves fewer of them
+  for (int at = 0; at < 12; at++) {
+    g_left = at;
+    Workers w(8);
+    g_left = -1;
+    if (int r = Check(w)) return 10 + r;
+  }
+  std::mt19937 rng(1);
+  for (int t = 0; t < 300; t++) {
+    const int n = (int)(rng() % 700), per = 1 + (int)(rng() % 300);
+    std::vector<int> list(n), ptr(n + 1, 0), ref;
+    for (int i = 0; i < n; i++) list[i] = i, ptr[i + 1] = ptr[i] + (int)(rng() % (t % 2 ? 5 : 40));
+    std::shuffle(list.begin(), list.end(), rng);
+    ref = list;
+    for (int a = 0; a < n; a += per)
+      std::stable_sort(ref.begin() + a, ref.begin() + std::min(n, a + per),
+                       [&](int u, int v) { return ptr[u + 1] - ptr[u] > ptr[v + 1] - ptr[v]; });
+    SortRangesByCount(list, per, ptr);
+    if (list != ref) return 20;
+  }
+  KeySort sort;
+  for (int t = 0; t < 300; t++) {
+    std::vector<uint64_t> key(rng() % 900);
+    for (auto& k : key)  // few and many equal ones, one bit in the highest byte, all bits
+      k = t % 3 == 0 ? rng() % 50 : t % 3 == 1 ? (uint64_t)(rng() & 1) << 63 | (uint64_t)(rng() % 9) << 32 | rng() % 100000
+                                               : (uint64_t)rng() << 32 | rng();
+    std::vector<int> pos, ref(key.size());
+    for (size_t i = 0; i < ref.size(); i++) ref[i] = (int)i;
+    std::stable_sort(ref.begin(), ref.end(), [&](int a, int b) { return key[a] < key[b]; });
+    sort(key, pos);
+    if (pos != ref) return 21;
+  }
+  return 0;
+}
+"""
+
+
+def test_workers_and_sort(tmp_path):
+    exe = compile_host(tmp_path, WORK)
+    assert subprocess.run([str(exe)], timeout=120).returncode == 0
