@@ -115,6 +115,10 @@ int ngsamd_csr_diagonal(ngsamd_op_t op, double* d_diag);
  * creation): the value vector of the matrix, BaseSparseMatrix::AsVector
  * (linalg/sparsematrix.hpp:312). */
 int ngsamd_csr_values(ngsamd_op_t op, double* h_vals);
+/* which kernels run: h_info[3] = {layout (0 row groups, 1 stream, 2 runs),
+ * workgroups of CG's product, 1 if Jacobi CG's product forms the search
+ * direction (two kernels an iteration), else 0} */
+int ngsamd_csr_info(ngsamd_op_t op, int64_t* h_info);
 
 /* ---------------------------------------------------------------- Jacobi */
 /* y += s * diag^{-1} x on free dofs, 0 on the others (linalg/jacobi.cpp:41-90).
@@ -206,6 +210,10 @@ int ngsamd_mf_create(ngsamd_op_t* op, int dim, int nd, int nq, int64_t ndof, int
  * number in h_elnr plus one (the row count of the tables if h_elnr was NULL);
  * element coefficients and element gradients are indexed by it */
 int ngsamd_mf_num_elements(ngsamd_op_t op, int64_t* ne);
+/* the element patches of the gather scatter: h_info[4] = {1 if the apply runs
+ * over patches, elements per patch, patches, dofs of several patches}; all 0
+ * where it does not */
+int ngsamd_mf_patch_info(ngsamd_op_t op, int64_t* h_info);
 /* Colour-ordered atomic-free scatter, as the reference's coloured element
  * loop (IterateElements over FESpace::ElementColoring, comp/fespace.cpp:518-760,
  * 2137-2200; comp/bilinearform.cpp:4669-4750): h_colors[nel] gives the colour

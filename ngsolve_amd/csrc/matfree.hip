@@ -2534,6 +2534,20 @@ extern "C" int ngsamd_mf_num_elements(ngsamd_op_t op, int64_t* ne) {
   });
 }
 
+extern "C" int ngsamd_mf_patch_info(ngsamd_op_t op, int64_t* h_info) {
+  return Guard([&] {
+    RequireInit();
+    NGSAMD_REQUIRE(op && op->kind == OpKind::MatrixFree, "ngsamd_mf_patch_info: not a matrix-free operator");
+    NGSAMD_REQUIRE(h_info, "ngsamd_mf_patch_info: null argument");
+    const MatFreeOp* M = static_cast<MatFreeOp*>(op);
+    const bool on = M->patch.ok && M->scatter == NGSAMD_SCATTER_GATHER;
+    h_info[0] = on ? 1 : 0;
+    h_info[1] = on ? 16 * M->patch.waves : 0;
+    h_info[2] = on ? M->patch.npatch : 0;
+    h_info[3] = on ? M->patch.nshared : 0;
+  });
+}
+
 extern "C" int ngsamd_mf_set_coloring(ngsamd_op_t op, const int* h_colors) {
   return Guard([&] {
     RequireInit();

@@ -800,6 +800,18 @@ extern "C" int ngsamd_csr_values(ngsamd_op_t op, double* h_vals) {
   });
 }
 
+extern "C" int ngsamd_csr_info(ngsamd_op_t op, int64_t* h_info) {
+  return Guard([&] {
+    RequireInit();
+    NGSAMD_REQUIRE(op && op->kind == OpKind::CSR, "ngsamd_csr_info: not a CSR operator");
+    NGSAMD_REQUIRE(h_info, "ngsamd_csr_info: null argument");
+    const CsrOp* A = static_cast<CsrOp*>(op);
+    h_info[0] = A->algo;
+    h_info[1] = DotWorkgroups(*A);
+    h_info[2] = A->FormsDirection() ? 1 : 0;
+  });
+}
+
 extern "C" int ngsamd_csr_diagonal(ngsamd_op_t op, double* d) {
   return Guard([&] {
     RequireInit();

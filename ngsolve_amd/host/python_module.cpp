@@ -734,6 +734,16 @@ PYBIND11_MODULE(_ngsamd, m) {
                                         seg.data(), with_f32 ? 1 : 0));
           return std::make_shared<Operator>(op, "batch");
         });
+  m.def("CSRInfo", [](Operator& A) {
+    int64_t v[3];
+    Check(ngsamd_csr_info(A.op, v));
+    return py::make_tuple(v[0], v[1], v[2] != 0);  // layout, workgroups of CG's product, it forms the direction
+  });
+  m.def("MatrixFreePatchInfo", [](Operator& A) {
+    int64_t v[4];
+    Check(ngsamd_mf_patch_info(A.op, v));
+    return py::make_tuple(v[0] != 0, v[1], v[2], v[3]);  // in use, elements per patch, patches, shared dofs
+  });
   m.def("BatchInfo", [](Operator& A) {
     int ns = 0, bn = 0, nb = 0;
     Check(ngsamd_batch_info(A.op, &ns, &bn, &nb));

@@ -23,10 +23,12 @@ def pcg(P, inv, f, u0, tol, maxiter):
 @pytest.mark.parametrize("dim,n,p", [(2, 2, 2), (2, 9, 3), (2, 20, 5), (3, 4, 3)])
 @pytest.mark.parametrize("maxiter", [1, 2, 3, 17, 2000])
 @pytest.mark.parametrize("chunk", [0, 2, 16])
-def test_against_oracle(device, dim, n, p, maxiter, chunk):
+def test_against_oracle(device, monkeypatch, dim, n, p, maxiter, chunk):
     say(f"[cg direction] {dim}D {n} p={p} maxiter={maxiter} chunk={chunk}")
+    monkeypatch.setenv("NGSAMD_SPMV", "runs")  # at p=2 the runs save too few column numbers
     P = problem(dim, n, p, seed_kappa=4)
     A = N.CreateCSR(P["ndof"], P["ndof"], P["rowptr"], P["cols"], P["vals"])
+    assert N.CSRInfo(A)[2]  # its product forms the direction
     free = P["fes"].freedofs.astype(np.uint8)
     diag, inv = O.jacobi_invdiag(P["rowptr"], P["cols"], P["vals"], free)
     C = N.CreateJacobi(diag, free)
@@ -43,9 +45,34 @@ def test_against_oracle(device, dim, n, p, maxiter, chunk):
             assert np.abs(du.download() - ref).max() <= 1e-9 * max(np.abs(ref).max(), 1e-300)
 
 
-def test_zero_right_hand_side(device):
+@pytest.mark.parametrize("dim,n,p,forms", [(2, 128, 3, True), (3, 13, 4, True), (3, 14, 4, False)])
+@pytest.mark.parametrize("chunk", [0, 16])
+def test_at_the_limit(device, dim, n, p, forms, chunk):
+    """The largest grids whose product forms the direction (1024 workgroups, up to
+    24 tasks each), and the first that leaves it to a kernel of its own."""
+    say(f"[cg direction] {dim}D {n} p={p} chunk={chunk}")
+    P = problem(dim, n, p, seed_kappa=4)
+    A = N.CreateCSR(P["ndof"], P["ndof"], P["rowptr"], P["cols"], P["vals"])
+    layout, workgroups, formed = N.CSRInfo(A)
+    assert layout == 2 and formed == forms and (workgroups == 1024) == forms
+    free = P["fes"].freedofs.astype(np.uint8)
+    diag, inv = O.jacobi_invdiag(P["rowptr"], P["cols"], P["vals"], free)
+    rng = np.random.default_rng(9)
+    f = np.where(free != 0, rng.uniform(-1, 1, P["ndof"]), 0.0)
+    u0 = np.where(free != 0, rng.uniform(-1, 1, P["ndof"]), 0.0)
+    ref, its_ref, res_ref = pcg(P, inv, f, u0, 1e-10, 18)
+    du = dvec(u0)
+    its, res = N.CGSolve(A, N.CreateJacobi(diag, free), dvec(f), du, False, 1e-10, -1.0, 18, chunk)
+    assert its == its_ref == 18
+    assert np.allclose(res, res_ref, rtol=1e-9, atol=0)
+    assert np.abs(du.download() - ref).max() <= 1e-9 * np.abs(ref).max()
+
+
+def test_zero_right_hand_side(device, monkeypatch):
+    monkeypatch.setenv("NGSAMD_SPMV", "runs")
     P = problem(2, 6, 2, seed_kappa=1)
     A = N.CreateCSR(P["ndof"], P["ndof"], P["rowptr"], P["cols"], P["vals"])
+    assert N.CSRInfo(A)[2]
     free = P["fes"].freedofs.astype(np.uint8)
     diag, _ = O.jacobi_invdiag(P["rowptr"], P["cols"], P["vals"], free)
     C = N.CreateJacobi(diag, free)
