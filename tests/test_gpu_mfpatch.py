@@ -100,6 +100,30 @@ def test_overlapping_vectors_and_new_coefficient(device, monkeypatch):
     d = dvec(x)
     A.op.mult(d, d)
     assert np.array_equal(d.download(), y)
+    # the same with FP32 vectors, accumulating, and with vectors that overlap in part
+    f = dvec(x, 4)
+    fy = N.DeviceVector(fes.ndof, 4)
+    A.op.mult_f32(f, fy)
+    A.op.mult_f32(f, f)
+    assert np.array_equal(f.download(), fy.download())
+    a, d = dvec(x), dvec(x)
+    A.op.mult_add(-0.5, d, d)
+    other = dvec(x)
+    A.op.mult_add(-0.5, other, a)
+    assert np.array_equal(d.download(), a.download())
+    n = fes.ndof
+    for itemsize in (8, 4):
+        for shift in (1, 37, n - 1):
+            both = N.DeviceVector(n + shift, itemsize)
+            for first in (0, shift):  # x before y, y before x
+                host = np.zeros(n + shift)
+                host[first:first + n] = x
+                both.upload(host.astype(np.float64 if itemsize == 8 else np.float32))
+                px = N.DeviceVector.wrap(both.ptr + itemsize * first, n, itemsize)
+                py = N.DeviceVector.wrap(both.ptr + itemsize * (shift - first), n, itemsize)
+                (A.op.mult if itemsize == 8 else A.op.mult_f32)(px, py)
+                got = both.download()[shift - first:shift - first + n]
+                assert np.array_equal(got, y if itemsize == 8 else fy.download())
     k2 = kappa[::-1].copy()
     B = build(monkeypatch, fes, k2, "f64", False)
     A.op.set_kappa(dvec(k2))
