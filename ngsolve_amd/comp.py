@@ -407,7 +407,7 @@ class DevMatrixFree(DeviceMatrix):
         op = N.CreateMatrixFree(dim, fes.space.nd_el, len(ir), fes.ndof, offsets, np.ascontiguousarray(bmat),
                                 np.ascontiguousarray(ir.weights), np.ascontiguousarray(dofs, dtype=np.int32),
                                 np.ascontiguousarray(metric), kap, el, PREC[precision],
-                                SCATTER["atomic" if atomic else "gather"])
+                                SCATTER["atomic" if atomic or coloring else "gather"])  # coloured: no patch tables
         if coloring:
             # FESpace element colouring (comp/fespace.cpp:518-760), in table order
             op.set_coloring(np.ascontiguousarray(N.ElementColoring(mesh)[el], dtype=np.int32))

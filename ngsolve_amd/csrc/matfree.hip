@@ -2029,6 +2029,7 @@ void MatFreeOp::SetColoring(const int* colors) {
   NGSAMD_HIP(hipStreamSynchronize(Stream()));
   ncolors = nc;
   scatter = NGSAMD_SCATTER_COLOR;
+  patch = MfPatchPlan();  // not used any more
   const MfSched S0 = OwnSched(*this);
   LaunchFacElements<2, double>(*this, nullptr, nullptr, 1.0, nullptr, nullptr, true, S0);
   LaunchFacElements<2, float>(*this, nullptr, nullptr, 1.0, nullptr, nullptr, true, S0);
@@ -2540,7 +2541,7 @@ extern "C" int ngsamd_mf_patch_info(ngsamd_op_t op, int64_t* h_info) {
     NGSAMD_REQUIRE(op && op->kind == OpKind::MatrixFree, "ngsamd_mf_patch_info: not a matrix-free operator");
     NGSAMD_REQUIRE(h_info, "ngsamd_mf_patch_info: null argument");
     const MatFreeOp* M = static_cast<MatFreeOp*>(op);
-    const bool on = M->patch.ok && M->scatter == NGSAMD_SCATTER_GATHER;
+    const bool on = M->patch.ok;
     h_info[0] = on ? 1 : 0;
     h_info[1] = on ? 16 * M->patch.waves : 0;
     h_info[2] = on ? M->patch.npatch : 0;

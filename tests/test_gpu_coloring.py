@@ -71,3 +71,26 @@ def test_bad_coloring_refused(device):
     A = mf_operator(P, 0)
     with pytest.raises(RuntimeError, match="share a dof"):
         A.set_coloring(np.zeros(P["mesh"].ne, dtype=np.int32))
+
+
+def test_coloring_drops_the_patches(device, monkeypatch):
+    """The element patches of the gather scatter go when colours replace it; the
+    colouring of the Python options never builds them."""
+    import ngsolve_amd as ngs
+    monkeypatch.setenv("NGSAMD_MF_PATCH", "1")
+    P = problem(3, 5, 3, seed_kappa=4)
+    A = mf_operator(P)
+    assert N.MatrixFreePatchInfo(A)[0]
+    dx, y0, y1 = dvec(np.random.default_rng(1).uniform(-1, 1, P["ndof"])), N.DeviceVector(P["ndof"], 8), N.DeviceVector(P["ndof"], 8)
+    A.mult(dx, y0)
+    A.set_coloring(_colors_table_order(P))
+    assert not any(N.MatrixFreePatchInfo(A))
+    A.mult(dx, y1)
+    assert relerr_inf(y1.download(), y0.download()) < 1e-14
+    fes = ngs.H1(ngs.MakeStructured3DMesh(nx=5, ny=5, nz=5), order=3, dirichlet=".*")
+    u, v = fes.TnT()
+    k = ngs.ElementCoefficient(P["kappa"])
+    B = ngs.BilinearForm(k * ngs.grad(u) * ngs.grad(v) * ngs.dx, mf=ngs.MFOpts(coloring=True)).Assemble().mat
+    assert not any(N.MatrixFreePatchInfo(B.op))
+    B.op.mult(dx, y1)
+    assert relerr_inf(y1.download(), y0.download()) < 1e-14
