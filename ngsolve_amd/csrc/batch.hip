@@ -87,7 +87,8 @@ struct BatchOp : ngsamd_op_s {
   std::vector<int64_t> seg_rows;
   int block_nnz = 2048;
   int nblocks = 0;
-  DevBuf<int> blk_row, blk_seg, seg_blk;
+  DevBuf<int> blk_row, blk_seg;  // stream layout
+  DevBuf<int> seg_blk;
   int nchunks = 0;
   DevBuf<int64_t> chunk_start;
   DevBuf<int> chunk_seg, seg_chunk;
@@ -409,8 +410,6 @@ BatchOp::BatchOp(int64_t n, const int64_t* rp, const int* c, const double* v, in
       }
       blk_info.alloc(info.size());
       blk_info.upload(info.data(), info.size());
-      blk_seg.alloc(std::max<size_t>(bs.size(), 1));
-      blk_seg.upload(bs.data(), bs.size());
       // first block of each problem (blocks are in problem order)
       std::vector<int> sb(ns + 1);
       for (int q = 0, b = 0; q <= ns; q++) {

@@ -1519,10 +1519,9 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
   // 3D 8192 elements (FP64 p=2 9K 9.4 / 8.9, p=4 17.3 / 15.6), 16-bit 16384
   // (p=4 9K 12.3 / 12.9, 16K 14.5 / 13.4); in 2D 240K element dofs (FP64 p=3
   // 9K elements 7.4 / 8.1, 30K 10.1 / 8.8), 16-bit 480K (p=4 16K 8.2 / 8.7,
-  // 60K 13.2 / 10.6), never for p=1 (150K 12.0 / 13.3).
+  // 60K 13.2 / 10.6), never for p=1 (150K 12.0 / 13.3: no PatchShape).
   const int64_t pmin = dim == 3 ? (half ? 16384 : 8192) : (half ? 480000 : 240000) / nd;
-  if (fac_kernel && scat == NGSAMD_SCATTER_GATHER && PatchShape(dim, nd, fac_kg) && !pnever &&
-      (pforce || dim == 3 || nd > 3))
+  if (fac_kernel && scat == NGSAMD_SCATTER_GATHER && PatchShape(dim, nd, fac_kg) && !pnever)
     patch.ok = patch.Build(dim, nd, ndof, prec, ks1, fstride * (half ? 2 : prec == NGSAMD_PREC_F64 ? 8 : 4), classes, S,
                            D, fac_rank, hdofs, hmetric, el.data(), DeviceMaxLds(), pforce ? 1 : (int)pmin);
   std::vector<int> gather_slots;  // element-major slots in gather order (kept for the tile-major copy)

@@ -492,9 +492,8 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   const bool half_ = prec == NGSAMD_PREC_BF16 || prec == NGSAMD_PREC_F16 || prec == NGSAMD_PREC_F16X3;
   const int nclass = (int)classes.size(), nc = dim * (dim + 1) / 2;
   const int64_t nel = nclass ? classes.back().end : 0;
-  // Below 8192 elements (128 patches) a patch's chain of phases is longer
-  // than the two wide kernels: 40^2 triangles p=3 split FP16 8.1 against 7.3 us
-  // (12^3 cubes p=4, 10,368 elements: FP64 15.7 against 18.4)
+  // on few patches a patch's chain of phases is longer than the two wide
+  // kernels (MatFreeOp's rule gives the number)
   if (nel < min_elements) return false;
   std::vector<ClassMap> map(nclass);
   const size_t ssz = (size_t)nc * nd * nd;
@@ -792,7 +791,7 @@ static void DispatchPatch(const MatFreeOp& A, const T* fm, const V* x, V* y, dou
                ? LaunchPatch(A, MfPatchKernel<T, DIM, NDP, ND, KG, V, 8>, fm, x, y, s, accumulate, stop, st, partials, prepare) \
                : LaunchPatch(A, MfPatchKernel<T, DIM, NDP, ND, KG, V, 4>, fm, x, y, s, accumulate, stop, st, partials, prepare);
   if constexpr (DIM == 2) {
-    NGSAMD_PATCH(4, 3, 1) NGSAMD_PATCH(8, 6, 1) NGSAMD_PATCH(12, 10, 2) NGSAMD_PATCH(16, 15, 3) NGSAMD_PATCH(24, 21, 4)
+    NGSAMD_PATCH(8, 6, 1) NGSAMD_PATCH(12, 10, 2) NGSAMD_PATCH(16, 15, 3) NGSAMD_PATCH(24, 21, 4)
   } else {
     NGSAMD_PATCH(4, 4, 1) NGSAMD_PATCH(12, 10, 1) NGSAMD_PATCH(20, 20, 3) NGSAMD_PATCH(36, 35, 5)
   }
@@ -809,8 +808,7 @@ static void DispatchPatch16(const MatFreeOp& A, const V* x, V* y, double s, int 
                ? LaunchPatch(A, MfPatch16Kernel<H, DIM, KS1, MT, KG, ND, V, SPLIT, 8>, A.fmat16.p, x, y, s, accumulate, stop, st, partials, prepare) \
                : LaunchPatch(A, MfPatch16Kernel<H, DIM, KS1, MT, KG, ND, V, SPLIT, 4>, A.fmat16.p, x, y, s, accumulate, stop, st, partials, prepare);
   if constexpr (DIM == 2) {
-    NGSAMD_PATCH(1, 1, 1, 3) NGSAMD_PATCH(1, 1, 1, 6) NGSAMD_PATCH(1, 1, 2, 10) NGSAMD_PATCH(1, 1, 3, 15)
-    NGSAMD_PATCH(1, 2, 4, 21)
+    NGSAMD_PATCH(1, 1, 1, 6) NGSAMD_PATCH(1, 1, 2, 10) NGSAMD_PATCH(1, 1, 3, 15) NGSAMD_PATCH(1, 2, 4, 21)
   } else {
     NGSAMD_PATCH(1, 1, 1, 4) NGSAMD_PATCH(1, 1, 1, 10) NGSAMD_PATCH(1, 2, 3, 20) NGSAMD_PATCH(2, 3, 5, 35)
   }
@@ -820,7 +818,7 @@ static void DispatchPatch16(const MatFreeOp& A, const V* x, V* y, double s, int 
 
 bool PatchShape(int dim, int nd, int kg) {
   auto is = [&](int n, int k) { return nd == n && kg == k; };
-  return dim == 2 ? is(3, 1) || is(6, 1) || is(10, 2) || is(15, 3) || is(21, 4)
+  return dim == 2 ? is(6, 1) || is(10, 2) || is(15, 3) || is(21, 4)
                   : is(4, 1) || is(10, 1) || is(20, 3) || is(35, 5);
 }
 

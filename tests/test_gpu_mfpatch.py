@@ -23,7 +23,7 @@ def build(monkeypatch, fes, kappa, precision, patch):
                            mf=ngs.MFOpts(precision=precision)).Assemble().mat
     # structured 3D meshes at p=4: three factors that round differently
     several = precision in ("f16", "bf16") and fes.mesh.ngmesh.dim == 3 and fes.order == 4
-    assert N.MatrixFreePatchInfo(mat.op)[0] == (patch and not several)
+    assert N.MatrixFreePatchInfo(mat.op)[0] == (patch and not several and (fes.mesh.ngmesh.dim, fes.order) != (2, 1))
     return mat
 
 
