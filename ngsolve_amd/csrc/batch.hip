@@ -211,16 +211,19 @@ struct BatchX {
 
 // The runs of one block (one problem and one R): 64 >> lg at a time, the next
 // ones' extent loaded meanwhile.
-template <int R, int U, class V, class M, bool ACCUM, bool DOT>
+template <int R, int U, class V, class M, bool ACCUM, bool DOT, bool HEAD>
 __device__ __forceinline__ void BatchRunRows(const int* __restrict__ run_ptr, const int* __restrict__ rcols,
                                              const M* __restrict__ rvals, const V* __restrict__ x,
                                              V* __restrict__ y, double s, int u0, int nr, int c00, int vb, int row0,
-                                             int lg, double& dotacc) {
+                                             int lg, int c0, int c1, double& dotacc) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> lg, l = lane & ((1 << lg) - 1);
   const int step = 64 >> lg;
   int u = min(g, nr - 1);
-  int c0 = run_ptr[u0 + u], c1 = run_ptr[u0 + u + 1];
+  if (!HEAD) {
+    c0 = run_ptr[u0 + u];
+    c1 = run_ptr[u0 + u + 1];
+  }
   for (int t = 0; t < nr; t += step) {
     const int un = min(t + step + g, nr - 1);
     const int n0 = run_ptr[u0 + un], n1 = run_ptr[u0 + un + 1];
@@ -251,12 +254,28 @@ __device__ __forceinline__ void BatchRunRows(const int* __restrict__ run_ptr, co
 // block per workgroup.
 // info[b]: {first run, runs, first column, first value},
 //          {first row, rows per run | log2(lanes per run) << 8, slots, problem}
-template <class V, class M, bool ACCUM, bool DOT>
-__device__ __forceinline__ void BatchRunsBlock(const int4* __restrict__ info, const int* __restrict__ run_ptr,
+// A block's records and, with HEAD (the walk has loaded them ahead), the lane's
+// first run.  A wide grid leaves them to the block: loaded before the test of
+// done they cost it 2 registers too many.
+struct BatchHead {
+  int4 a, e;
+  int c0, c1;
+  __device__ __forceinline__ void Records(const int4* __restrict__ info, int b) {
+    a = info[2 * b];
+    e = info[2 * b + 1];
+  }
+  __device__ __forceinline__ void Extent(const int* __restrict__ run_ptr) {
+    const int u = a.x + min((int)(threadIdx.x & 63) >> (e.y >> 8), a.y - 1);
+    c0 = run_ptr[u];
+    c1 = run_ptr[u + 1];
+  }
+};
+template <class V, class M, bool ACCUM, bool DOT, bool HEAD>
+__device__ __forceinline__ void BatchRunsBlock(const BatchHead& h, const int* __restrict__ run_ptr,
                                                const int* __restrict__ rcols, const M* __restrict__ rvals,
                                                const V* __restrict__ x, V* __restrict__ y, double s,
                                                const int* __restrict__ done, double* __restrict__ partials, int b) {
-  const int4 a = info[2 * b], e = info[2 * b + 1];
+  const int4 a = h.a, e = h.e;
   const int nr = __builtin_amdgcn_readfirstlane(a.y), slots = __builtin_amdgcn_readfirstlane(e.z);
   const int R = __builtin_amdgcn_readfirstlane(e.y & 255), lg = __builtin_amdgcn_readfirstlane(e.y >> 8);
   if (done && done[e.w]) {
@@ -266,8 +285,8 @@ __device__ __forceinline__ void BatchRunsBlock(const int4* __restrict__ info, co
   const int m = max(1, (slots + (nr << lg) - 1) / (nr << lg));
   double dotacc = 0.0;
   ForRunShape<1>(R, m, [&](auto r, auto u) __attribute__((always_inline)) {
-    BatchRunRows<decltype(r)::value, decltype(u)::value, V, M, ACCUM, DOT>(run_ptr, rcols, rvals, x, y, s, a.x, nr,
-                                                                          a.z, a.w, e.x, lg, dotacc);
+    BatchRunRows<decltype(r)::value, decltype(u)::value, V, M, ACCUM, DOT, HEAD>(
+        run_ptr, rcols, rvals, x, y, s, a.x, nr, a.z, a.w, e.x, lg, HEAD ? h.c0 : 0, HEAD ? h.c1 : 0, dotacc);
   });
   if (DOT) {
     dotacc = GroupSum(dotacc, 6);
@@ -283,8 +302,11 @@ __global__ __launch_bounds__(kBatchBlock, 6) void BatchRunsKernel(
   const int lb = XcdBlock(blockIdx.x, gridDim.x);
   const int b0 = (lb * (kBatchBlock / 64) + (threadIdx.x >> 6)) * blocks_per_wave;
   const int b1 = min(b0 + blocks_per_wave, nblocks);
-  for (int b = b0; b < b1; b++)
-    BatchRunsBlock<V, M, ACCUM, DOT>(info, run_ptr, rcols, rvals, x, y, s, done, partials, b);
+  for (int b = b0; b < b1; b++) {
+    BatchHead h;
+    h.Records(info, b);
+    BatchRunsBlock<V, M, ACCUM, DOT, false>(h, run_ptr, rcols, rvals, x, y, s, done, partials, b);
+  }
 }
 
 template <class V, class M, bool ACCUM, bool DOT>
@@ -903,9 +925,25 @@ __global__ __launch_bounds__(kBatchBlock) void BatchCgPersistentKernel(Persisten
     // (S) w = A s, <s, A s> per row block
     if constexpr (RUNS) {
       constexpr int waves = kBatchBlock / 64;
-      for (int b = lb * waves + (threadIdx.x >> 6); b < P.nblocks; b += G * waves)
-        BatchRunsBlock<double, double, false, true>(P.blk_info, P.run_ptr, P.rcols, P.rvals, P.s, P.w, 1.0, S.done,
-                                                    P.bpart, b);
+      int b = lb * waves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+      // 8 wavefronts per CU: the next block's run and the records of the one
+      // after it are loaded meanwhile (512 problems 1.096 -> 1.058 s; 1.071
+      // with a block per workgroup through LDS)
+      const int last = P.nblocks - 1;
+      BatchHead h, next;
+      if (b <= last) {
+        h.Records(P.blk_info, b);
+        h.Extent(P.run_ptr);
+        next.Records(P.blk_info, min(b + G * waves, last));
+      }
+      for (; b <= last; b += G * waves) {
+        BatchHead after;
+        after.Records(P.blk_info, min(b + 2 * G * waves, last));
+        next.Extent(P.run_ptr);
+        BatchRunsBlock<double, double, false, true, true>(h, P.run_ptr, P.rcols, P.rvals, P.s, P.w, 1.0, S.done, P.bpart, b);
+        h = next;
+        next = after;
+      }
     } else {
       for (int b = lb; b < P.nblocks; b += G)
         BatchSpmvBlock<NNZ, double, double, false, true>(P.rowptr, P.cols, P.vals, P.s, P.w, 1.0, P.blk_row,
