@@ -331,8 +331,9 @@ int ngsamd_cg_solve(ngsamd_op_t mat, ngsamd_op_t pre, const double* d_rhs, doubl
  * until the process ends): at most 4,194,304 dofs and maxiter <= 65536, or
  * the call fails with NGSAMD_E_ARG.  Kernels are launched directly (no
  * graph); the host reads the device scalars every 16 iterations with a
- * plain copy.  Same kernels in the same order as ngsamd_cg_solve, so the
- * same iterates.  Every call on one GPU shares that array: calls that overlap
+ * plain copy.  The steps of ngsamd_cg_solve in the same order and rounding, so
+ * the same iterates; a small CSR operator's iteration is three kernels here
+ * where ngsamd_cg_solve takes two.  Every call on one GPU shares that array: calls that overlap
  * on one GPU (several host threads or streams) race. */
 int ngsamd_cg_solve_noalloc(ngsamd_op_t mat, ngsamd_op_t pre, const double* d_rhs, double* d_sol,
                             int initialize, double tol, double atol, int maxiter,

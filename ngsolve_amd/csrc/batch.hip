@@ -246,19 +246,11 @@ __device__ __forceinline__ void BatchRunRows(const int* __restrict__ run_ptr, co
   }
 }
 
-// Runs-layout form of BatchSpmvKernel (the runs kernel of spmv.hip with the
-// frozen-problem skip and one partial per block): one block of up to 1024
-// values per wavefront, row sums in registers, neither LDS nor barriers.
-// What bounds it is the chain block record, run extent, columns, x: 48 2D
-// problems (32584 blocks, FP64, about 290 MB) take 0.106 ms, 0.128 with a
-// block per workgroup.
-// info[b]: {first run, runs, first column, first value},
-//          {first row, rows per run | log2(lanes per run) << 8, slots, problem}
 // A block's records and, with HEAD (the walk has loaded them ahead), the lane's
 // first run.  A wide grid leaves them to the block: loaded before the test of
-// done they cost it 2 registers too many.
+// done they would put 28 bytes of registers into scratch.
 struct BatchHead {
-  int4 a, e;
+  int4 a, e;  // info[2 b], info[2 b + 1] of BatchRunsBlock
   int c0, c1;
   __device__ __forceinline__ void Records(const int4* __restrict__ info, int b) {
     a = info[2 * b];
@@ -270,6 +262,14 @@ struct BatchHead {
     c1 = run_ptr[u + 1];
   }
 };
+// Runs-layout form of BatchSpmvKernel (the runs kernel of spmv.hip with the
+// frozen-problem skip and one partial per block): one block of up to 1024
+// values per wavefront, row sums in registers, neither LDS nor barriers.
+// What bounds it is the chain block record, run extent, columns, x: 48 2D
+// problems (32584 blocks, FP64, about 290 MB) take 0.106 ms, 0.128 with a
+// block per workgroup.
+// info[b]: {first run, runs, first column, first value},
+//          {first row, rows per run | log2(lanes per run) << 8, slots, problem}
 template <class V, class M, bool ACCUM, bool DOT, bool HEAD>
 __device__ __forceinline__ void BatchRunsBlock(const BatchHead& h, const int* __restrict__ run_ptr,
                                                const int* __restrict__ rcols, const M* __restrict__ rvals,
@@ -999,8 +999,8 @@ static void LaunchPersistent(const PersistentArgs& P, hipStream_t st) {
   // another count, at most the occupancy).  A grid at the full occupancy
   // has once timed out at a barrier (a workgroup not resident while the
   // others waited); well below it every workgroup finds a slot even when
-  // the dispatcher does not spread them evenly, and 2 to 8 per CU measured
-  // the same time.
+  // the dispatcher does not spread them evenly (512 problems, runs layout: 3
+  // of the 4 that fit take 3 to 5% less).
   const char* wenv = getenv("NGSAMD_BATCH_PERSISTENT_WG");
   occ = std::max(1, std::min(occ, wenv ? atoi(wenv) : 2));
   int64_t g = std::min<int64_t>((int64_t)occ * DeviceCUs(), std::max({P.nblocks, P.nchunks, P.nseg}));

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(kCgBlock) void CgInitKernel(const V* __restrict__ i
     const V wi = inv ? inv[i] * di : w[i];
     w[i] = wi;
     s[i] = wi;
-    acc += (double)wi * (double)di;
+    acc = CgFma((double)wi, (double)di, acc);
   }
   StorePartial<kCgBlock>(acc, partials, lds);
 }
@@ -162,13 +162,13 @@ __global__ __launch_bounds__(kCgBlock) void CgUpdateKernel(const V* __restrict__
   double acc = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)kCgBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kCgBlock) {
     const V si = s[i], wi = w[i];
-    u[i] += alv * si;
-    const V di = d[i] - alv * wi;
+    u[i] = CgFma(alv, si, u[i]);
+    const V di = CgFma(-alv, wi, d[i]);
     d[i] = di;
     if (inv) {
       const V zi = inv[i] * di;
       w[i] = zi;
-      acc += (double)zi * (double)di;
+      acc = CgFma((double)zi, (double)di, acc);
     }
   }
   if (inv) StorePartial<kCgBlock>(acc, pw, lds);
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(kCgBlock) void CgDirectionKernel(V* __restrict__ s,
   }
   const V bv = (V)beta;
   for (int64_t i = blockIdx.x * (int64_t)kCgBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kCgBlock)
-    s[i] = bv * s[i] + w[i];
+    s[i] = CgFma(bv, s[i], w[i]);
 }
 
 // Start of a solve whose operator forms the direction: w = C d, pairs {0, w};
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kCgBlock) void CgInitPairKernel(const double* __res
     const double wi = inv[i] * di;
     pair[2 * i] = 0.0;
     pair[2 * i + 1] = wi;
-    acc += wi * di;
+    acc = CgFma(wi, di, acc);
   }
   StorePartial<kCgBlock>(acc, partials, lds);
 }
@@ -237,12 +237,12 @@ __global__ __launch_bounds__(kCgBlock) void CgUpdatePairKernel(const double* __r
   double acc = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)kCgBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kCgBlock) {
     const double si = pair[2 * i], wi = w[i];
-    u[i] += alv * si;
-    const double di = d[i] - alv * wi;
+    u[i] = CgFma(alv, si, u[i]);
+    const double di = CgFma(-alv, wi, d[i]);
     d[i] = di;
     const double zi = inv[i] * di;
     pair[2 * i + 1] = zi;
-    acc += zi * di;
+    acc = CgFma(zi, di, acc);
   }
   StorePartial<kCgBlock>(acc, pw, lds);
 }
@@ -567,8 +567,9 @@ void InitCgScratch(int device) {
 // CG from an initialised d (= f - A u) to the stopping test, every kernel
 // launched directly (no graph, no events, no pinned memory): `chunk`
 // iterations are enqueued, then the device scalars are copied to the host
-// and checked.  Same kernels in the same order as IterateCg: the same
-// iterates.
+// and checked.  IterateCg's kernels in its order; where its operator forms the
+// direction (FormsDirection), the same steps in three kernels: the same
+// iterates bit for bit.
 static CgResult IterateCgDirect(ngsamd_op_t A, const double* inv, ngsamd_op_t pre, double* u, double* d, double* w,
                                 double* s, double* residuals, CGScalars* dS, int64_t n, double tol, double atol,
                                 int maxiter, hipStream_t st) {

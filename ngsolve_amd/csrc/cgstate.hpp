@@ -20,6 +20,12 @@ struct CGScalars {
 
 constexpr int kCgBlock = 256;
 
+// The steps of one entry, spelled out so that every kernel that takes them
+// rounds alike: the solvers with and without the direction in the product give
+// the same iterates bit for bit.
+__device__ __forceinline__ double CgFma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float CgFma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 __device__ __forceinline__ void CheckResidual(CGScalars* S, double* residuals, double res) {
   S->it += 1;
   if (S->it <= S->maxiter) residuals[S->it - 1] = res;

@@ -195,7 +195,7 @@ struct PairX {
   double beta;
   __device__ __forceinline__ double operator()(int i) const {
     const double2 t = pair[i];
-    return __builtin_fma(beta, t.x, t.y);
+    return CgFma(beta, t.x, t.y);
   }
 };
 

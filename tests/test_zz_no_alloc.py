@@ -110,3 +110,24 @@ def test_noalloc_refuses_sizes_beyond_scratch(device):
     fb, ub = N.DeviceVector(n, 8), N.DeviceVector(n, 8)
     rc, _, _ = noalloc(big, Cb, fb, ub)
     assert rc == 2 and b"4194304" in lib().ngsamd_last_error()
+
+
+@pytest.mark.parametrize("op,dim,n,p,layout", [("csr", 2, 20, 3, "runs"), ("csr", 3, 6, 4, "runs"),
+                                               ("csr", 3, 14, 4, "runs"), ("csr", 2, 30, 2, "stream"), ("mf", 3, 6, 3, "")])
+def test_noalloc_same_bits(device, monkeypatch, op, dim, n, p, layout):
+    """The same iterates as ngsamd_cg_solve, whose product forms the direction on
+    the smaller CSR operators in runs."""
+    if layout:
+        monkeypatch.setenv("NGSAMD_SPMV", layout)
+    P, A, C, f = _case(dim, n, p, 7, op)
+    if op == "csr":
+        assert N.CSRInfo(A)[2] == (layout == "runs" and (dim, n) != (3, 14))
+    df = dvec(f)
+    for maxiter in (1, 2, 17, 150):
+        for u0 in (None, np.random.default_rng(6).uniform(-1, 1, P["ndof"])):
+            u_ref, u = (dvec(np.zeros(P["ndof"]) if u0 is None else u0) for _ in range(2))
+            its_ref, res_ref = N.CGSolve(A, C, df, u_ref, u0 is None, 1e-10, -1.0, maxiter, 16)
+            rc, its, res = noalloc(A, C, df, u, u0 is None, maxiter=maxiter)
+            assert rc == 0, lib().ngsamd_last_error()
+            assert its == its_ref and np.array_equal(res, res_ref)
+            assert np.array_equal(u.download(), u_ref.download())
