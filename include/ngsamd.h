@@ -115,9 +115,10 @@ int ngsamd_csr_diagonal(ngsamd_op_t op, double* d_diag);
  * creation): the value vector of the matrix, BaseSparseMatrix::AsVector
  * (linalg/sparsematrix.hpp:312). */
 int ngsamd_csr_values(ngsamd_op_t op, double* h_vals);
-/* which kernels run: h_info[3] = {layout (0 row groups, 1 stream, 2 runs),
+/* which kernels run: h_info[4] = {layout (0 row groups, 1 stream, 2 runs),
  * workgroups of CG's product, 1 if Jacobi CG's product forms the search
- * direction (two kernels an iteration), else 0} */
+ * direction (two kernels an iteration), else 0, bytes of the layout and of x
+ * and y that an apply reads or writes once} */
 int ngsamd_csr_info(ngsamd_op_t op, int64_t* h_info);
 
 /* ---------------------------------------------------------------- Jacobi */

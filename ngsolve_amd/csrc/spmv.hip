@@ -292,7 +292,7 @@ __device__ __forceinline__ void RunTaskRows(const RunHead& h, const int* __restr
 // kernel (products of 2048-value blocks through LDS, one column and x load
 // per value), us per apply: 32^3 p=4 (159M nonzeros) 389 -> 298 (4.3 TB/s of
 // values alone, 5.2 TB/s with the shared columns), 20x16x24 p=4 97 -> 64,
-// 61x67 p=3 6.0 -> 4.3.
+// 61x67 p=3 7.8 -> 4.7.
 // DIR (with DOT): x is the new search direction, formed from the pairs of D
 // and stored by the rows' owners (CgDirection, which holds the stop flag).
 template <bool ACCUM, bool DOT, bool DIR>
@@ -811,6 +811,9 @@ extern "C" int ngsamd_csr_info(ngsamd_op_t op, int64_t* h_info) {
     h_info[2] = A->FormsDirection() ? 1 : 0;
   });
 }
+    h_info[3] = 8 * (A->nnz + A->width + A->height) +
+                (A->algo == 2 ? 4 * (A->nshared + A->nruns + 1) + 16 * (int64_t)A->ntasks
+                              : 4 * (A->nnz + A->height + 1));
 
 extern "C" int ngsamd_csr_diagonal(ngsamd_op_t op, double* d) {
   return Guard([&] {

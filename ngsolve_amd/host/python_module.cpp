@@ -735,9 +735,9 @@ PYBIND11_MODULE(_ngsamd, m) {
           return std::make_shared<Operator>(op, "batch");
         });
   m.def("CSRInfo", [](Operator& A) {
-    int64_t v[3];
+    int64_t v[4];
     Check(ngsamd_csr_info(A.op, v));
-    return py::make_tuple(v[0], v[1], v[2] != 0);  // layout, workgroups of CG's product, it forms the direction
+    return py::make_tuple(v[0], v[1], v[2] != 0, v[3]);  // layout, workgroups of CG's product, it forms the direction, bytes
   });
   m.def("MatrixFreePatchInfo", [](Operator& A) {
     int64_t v[4];

@@ -53,7 +53,7 @@ def test_at_the_limit(device, dim, n, p, forms, chunk):
     say(f"[cg direction] {dim}D {n} p={p} chunk={chunk}")
     P = problem(dim, n, p, seed_kappa=4)
     A = N.CreateCSR(P["ndof"], P["ndof"], P["rowptr"], P["cols"], P["vals"])
-    layout, workgroups, formed = N.CSRInfo(A)
+    layout, workgroups, formed, _ = N.CSRInfo(A)
     assert layout == 2 and formed == forms and (workgroups == 1024) == forms
     free = P["fes"].freedofs.astype(np.uint8)
     diag, inv = O.jacobi_invdiag(P["rowptr"], P["cols"], P["vals"], free)
