@@ -413,11 +413,13 @@ static int RunsGrid(const CsrOp& A, int cap) {
 }
 
 // The runs kernel with partial sums: a fold kernel (4.4 us) follows a grid of
-// over 1024 workgroups, so up to 6144 workgroups' worth of tasks run on 1024
-// (CG iteration on 128^2 p=5, 5,100: 41.8 -> 39.2 us; 23x19x27 p=3, 9,300:
-// 57.5 against 57.9, 20x16x24 p=4, 11,500: 100.5 against 103.2).
+// over 1024 workgroups, so up to 7168 workgroups' worth of tasks run on 1024
+// and, with Jacobi, form the direction (us per CG iteration, wide grid / 1024:
+// 14^3 p=4, 6,150 workgroups, 40.1 / 37.0; 128^2 p=5, 6,193, 42.7 / 40.1; 16^3
+// p=3, 6,303, 33.7 / 29.1; 140^2 p=5, 7,403, 44.9 / 46.2; 200^2 p=3, 7,526, 37.4
+// / 34.7; 150^2 p=5, 8,513, 49.3 / 51.6; 23x19x27 p=3, 17,964, 58.8 / 64.1).
 static int RunsDotCap(const CsrOp& A) {
-  return std::min(A.walk_grid, A.nblocks <= 6144 ? 1024 : kMaxWideBlocks);
+  return std::min(A.walk_grid, A.nblocks <= 7168 ? 1024 : kMaxWideBlocks);
 }
 
 void CsrOp::MultMulti(int K, const double* x, double* y, hipStream_t st, const int* stop) {
@@ -809,11 +811,11 @@ extern "C" int ngsamd_csr_info(ngsamd_op_t op, int64_t* h_info) {
     h_info[0] = A->algo;
     h_info[1] = DotWorkgroups(*A);
     h_info[2] = A->FormsDirection() ? 1 : 0;
-  });
-}
     h_info[3] = 8 * (A->nnz + A->width + A->height) +
                 (A->algo == 2 ? 4 * (A->nshared + A->nruns + 1) + 16 * (int64_t)A->ntasks
                               : 4 * (A->nnz + A->height + 1));
+  });
+}
 
 extern "C" int ngsamd_csr_diagonal(ngsamd_op_t op, double* d) {
   return Guard([&] {
