@@ -212,8 +212,9 @@ int ngsamd_mf_create(ngsamd_op_t* op, int dim, int nd, int nq, int64_t ndof, int
  * element coefficients and element gradients are indexed by it */
 int ngsamd_mf_num_elements(ngsamd_op_t op, int64_t* ne);
 /* the element patches of the gather scatter: h_info[4] = {1 if the apply runs
- * over patches, elements per patch, patches, dofs of several patches}; all 0
- * where it does not */
+ * over patches, tile columns per patch (an element each, 16 fewer elements where
+ * tiles have one of two reference classes), patches, dofs of several patches};
+ * all 0 where it does not */
 int ngsamd_mf_patch_info(ngsamd_op_t op, int64_t* h_info);
 /* Colour-ordered atomic-free scatter, as the reference's coloured element
  * loop (IterateElements over FESpace::ElementColoring, comp/fespace.cpp:518-760,

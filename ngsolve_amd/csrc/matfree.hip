@@ -1524,6 +1524,12 @@ MatFreeOp::MatFreeOp(int dim_, int nd_, int nq_, int64_t ndof, int nclass, const
   if (fac_kernel && scat == NGSAMD_SCATTER_GATHER && PatchShape(dim, nd, fac_kg) && !pnever)
     patch.ok = patch.Build(dim, nd, ndof, prec, ks1, fstride * (half ? 2 : prec == NGSAMD_PREC_F64 ? 8 : 4), classes, S,
                            D, fac_rank, hdofs, hmetric, el.data(), DeviceMaxLds(), pforce ? 1 : (int)pmin);
+  if (patch.ok && patch.reps.size() > 1) {
+    patch.d_reps.alloc(patch.reps.size() * fstride);
+    for (size_t r = 0; r < patch.reps.size(); r++)
+      NGSAMD_HIP(hipMemcpyAsync(patch.d_reps.p + r * fstride, fmat16.p + patch.reps[r] * fstride, 2 * fstride,
+                                hipMemcpyDeviceToDevice, Stream()));
+  }
   std::vector<int> gather_slots;  // element-major slots in gather order (kept for the tile-major copy)
   // dof -> contribution slots, ascending slot order (the order of each sum)
   std::vector<int> cnt(ndof + 1, 0);

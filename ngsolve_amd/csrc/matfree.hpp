@@ -11,13 +11,16 @@ struct MfClass {
   int64_t begin = 0, end = 0;  // element range in the (class-sorted) tables
 };
 
-// The patch kernels' tables (mfpatch.hip): elements in patches of 16 * waves
-// of one reference class, per patch its dofs in groups of 64 with the LDS
+// The patch kernels' tables (mfpatch.hip): elements in patches of up to 16 * waves,
+// mapped to one reference class (or two), per patch its dofs in groups of 64 with the LDS
 // positions of their contributions, and the gather of the dofs that several
 // patches share.
 struct MfPatchPlan {
   bool ok = false;
   int waves = 0, npatch = 0;
+  std::vector<int> reps;    // the reference classes, one for each tile
+  DevBuf<uint16_t> d_reps;  // with two: their factors, one after the other
+  DevBuf<int> d_tile_rep;   // and each tile's
   int nx = 0;               // x entries of a patch in LDS
   size_t lds = 0;
   mutable int occ[2] = {1, 1};  // resident workgroups per CU [FP64 vectors]
@@ -30,9 +33,8 @@ struct MfPatchPlan {
   DevBuf<int> s_rowptr, s_slots, s_order;  // shared dofs: their partial sums
   DevBuf<double> part;
   // S, D: the classes' reference matrices and their factors of rank `rank`.
-  // false: fewer than min_elements, some class is no relabelling of class 0
-  // (FP16 / BF16: its rounded factor is none), a dof belongs to no element, or
-  // a patch does not fit into LDS
+  // false: fewer than min_elements, some class is no relabelling of a reference
+  // class, a dof belongs to no element, or a patch does not fit into LDS
   bool Build(int dim, int nd, int64_t ndof, int prec, int ks1, int64_t fbytes, const std::vector<MfClass>& classes,
              const std::vector<double>& S, const std::vector<double>& D, int rank, const int* dofs,
              const double* metric, const int* elnr, int max_lds, int64_t min_elements);

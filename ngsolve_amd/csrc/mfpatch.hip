@@ -15,7 +15,11 @@
 // All vertex orders use one reference class (ClassMap: the dofs of the other
 // classes permuted, some with their signs turned, the metric transformed), so that a
 // patch's tiles are full whatever the classes of its elements and one D block
-// stays in LDS.  Signs ride in bit 15 of the 16-bit LDS indices.
+// stays in LDS.  Where a class's 16-bit D is other numbers than the reference's
+// (BF16 / FP16, 3D p=4) there are two, both in LDS, and a tile has one of them:
+// patches of 112 elements in 8 tiles, 48 in 4 (32^3 p=4 BF16 43.8 us per apply
+// with FP64 vectors, 40.9 with FP32; the general gather 71.1, 50.7).  Signs ride
+// in bit 15 of the 16-bit LDS indices.
 //
 // What bounds it: per patch two barriers and the chain dof list -> x -> LDS
 // -> MFMA -> LDS -> sums, overlapped between the workgroups of a CU.
@@ -298,13 +302,15 @@ __global__ __launch_bounds__(64 * WAVES, 4) void MfPatchKernel(const T* __restri
 }
 
 // 16-bit contraction (BF16, FP16, split FP16); D in LDS in the layout of MfFac16Kernel
-template <class H, int DIM, int KS1, int MT, int KG, int ND, class V, bool SPLIT, int WAVES>
+// TWO: the factors of two reference classes, tile_rep the one of each tile
+template <class H, int DIM, int KS1, int MT, int KG, int ND, class V, bool SPLIT, int WAVES, bool TWO>
 __global__ __launch_bounds__(64 * WAVES, 4) void MfPatch16Kernel(const uint16_t* __restrict__ fmat, int64_t fstride,
                                                               NGSAMD_PATCH_PARAMS, const double* __restrict__ kappa,
                                                               const V* __restrict__ x, V* __restrict__ y,
                                                               double* __restrict__ part, double s, int accumulate,
                                                               const int* __restrict__ stop,
-                                                              double* __restrict__ partials) {
+                                                              double* __restrict__ partials,
+                                                              const int* __restrict__ tile_rep) {
   if (stop && *stop) return;
   typedef typename Vec8<H>::type h8;
   typedef uint16_t Idx __attribute__((ext_vector_type(8)));  // 8 LDS indices of a lane
@@ -315,15 +321,16 @@ __global__ __launch_bounds__(64 * WAVES, 4) void MfPatch16Kernel(const uint16_t*
   constexpr int TT = ((NSL + 3) / 4 + 1) / 2 * 2;
   constexpr int KS2 = TT / 2;
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  float* xs = reinterpret_cast<float*>(lds_raw + fstride * 2);
+  float* xs = reinterpret_cast<float*>(lds_raw + fstride * (TWO ? 4 : 2));
   float* cs = xs;  // after the x entries have been read
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 15, grp = lane >> 4;
-  CopyToLds<64 * WAVES>(lds_raw, fmat, (int)(fstride / 8));
+  CopyToLds<64 * WAVES>(lds_raw, fmat, (int)(fstride / (TWO ? 4 : 8)));
   const h8* a1 = reinterpret_cast<const h8*>(lds_raw) + lane;
   const h8* a2 = a1 + TT * KS1 * 64;
   const h8* a1l = a1 + (TT * KS1 + MT * KS2) * 64;
   const h8* a2l = a1l + TT * KS1 * 64;
+  int rep = 0;
   double dacc = 0.0;
   const int wg = XcdContiguousBlock(blockIdx.x, gridDim.x);
   const int p0 = (int)((int64_t)wg * npatch / gridDim.x), p1 = (int)((int64_t)(wg + 1) * npatch / gridDim.x);
@@ -341,6 +348,12 @@ __global__ __launch_bounds__(64 * WAVES, 4) void MfPatch16Kernel(const uint16_t*
 #pragma unroll
     for (int c = 0; c < NC; c++) mv[c] = metric[(tile * NC + c) * 16 + col];
     const double kap = kappa[elnr[tile * 16 + col]];
+    if constexpr (TWO) {
+      const int r = __builtin_amdgcn_readfirstlane(tile_rep[tile]);
+      a1 += (r - rep) * (int)(fstride / 8);
+      a2 += (r - rep) * (int)(fstride / 8);
+      rep = r;
+    }
     StageX<WAVES>(R, h, x, xs, nx, xdof, js, grp_tab, wave, lane);
     int xn[NG];  // the next patch's dofs
     LoadDofs<WAVES>(xn, hn, xdof, wave, lane);
@@ -484,6 +497,10 @@ class HostTable {
   std::unique_ptr<T[]> p_;
 };
 
+// whether the one-term 16-bit kernels have an instance for two reference
+// classes: tetrahedra of order 4, the first order whose classes round apart
+static bool PatchShapeOfTwo(int dim, int nd) { return dim == 3 && nd == 35; }
+
 bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64_t fbytes,
                         const std::vector<MfClass>& classes, const std::vector<double>& S,
                         const std::vector<double>& D, int rank, const int* dofs, const double* metric, const int* elnr,
@@ -495,19 +512,30 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   // on few patches a patch's chain of phases is longer than the two wide
   // kernels (MatFreeOp's rule gives the number)
   if (nel < min_elements) return false;
-  std::vector<ClassMap> map(nclass);
-  const size_t ssz = (size_t)nc * nd * nd;
-  for (int c = 0; c < nclass; c++)
-    if (!MapClass(dim, nd, S.data(), S.data() + c * ssz, map[c])) return false;
+  // Each class as a relabelling of a reference class, the first one where that can be.
   // One 16-bit term: a class's results change with the rounding of its factor (3D
   // p=4 structured meshes: one class of three maps with A = (1 0 0; -1 -1 -1;
-  // 0 1 0), BF16 results 4e-4 apart), so that the first class's must be the same
-  // rounded numbers.  Split FP16 and FP32 differ by less than their sums' rounding.
-  if (half_ && prec != NGSAMD_PREC_F16X3)
-    for (int c = 0; c < nclass; c++) {
-      const double* Dc = D.data() + (size_t)c * dim * nd * rank;
-      if (!SameRoundedFactor(dim, nd, rank, D.data(), Dc, map[c], prec == NGSAMD_PREC_F16 ? ToF16 : ToBf16)) return false;
-    }
+  // 0 1 0), BF16 results 4e-4 apart), so that the reference class's must be the
+  // same rounded numbers, and a class without one becomes the second.  Split FP16
+  // and FP32 differ by less than their sums' rounding.
+  const bool one_term = half_ && prec != NGSAMD_PREC_F16X3;
+  std::vector<ClassMap> map(nclass);
+  std::vector<int> rep(nclass, -1);  // index among reps
+  const size_t ssz = (size_t)nc * nd * nd, dsz = (size_t)dim * nd * rank;
+  reps.clear();
+  for (int c = 0; c < nclass; c++) {
+    auto maps_to = [&](int r) {
+      return MapClass(dim, nd, S.data() + r * ssz, S.data() + c * ssz, map[c]) &&
+             (!one_term || SameRoundedFactor(dim, nd, rank, D.data() + r * dsz, D.data() + c * dsz, map[c],
+                                             prec == NGSAMD_PREC_F16 ? ToF16 : ToBf16));
+    };
+    for (size_t r = 0; r < reps.size() && rep[c] < 0; r++)
+      if (maps_to(reps[r])) rep[c] = (int)r;
+    if (rep[c] >= 0) continue;
+    if (reps.size() >= (one_term && PatchShapeOfTwo(dim, nd) ? 2 : 1) || !maps_to(c)) return false;
+    rep[c] = (int)reps.size();
+    reps.push_back(c);
+  }
   // elements by number: neighbours in the mesh are mostly near each other
   int64_t kmax = 0;
   for (int64_t e = 0; e < nel; e++) kmax = std::max<int64_t>(kmax, elnr[e]);
@@ -526,8 +554,10 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   // triangles p=5 (574) FP32 18.6 against 16.2, 23x19x27 p=3 (553) split FP16
   // 19.4 against 18.1
   waves = nel >= (int64_t)4 * 128 * DeviceCUs() ? 8 : 4;
-  const int size = 16 * waves;
-  npatch = (int)((nel + size - 1) / size);
+  // A tile's elements have one reference class: with two of them, 16 elements
+  // less always fit.
+  const int size = 16 * waves, fill = size - 16 * ((int)reps.size() - 1);
+  npatch = (int)((nel + fill - 1) / fill);
   // grown in chunks of 128 patches (whatever the number of threads)
   std::vector<int> order(nel);  // element rows, patch by patch
   {
@@ -535,14 +565,28 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
     std::vector<int> vptr, vadj, vd((size_t)nel * nv);  // vd: the elements' vertex dofs
     for (int64_t i = 0; i < nel; i++) std::copy_n(dofs + (int64_t)row[i] * nd, nv, &vd[(size_t)i * nv]);
     VertexElements(nel, nv, nv, vd.data(), vptr, vadj);
-    const int64_t chunk = (int64_t)128 * size;
+    const int64_t chunk = (int64_t)128 * fill;
     workers.Run((nel + chunk - 1) / chunk, 1, [&](Workers::Ranges& r) {
       std::vector<int> stamp(vptr.size(), 0);
       int patch = 0;
       for (int64_t c, c1; r.Next(c, c1);)
-        GrowPatches(c * chunk, std::min(nel, c1 * chunk), nv, nv, vd.data(), vptr, vadj, size, stamp, patch, order.data());
+        GrowPatches(c * chunk, std::min(nel, c1 * chunk), nv, nv, vd.data(), vptr, vadj, fill, stamp, patch, order.data());
     });
     for (int64_t i = 0; i < nel; i++) order[i] = row[order[i]];
+  }
+
+  // the element row of every tile column, -1: none
+  std::vector<int> slot((size_t)npatch * size, -1), trep((size_t)npatch * waves, 0);
+  for (int64_t p = 0; p < npatch; p++) {
+    int64_t at = p * size;
+    for (int r = 0; r < (int)reps.size(); r++) {
+      at = (at + 15) / 16 * 16;
+      for (int64_t i = p * fill; i < std::min(nel, (p + 1) * fill); i++)
+        if (rep[cls[order[i]]] == r) {
+          trep[at / 16] = r;
+          slot[at++] = order[i];
+        }
+    }
   }
 
   // dofs of more than one patch (whichever thread meets a dof first owns it,
@@ -551,9 +595,9 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   std::vector<unsigned char> shared(ndof, 0);
   workers.Run(npatch, 32, [&](Workers::Ranges& r) {
     r.Each([&](int64_t p) {
-      for (int64_t i = p * size; i < std::min(nel, (p + 1) * size); i++)
-        for (int k = 0; k < nd; k++) {
-          const int d = dofs[(int64_t)order[i] * nd + k];
+      for (int64_t i = p * size; i < (p + 1) * size; i++)
+        for (int k = 0; k < nd && slot[i] >= 0; k++) {
+          const int d = dofs[(int64_t)slot[i] * nd + k];
           int was = __atomic_load_n(&owner[d], __ATOMIC_RELAXED);
           if (was < 0 && __atomic_compare_exchange_n(&owner[d], &was, (int)p, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED))
             continue;
@@ -578,7 +622,7 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   HostTable<uint16_t> lidx((size_t)ntile * 64 * ki);
   HostTable<double> tm((size_t)ntile * nc * 16);
   HostTable<int> te((size_t)ntile * 16);
-  HostTable<uint16_t> local((size_t)nel * nd);  // position of each element dof in its patch's list
+  HostTable<uint16_t> local((size_t)npatch * size * nd);  // position of each element dof in its patch's list
   const int zero_cs = 16 * waves * nd;
   auto pos_of = [&](int k) {  // row order of the contributions in LDS (see the kernels)
     if (f64_ || (k & ~15) + 16 > nd) return k;
@@ -595,13 +639,13 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
     KeySort sort;
     r.Each([&](int64_t p) {
       Patch& P = pt[p];
-      const int64_t i0 = p * size, i1 = std::min<int64_t>(nel, i0 + size);
+      const int64_t i0 = p * size, i1 = i0 + size;
       dl.clear();
       c.clear();
       number.Clear();
       for (int64_t i = i0; i < i1; i++)
-        for (int k = 0; k < nd; k++) {
-          const int d = dofs[(int64_t)order[i] * nd + k], a = number.Add(d);
+        for (int k = 0; k < nd && slot[i] >= 0; k++) {
+          const int d = dofs[(int64_t)slot[i] * nd + k], a = number.Add(d);
           at[(size_t)(i - i0) * nd + k] = a;
           if (a == (int)dl.size()) {
             dl.push_back(d);
@@ -636,7 +680,8 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
       P.jx.assign((size_t)rows[ng] * 256, (uint16_t)zero_cs);
       filled.assign(dl.size(), 0);
       for (int64_t i = i0; i < i1; i++) {
-        const int e = order[i];
+        const int e = slot[i];
+        if (e < 0) continue;
         const ClassMap& m = map[cls[e]];
         for (int k = 0; k < nd; k++) {
           const int a = at[(size_t)(i - i0) * nd + k], pl = place[a];
@@ -655,7 +700,7 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   if (nx > 0x7fff || zero_cs > 0x7fff) return false;
   nx = (nx + 3) / 4 * 4;
   const size_t ts = f64_ ? 8 : 4;
-  lds = (size_t)fbytes + ts * (size_t)std::max(nx, zero_cs + 1);  // the contributions take the x entries' place
+  lds = (size_t)fbytes * reps.size() + ts * (size_t)std::max(nx, zero_cs + 1);  // the contributions take the x entries' place
   lds = (lds + 15) / 16 * 16;
   if (lds + 1024 > (size_t)max_lds) return false;
 
@@ -663,19 +708,18 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
     r.Each([&](int64_t t) {
       for (int l = 0; l < 64; l++) {
         const int64_t i = t * 16 + l % 16;
-        const int g = l / 16;
+        const int g = l / 16, e = slot[i];
         uint16_t* out = &lidx[((size_t)t * 64 + l) * ki];
         for (int q = 0; q < ki; q++) {
           const int k = half_ ? 32 * (q / 8) + 8 * g + q % 8 : 4 * q + g;
-          out[q] = i < nel && k < nd ? local[(size_t)i * nd + k] : (uint16_t)(nx - 1);
+          out[q] = e >= 0 && k < nd ? local[(size_t)i * nd + k] : (uint16_t)(nx - 1);
         }
         if (g) continue;
-        if (i >= nel) {  // lanes past the last element: metric 0, some element's coefficient
+        if (e < 0) {  // lanes without an element: metric 0, some element's coefficient
           for (int q = 0; q < nc; q++) tm[((size_t)t * nc + q) * 16 + l % 16] = 0.0;
           te[(size_t)t * 16 + l % 16] = elnr[order[nel - 1]];
           continue;
         }
-        const int e = order[i];
         const double* A = map[cls[e]].A;
         const double* m = metric + (int64_t)e * nc;
         const double G3[9] = {m[0], m[nc > 3 ? 3 : 0], m[nc > 3 ? 4 : 0], m[nc > 3 ? 3 : 0], m[1], m[nc > 3 ? 5 : 0],
@@ -755,6 +799,7 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
   up(d_lidx, lidx);
   up(d_metric, tm);
   up(d_elnr, te);
+  if (reps.size() > 1) up(d_tile_rep, trep);
   up(s_rowptr, grow);
   up(s_slots, gslot);
   up(s_order, gorder);
@@ -764,9 +809,9 @@ bool MfPatchPlan::Build(int dim, int nd, int64_t ndof, int prec, int ks1_, int64
 }
 
 // prepare: enable the dynamic LDS size and record the occupancy
-template <class K, class F, class V>
+template <class K, class F, class V, class... More>
 static void LaunchPatch(const MatFreeOp& A, K kern, const F* fmat, const V* x, V* y, double s, int accumulate,
-                        const int* stop, hipStream_t st, double* partials, bool prepare) {
+                        const int* stop, hipStream_t st, double* partials, bool prepare, More... more) {
   const MfPatchPlan& L = A.patch;
   if (prepare) {
     NGSAMD_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.lds));
@@ -778,7 +823,7 @@ static void LaunchPatch(const MatFreeOp& A, K kern, const F* fmat, const V* x, V
   kern<<<L.Grid(sizeof(V) == 8), 64 * L.waves, L.lds, st>>>(
       fmat, A.fstride, L.d_hdr.p, L.d_xdof.p, reinterpret_cast<const ushort4v*>(L.d_js.p), L.d_grp.p,
       reinterpret_cast<const ushort4v*>(L.d_jx.p), L.d_lidx.p, L.d_metric.p, L.d_elnr.p, L.npatch, L.nx, A.Kappa(), x,
-      y, L.part.p, s, accumulate, stop, partials);
+      y, L.part.p, s, accumulate, stop, partials, more...);
   NGSAMD_CHECK_LAUNCH();
 }
 
@@ -802,15 +847,22 @@ static void DispatchPatch(const MatFreeOp& A, const T* fm, const V* x, V* y, dou
 template <class H, int DIM, bool SPLIT, class V>
 static void DispatchPatch16(const MatFreeOp& A, const V* x, V* y, double s, int accumulate, const int* stop,
                             hipStream_t st, double* partials, bool prepare) {
-#define NGSAMD_PATCH(KS1, MT, KG, ND)                                                                                \
-  if (A.nd == ND && A.fac_kg == KG)                                                                                  \
+  const uint16_t* fm = A.patch.reps.size() > 1 ? A.patch.d_reps.p : A.fmat16.p;
+  const int* tile_rep = A.patch.d_tile_rep.p;
+#define NGSAMD_PATCH(KS1, MT, KG, ND, TWO)                                                                           \
+  if (A.nd == ND && A.fac_kg == KG && TWO == (A.patch.reps.size() > 1))                                              \
     return A.patch.waves == 8                                                                                        \
-               ? LaunchPatch(A, MfPatch16Kernel<H, DIM, KS1, MT, KG, ND, V, SPLIT, 8>, A.fmat16.p, x, y, s, accumulate, stop, st, partials, prepare) \
-               : LaunchPatch(A, MfPatch16Kernel<H, DIM, KS1, MT, KG, ND, V, SPLIT, 4>, A.fmat16.p, x, y, s, accumulate, stop, st, partials, prepare);
+               ? LaunchPatch(A, MfPatch16Kernel<H, DIM, KS1, MT, KG, ND, V, SPLIT, 8, TWO>, fm, x, y, s, accumulate, stop, st, partials, prepare, tile_rep) \
+               : LaunchPatch(A, MfPatch16Kernel<H, DIM, KS1, MT, KG, ND, V, SPLIT, 4, TWO>, fm, x, y, s, accumulate, stop, st, partials, prepare, tile_rep);
   if constexpr (DIM == 2) {
-    NGSAMD_PATCH(1, 1, 1, 6) NGSAMD_PATCH(1, 1, 2, 10) NGSAMD_PATCH(1, 1, 3, 15) NGSAMD_PATCH(1, 2, 4, 21)
+    NGSAMD_PATCH(1, 1, 1, 6, false) NGSAMD_PATCH(1, 1, 2, 10, false) NGSAMD_PATCH(1, 1, 3, 15, false)
+    NGSAMD_PATCH(1, 2, 4, 21, false)
   } else {
-    NGSAMD_PATCH(1, 1, 1, 4) NGSAMD_PATCH(1, 1, 1, 10) NGSAMD_PATCH(1, 2, 3, 20) NGSAMD_PATCH(2, 3, 5, 35)
+    NGSAMD_PATCH(1, 1, 1, 4, false) NGSAMD_PATCH(1, 1, 1, 10, false) NGSAMD_PATCH(1, 2, 3, 20, false)
+    NGSAMD_PATCH(2, 3, 5, 35, false)
+    if constexpr (!SPLIT) {
+      NGSAMD_PATCH(2, 3, 5, 35, true)
+    }
   }
 #undef NGSAMD_PATCH
   throw Error(NGSAMD_E_STATE, "matrix-free: unsupported 16-bit patch shape");
