@@ -140,11 +140,26 @@ __device__ __forceinline__ void SumPatch(const PatchRegs<NG, V>& R, const int4 h
   }
 }
 
+// An x entry as the contraction holds it in LDS.  For BF16 operands an FP64 entry
+// goes to FP32 by rounding to odd, so that its rounding to BF16 is that of the
+// FP64 value (one rounding, as in the general kernel; two differ in one of 1e4
+// entries, 1e-5 of the result).
+template <class T, bool ODD, class V>
+__device__ __forceinline__ T PatchX(V v) {
+  const T t = (T)v;
+  if constexpr (ODD && sizeof(V) == 8) {
+    const double r = (double)t;
+    const int b = __float_as_int(t) - (fabs(r) > fabs(v) ? 1 : 0);  // toward 0
+    return r < v || r > v ? __int_as_float(b | 1) : t;
+  }
+  return t;
+}
+
 // The start of a patch, whose dofs and x entries R holds: when the other
 // wavefronts have finished the previous patch (its contributions share the
 // LDS), the x entries go into LDS.  The first contributions' positions are
 // loaded for the sums.
-template <int WAVES, int NG, class T, class V>
+template <int WAVES, bool ODD, int NG, class T, class V>
 __device__ __forceinline__ void StageX(PatchRegs<NG, V>& R, const int4 h, const V* __restrict__ x, T* xs, int nx,
                                        const int* __restrict__ xdof, const ushort4v* __restrict__ js,
                                        const int2* __restrict__ grp_tab, int wave, int lane) {
@@ -158,9 +173,9 @@ __device__ __forceinline__ void StageX(PatchRegs<NG, V>& R, const int4 h, const 
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NG; i++)
-    if (wave + i * WAVES < h.z) xs[(wave + i * WAVES) * 64 + lane] = (T)R.v[i];
+    if (wave + i * WAVES < h.z) xs[(wave + i * WAVES) * 64 + lane] = PatchX<T, ODD>(R.v[i]);
   for (int g = wave + NG * WAVES; g < h.z; g += WAVES)
-    xs[g * 64 + lane] = (T)x[max(xdof[(int64_t)(h.x + g) * 64 + lane], 0)];
+    xs[g * 64 + lane] = PatchX<T, ODD>(x[max(xdof[(int64_t)(h.x + g) * 64 + lane], 0)]);
   if (threadIdx.x == 0) xs[nx - 1] = (T)0;
   __syncthreads();
 }
@@ -214,7 +229,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void MfPatchKernel(const T* __restri
 #pragma unroll
     for (int c = 0; c < NC; c++) mv[c] = metric[(tile * NC + c) * 16 + col];
     const double kap = kappa[elnr[tile * 16 + col]];
-    StageX<WAVES>(R, h, x, xs, nx, xdof, js, grp_tab, wave, lane);
+    StageX<WAVES, false>(R, h, x, xs, nx, xdof, js, grp_tab, wave, lane);
     int xn[NG];  // the next patch's dofs
     LoadDofs<WAVES>(xn, hn, xdof, wave, lane);
     T xk[KS];
@@ -354,7 +369,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void MfPatch16Kernel(const uint16_t*
       a2 += (r - rep) * (int)(fstride / 8);
       rep = r;
     }
-    StageX<WAVES>(R, h, x, xs, nx, xdof, js, grp_tab, wave, lane);
+    StageX<WAVES, std::is_same<H, __bf16>::value>(R, h, x, xs, nx, xdof, js, grp_tab, wave, lane);
     int xn[NG];  // the next patch's dofs
     LoadDofs<WAVES>(xn, hn, xdof, wave, lane);
     float xf[KS1][8];
