@@ -195,3 +195,55 @@ def check_16bit(monkeypatch, mesh, p, precision):
     # element's result at worst, its terms' errors independent 60^(1/2) * 2^-24 = 5e-7
     assert np.linalg.norm(out[0] - out[1]) <= 1e-6 * np.linalg.norm(out[1])
     return A
+
+
+def shuffled(mesh, seed=3):
+    """The mesh with its vertices renumbered and each element's given in another
+    (even) order: elements of every vertex order."""
+    m, rng = mesh.ngmesh, np.random.default_rng(seed)
+    num = rng.permutation(m.nv)
+    els, bnd = num[np.asarray(m.elements)], num[np.asarray(m.boundary)]
+    even = {2: [(0, 1, 2), (1, 2, 0), (2, 0, 1)],
+            3: [(0, 1, 2, 3), (1, 2, 0, 3), (2, 0, 1, 3), (1, 0, 3, 2), (0, 3, 1, 2), (3, 1, 0, 2), (2, 3, 0, 1),
+                (0, 2, 3, 1), (3, 0, 2, 1), (3, 2, 1, 0), (1, 3, 2, 0), (2, 1, 3, 0)]}[m.dim]
+    els = np.stack([e[list(even[k])] for e, k in zip(els, rng.integers(0, len(even), len(els)))])
+    pts = np.zeros((m.nv, 3))
+    pts[num, :m.dim] = np.asarray(m.coords)
+    line = lambda head, a: [head + " ".join(str(v + 1) for v in r) for r in a]  # noqa: E731
+    text = ["mesh3d", "dimension", str(m.dim)]
+    if m.dim == 2:
+        text += ["surfaceelements", str(len(els))] + line("1 1 0 0 3 ", els)
+        text += ["edgesegmentsgi2", str(len(bnd))] + line("1 0 ", bnd)
+    else:
+        text += ["surfaceelements", str(len(bnd))] + line("1 1 1 0 3 ", bnd)
+        text += ["volumeelements", str(len(els))] + line("1 4 ", els)
+    text += ["points", str(m.nv)] + [" ".join(repr(float(v)) for v in r) for r in pts] + ["endmesh"]
+    return ngs.Mesh(N.ReadVolMesh("\n".join(text)))
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32", "f16x3", "f16", "bf16"])
+@pytest.mark.parametrize("dim,p", [(2, 2), (2, 3), (2, 4), (2, 5), (3, 1), (3, 2), (3, 3), (3, 4)])
+def test_every_vertex_order(device, monkeypatch, dim, p, precision):
+    """One reference class for all 6 or 24 vertex orders; one-term 16-bit operators
+    whose factors round to more than two sets of numbers keep the general gather."""
+    say(f"[mfpatch orders] {dim}D p={p} {precision}")
+    mesh = shuffled(ngs.MakeStructured2DMesh(nx=23, ny=17) if dim == 2 else ngs.MakeStructured3DMesh(nx=6, ny=5, nz=7))
+    fes = ngs.H1(mesh, order=p, dirichlet=".*")
+    assert len(N.BuildClasses(fes.space, fes.integration_rule(2 * p))) == (6 if dim == 2 else 24)
+    rng = np.random.default_rng(2)
+    kappa, x = np.exp(rng.standard_normal(mesh.ne)), rng.uniform(-1, 1, fes.ndof)
+    out = []
+    for patch in "10":
+        monkeypatch.setenv("NGSAMD_MF_PATCH", patch)
+        u, v = fes.TnT()
+        M = ngs.BilinearForm(ngs.ElementCoefficient(kappa) * ngs.grad(u) * ngs.grad(v) * ngs.dx,
+                             mf=ngs.MFOpts(precision=precision)).Assemble().mat
+        on = N.MatrixFreePatchInfo(M.op)[0]
+        say(f"  patches: {on}")
+        assert on == (patch == "1") or (patch == "1" and precision in ("f16", "bf16"))
+        dx, dy = dvec(x), N.DeviceVector(fes.ndof, 8)
+        M.op.mult(dx, dy)
+        out.append(dy.download())
+    # as in compare; the 16-bit operands are the same numbers (test_16bit_rounding_of_every_class)
+    t = {"f64": 1e-14, "f32": 2e-6, "f16x3": 2e-6, "f16": 1e-6, "bf16": 1e-6}[precision]
+    assert np.linalg.norm(out[0] - out[1]) <= t * np.linalg.norm(out[1])
